@@ -6,6 +6,7 @@
 // flag (the values the Fortran driver needs before rigid() and ttime()).
 #include "fribo_internal.h"
 #include "fribo_batch.h"
+#include "fribo_xfer.h"
 #include "../../include/fribo_gpu.h"
 
 #include <algorithm>
@@ -67,6 +68,7 @@ struct fribo_ctx {
     StepIn* in = nullptr;
     DevScalars* hsp = nullptr;   // pinned landing buffer of the scalars read back after a step
     hipEvent_t ev_rb = nullptr;  // the read-back copy of those scalars
+    XferRing xfer;               // staging ring of the state transfers
     // k_cfl of the next step already enqueued behind the read-back of this
     // one (it reads only q2/q3, so it runs while the host prepares the next
     // step); cleared by anything that changes the velocities in between
@@ -608,6 +610,7 @@ extern "C" int fribo_finalize(fribo_handle h)
     if (h->in) hipHostFree(h->in);
     if (h->hsp) hipHostFree(h->hsp);
     if (h->ev_rb) hipEventDestroy(h->ev_rb);
+    xfer_free(h->xfer);
     for (auto ev : h->evpool) hipEventDestroy(ev);
     for (void* q : h->mk_allocs) hipFree(q);
     if (h->mk_stage) hipHostFree(h->mk_stage);
@@ -619,21 +622,38 @@ extern "C" int fribo_finalize(fribo_handle h)
 }
 
 // ---------------------------------------------------------------------------
-// State transfer (pitched copies between the reference layout and the device)
-static int put_field(fribo_ctx* c, double* dev, const double* host, int kfirst, int nplanes)
+// State transfer between the reference layout and the device (fribo_xfer.hip)
+static XferSeg field_seg(const FluidDev& F, double* dev, const double* host, int kfirst, int nplanes, bool pressure)
 {
-    const FluidDev& F = c->F;
-    HIPCHK(hipMemcpy2DAsync(dev + fidx(F, 1, kfirst), F.P * sizeof(double), host, F.n2 * sizeof(double),
-                            F.n2 * sizeof(double), nplanes, hipMemcpyHostToDevice, c->st));
-    return FRIBO_OK;
+    return XferSeg{dev + fidx(F, 1, kfirst), const_cast<double*>(host), F.n2, F.P, nplanes, kfirst, pressure ? 1 : 0};
 }
 
-static int get_field(fribo_ctx* c, double* host, const double* dev, int kfirst, int nplanes)
+static int xfer(fribo_ctx* c, XferSeg* segs, int nseg, bool put)
 {
-    const FluidDev& F = c->F;
-    HIPCHK(hipMemcpy2DAsync(host, F.n2 * sizeof(double), dev + fidx(F, 1, kfirst), F.P * sizeof(double),
-                            F.n2 * sizeof(double), nplanes, hipMemcpyDeviceToHost, c->st));
-    return FRIBO_OK;
+    const hipError_t he = xfer_run(c->xfer, c->F, segs, nseg, put, c->st);
+    return he == hipSuccess ? FRIBO_OK : set_err(FRIBO_ERR_HIP, std::string("state transfer: ") + hipGetErrorString(he));
+}
+
+static int get_field(fribo_ctx* c, double* host, double* dev, int kfirst, int nplanes)
+{
+    XferSeg s = field_seg(c->F, dev, host, kfirst, nplanes, false);
+    return xfer(c, &s, 1, false);
+}
+
+// The prognostic arrays of fribo_set_state / fribo_get_state (NULL: skipped).
+static int state_segs(const FluidDev& F, XferSeg* seg, const double* q2, const double* q3, const double* pr,
+                      const double* ru2, const double* ru3, const double* const* b)
+{
+    int n = 0;
+    if (q2) seg[n++] = field_seg(F, F.q2, q2, -2, F.nk, false);
+    if (q3) seg[n++] = field_seg(F, F.q3, q3, -2, F.nk, false);
+    if (pr) seg[n++] = field_seg(F, F.pr, pr, -2, F.nk, true);
+    if (ru2) seg[n++] = field_seg(F, F.ru2, ru2, 1, F.n3m, false);
+    if (ru3) seg[n++] = field_seg(F, F.ru3, ru3, 1, F.n3m, false);
+    double* d[] = {F.qb2s, F.qb3s, F.qb2n, F.qb3n, F.dq2x2o, F.dq3x2o};
+    for (int i = 0; i < 6; ++i)
+        if (b[i]) seg[n++] = XferSeg{d[i] + 1, const_cast<double*>(b[i]), F.n2, F.n2, 1, 0, 0};
+    return n;
 }
 
 static void enqueue_cfl(fribo_ctx* c);
@@ -663,18 +683,9 @@ extern "C" int fribo_set_state(fribo_handle h, const double* q2, const double* q
     h->cfl_ready = false;
     FluidDev& F = h->F;
     int e = 0;
-    if (q2 && !e) e = put_field(h, F.q2, q2, -2, F.nk);
-    if (q3 && !e) e = put_field(h, F.q3, q3, -2, F.nk);
-    if (pr && !e) e = put_field(h, F.pr, pr, -2, F.nk);
-    if (ru2 && !e) e = put_field(h, F.ru2, ru2, 1, F.n3m);
-    if (ru3 && !e) e = put_field(h, F.ru3, ru3, 1, F.n3m);
     const double* b[] = {qb2s, qb3s, qb2n, qb3n, dq2x2o, dq3x2o};
-    double* d[] = {F.qb2s, F.qb3s, F.qb2n, F.qb3n, F.dq2x2o, F.dq3x2o};
-    for (int i = 0; i < 6 && !e; ++i)
-        if (b[i]) {
-            hipError_t he = hipMemcpyAsync(d[i] + 1, b[i], F.n2 * sizeof(double), hipMemcpyHostToDevice, h->st);
-            if (he != hipSuccess) e = set_err(FRIBO_ERR_HIP, hipGetErrorString(he));
-        }
+    XferSeg seg[XFER_MAXSEG];
+    e = xfer(h, seg, state_segs(F, seg, q2, q3, pr, ru2, ru3, b), true);
     if (e) return e;
     if (pr) {
         // the uploaded pressure is already mean-free: nothing pending
@@ -693,35 +704,11 @@ extern "C" int fribo_get_state(fribo_handle h, double* q2, double* q3, double* p
                                double* dq3x2o)
 {
     if (!h) return set_err(FRIBO_ERR_ARG, "null handle");
-    FluidDev& F = h->F;
-    int e = 0;
-    if (q2 && !e) e = get_field(h, q2, F.q2, -2, F.nk);
-    if (q3 && !e) e = get_field(h, q3, F.q3, -2, F.nk);
-    if (pr && !e) e = get_field(h, pr, F.pr, -2, F.nk);
-    if (ru2 && !e) e = get_field(h, ru2, F.ru2, 1, F.n3m);
-    if (ru3 && !e) e = get_field(h, ru3, F.ru3, 1, F.n3m);
-    double* b[] = {qb2s, qb3s, qb2n, qb3n, dq2x2o, dq3x2o};
-    double* d[] = {F.qb2s, F.qb3s, F.qb2n, F.qb3n, F.dq2x2o, F.dq3x2o};
-    for (int i = 0; i < 6 && !e; ++i)
-        if (b[i]) {
-            hipError_t he = hipMemcpyAsync(b[i], d[i] + 1, F.n2 * sizeof(double), hipMemcpyDeviceToHost, h->st);
-            if (he != hipSuccess) e = set_err(FRIBO_ERR_HIP, hipGetErrorString(he));
-        }
-    if (e) return e;
-    if ((e = read_scalars(h))) return e;
-    if (pr) {
-        // apply the pending means (updvp.F90:141): the last one to the
-        // interior, their running sum to row n2 and the ghost planes
-        const double pend = h->hs.pend, goff = h->hs.goff;
-        for (int k = -2; k <= F.n3m + 3; ++k) {
-            const bool ghost = (k < 1 || k > F.n3m);
-            for (int j = 1; j <= F.n2; ++j) {
-                double& v = pr[(size_t)(j - 1) + (size_t)(k + 2) * F.n2];
-                v = v - ((ghost || j == F.n2) ? goff : pend);
-            }
-        }
-    }
-    return FRIBO_OK;
+    // the kernel applies the pending means (updvp.F90:141): the last one to
+    // the interior, their running sum to row n2 and the ghost planes
+    const double* b[] = {qb2s, qb3s, qb2n, qb3n, dq2x2o, dq3x2o};
+    XferSeg seg[XFER_MAXSEG];
+    return xfer(h, seg, state_segs(h->F, seg, q2, q3, pr, ru2, ru3, b), false);
 }
 
 extern "C" int fribo_set_markers(fribo_handle h, int32_t nlm, const double* lmcc, const double* lmvel,
@@ -808,30 +795,19 @@ extern "C" int fribo_fetch_fields(fribo_handle h, int32_t mask, int32_t kfirst, 
     FluidDev& F = h->F;
     if (kfirst < -2 || klast > F.n3m + 3 || kfirst > klast) return set_err(FRIBO_ERR_ARG, "bad plane window");
     double* hf[5] = {q2, q3, pr, ru2, ru3};
-    const double* df[5] = {F.q2, F.q3, F.pr, F.ru2, F.ru3};
-    int e = 0;
-    for (int f = 0; f < 5 && !e; ++f) {
+    double* df[5] = {F.q2, F.q3, F.pr, F.ru2, F.ru3};
+    XferSeg seg[XFER_MAXSEG];
+    int n = 0;
+    for (int f = 0; f < 5; ++f) {
         if (!((mask >> f) & 1)) continue;
         if (!hf[f]) return set_err(FRIBO_ERR_ARG, "null array for a selected field");
         const bool ru = f >= 3;
         const int a = ru ? std::max<int>(kfirst, 1) : kfirst, b = ru ? std::min<int>(klast, F.n3m) : klast;
         if (a > b) continue;
         const int base = ru ? 1 : -2;
-        e = get_field(h, hf[f] + (size_t)(a - base) * F.n2, df[f], a, b - a + 1);
+        seg[n++] = field_seg(F, df[f], hf[f] + (size_t)(a - base) * F.n2, a, b - a + 1, f == 2);
     }
-    if (e) return e;
-    if ((e = read_scalars(h))) return e;
-    if ((mask & 4) && pr) {
-        const double pend = h->hs.pend, goff = h->hs.goff;
-        for (int k = kfirst; k <= klast; ++k) {
-            const bool ghost = (k < 1 || k > F.n3m);
-            for (int j = 1; j <= F.n2; ++j) {
-                double& v = pr[(size_t)(j - 1) + (size_t)(k + 2) * F.n2];
-                v = v - ((ghost || j == F.n2) ? goff : pend);
-            }
-        }
-    }
-    return FRIBO_OK;
+    return xfer(h, seg, n, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -1825,11 +1801,12 @@ static int batch_refresh(fribo_batch_ctx* b)
     return FRIBO_OK;
 }
 
-// The marker-staging event of an instance whose stream is about to be
-// destroyed: its last record would be on that stream, so a fresh
-// (unrecorded) event takes its place.
-static void rearm_marker_event(fribo_ctx* h)
+// The staging events of an instance whose stream is about to be destroyed:
+// their last records would be on that stream, so a fresh (unrecorded) marker
+// event takes the old one's place, and the transfer ring makes its own again.
+static void rearm_events(fribo_ctx* h)
 {
+    xfer_free(h->xfer);
     if (!h->ev_mk) return;
     hipEventSynchronize(h->ev_mk);
     hipEventDestroy(h->ev_mk);
@@ -1857,7 +1834,7 @@ static void batch_free(fribo_batch_ctx* b)
     // the instances get streams of their own again
     for (auto h : b->inst) {
         if (h->batch != b) continue;
-        rearm_marker_event(h);
+        rearm_events(h);
         hipStreamCreate(&h->st);
         h->batch = nullptr;
     }
@@ -1915,7 +1892,7 @@ extern "C" int fribo_batch_create(const fribo_handle* hs, int32_t n, fribo_batch
         }
         h->cfl_ready = false;
         fribo_set_transform(h, all_y ? 1 : 0);
-        rearm_marker_event(h);
+        rearm_events(h);
         hipStreamDestroy(h->st);
         h->st = b->st;
         h->batch = b;
