@@ -234,7 +234,7 @@ def run_ensemble(args):
                       for c, m in zip(cs, mirror)))
     gemm_ms = float(tune_ms[best])
     achieved = flops / (gemm_ms * 1e-3) / 1e12
-    shapes = {0: "32x32", 1: "64x64", 2: "96x128", 3: "direct-to-LDS 96x128", 4: "direct-to-LDS 96x64"}
+    shapes = {0: "32x32", 1: "64x64", 2: "register-staged 96x128", 3: "direct-to-LDS 96x128", 4: "direct-to-LDS 96x64"}
     out = {
         "metric": "Mcell-steps/s (batched ensemble, plain FP64)",
         "value": round(value, 3),
@@ -475,10 +475,7 @@ def main():
     mirror = axis == "y" and g.ymirror and args.precision < 0
     gemm_flops = (1.0 if mirror else 2.0) * n3m * n2m * n2m if axis == "y" else 2.0 * n2m * n3m * n3m
     achieved = gemm_flops / gemm_avg_s / 1e12
-    # the transforms of this workload take the direct-to-LDS kernel (at least
-    # 192 tiles of 96x128 in the library's size test, operands with padded
-    # leading dimensions)
-    gemm_kernel = "k_gemm_dma" if -(-n2m // 96) * -(-n3m // 128) >= 192 else "k_gemm_nt"
+    gemm_kernel = "k_gemm_dma"
     peak = PEAK_FP64_MFMA_TFLOPS
     if args.precision >= 0:
         gemm_kernel, peak = "k_gemm32", PEAK_FP32_MFMA_TFLOPS

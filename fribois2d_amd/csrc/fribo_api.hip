@@ -86,7 +86,6 @@ struct fribo_ctx {
     hipGraphExec_t gexec = nullptr;
     int graph_nlm = -1;
     int mk_gen = 0;              // bumped whenever the marker buffers are reallocated
-    int ngpart64 = 0;            // tile columns of the FP64 backward transform along y
     int ysh_avail = 0;           // n2m / 2 when the mirror form of the y transform is set up
     bool dph_mirror = false;     // dph holds the mirror form's result before its pair butterfly
     bool ymirror_on = true;      // the mirror form selected (used while the transform is along y in FP64)
@@ -316,7 +315,9 @@ static int upload1i(fribo_ctx* c, int** dst, const std::vector<int>& h)
 static int ngpart_for(const fribo_ctx* c)
 {
     if (c->F.refine >= 0) return gemm32_tiles_n(c->F.n3m);
-    return c->F.ysh > 0 ? 2 * c->ngpart64 : c->ngpart64;
+    const FluidDev& F = c->F;
+    const int n = gemm_nn_tiles_n(F.n2m, F.n3m, F.n2m, F.ymm, F.ldy, F.hmn, F.P, F.ysh);
+    return F.ysh > 0 ? 2 * n : n;
 }
 
 // F.ysh from the options: n2m / 2 while the mirror form runs (selected,
@@ -361,10 +362,9 @@ static int setup_ytransform(fribo_ctx* c, const double* zmmt, int ldz)
     if (!e) e = dalloc(c, &F.wy, n);
     if (!e) e = dalloc(c, &F.zg, F.n3m);
     if (!e) e = dalloc(c, &F.ysum, (size_t)7 * n * FRIBO_KMAXCH);
-    c->ngpart64 = gemm_nn_tiles_n(n, F.n3m, n, F.ymm, F.ldy, F.hmn, F.P);
-    // room for the gauge partials of any tile shape (a batch may use
-    // 32-column tiles) and of the mirror form (two per tile column)
-    if (!e) e = dalloc(c, &F.gpart, 2 * std::max(c->ngpart64, (F.n3m + 31) / 32));
+    // room for the gauge partials of any tile shape (32 columns at least) and
+    // of the mirror form (two per tile column)
+    if (!e) e = dalloc(c, &F.gpart, 2 * ((F.n3m + 31) / 32));
     if (e) return e;
     HIPCHK(hipMemcpy(F.ymm, Y.data(), Y.size() * sizeof(double), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(F.ymmi, Yi.data(), Yi.size() * sizeof(double), hipMemcpyHostToDevice));

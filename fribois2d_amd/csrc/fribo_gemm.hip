@@ -11,46 +11,57 @@
 //
 // v_mfma_f64_16x16x4_f64 fragment layout: A fragment lane l holds
 // A[l%16][l/16]; B fragment lane l holds B[l/16][l%16]; accumulator element v
-// of lane l is C[l/16 + 4v][l%16].
+// of lane l is D[l/16 + 4v][l%16].  The kernels pass the B fragment as the
+// first operand, so D is the block of C transposed: lane l's element v is
+// C[l%16][l/16 + 4v], and a store writes whole 128-byte runs of four columns
+// (16 runs of 32 bytes the other way round).
 //
 // Tiling (template): BM x BN output tile per workgroup of WM x WN waves, each
-// wave owning (BM/WM) x (BN/WN) as 16x16 MFMA blocks; BK = 16 with two LDS
-// buffers (one barrier per K-slice: the next slice is fetched into registers
-// while the current one is multiplied, then stored into the other buffer).
-// LDS rows are padded to 16 (mod 32) doubles so the four k-rows a fragment
-// read touches fall in disjoint bank halves.  In the NN form (the transforms
-// along y, whose B operand is the field itself, k-contiguous) the B slice is
-// read as 16-double runs of each column and stored with a row pitch of BN+1,
-// which spreads the transposing LDS stores over the banks.
+// wave owning (BM/WM) x (BN/WN) as 16x16 MFMA blocks.  Every shape adds each
+// output element over k in the same order.
 //
-// Large problems (k_gemm_dma): 96 x 128 tiles of 16 waves (48 x 16 each, one
-// workgroup per CU; 96 x 64 tiles of 8 waves, two per CU, measured 1-5%
-// slower), K-slices of 24 (144 KB of LDS for the three stages; 16-deep
-// slices, one more barrier per 48 k, measured 3.5% slower on the 768-deep
-// products of the mirror form), and the operand slices move from global
-// memory straight into LDS
-// (global_load_lds_dwordx4, 16 bytes per lane, no register staging) through
-// three stages, so two K-slices of loads are in flight while one is
-// multiplied.  Each stage is its own LDS array, the slice loop is unrolled
-// by three, and the loads are issued as inline assembly: the compiler then
-// neither tracks them nor waits for every outstanding load before a
-// fragment read.  Every wave issues the same number of loads per slice
-// (addresses clamped into the matrix), so "slice s has landed" is
-// vmcnt(loads per slice), waited for explicitly: slice s+1 may stay in
-// flight; the workgroup barrier is a plain s_barrier for the same reason.
-// The loads of a slice are issued at raised wave priority.
-// A direct LDS write lands lane-contiguous, so the LDS layout follows the
-// global one: A and the NT-form B as k-rows (pitch 112 / 144 doubles: 48 / 64
-// used 16-byte slots of 56 / 72), the NN-form B as n-rows of BK k-values with
-// pitch BK+2 (the fragment read then hits 16 distinct bank groups).  Clamped
-// loads past the matrix only feed rows and columns that are not stored, or
-// the k-rows past K of the last slice, which are cleared before use; when
-// the load count of a stage does not divide evenly among the waves, the spare
-// loads land past the stage's B block.  The 1536 x 2048 transforms of the
-// 2048x1536-cell grid give 256 workgroups, one per CU; workgroups are
+// k_gemm_dma (all of the library's own operands: 16-byte aligned, even
+// leading dimensions): the operand slices move from global memory straight
+// into LDS (global_load_lds_dwordx4, 16 bytes per lane, no register staging)
+// through three stages, so two K-slices of loads are in flight while one is
+// multiplied.  The loads are issued as inline assembly: the compiler then
+// neither tracks them nor waits for every outstanding load before a fragment
+// read.  Every wave issues the same number of loads per slice (addresses
+// clamped into the matrix), so "slice s has landed" is vmcnt(loads per
+// slice), waited for explicitly: slice s+1 may stay in flight; the workgroup
+// barrier is a plain s_barrier for the same reason.  The loads of a slice are
+// issued at raised wave priority, with one lane offset per load that is the
+// same for every slice and a uniform base that advances (address arithmetic
+// per lane and slice cost 10-15% of the smaller tiles' time).
+// Clamped loads past the matrix only feed rows and columns that are not
+// stored, or the k-rows past K of the last slice, which are cleared before
+// use; when the load count of a stage does not divide evenly among the waves,
+// the spare loads land past the stage's B block.
+// What bounds it (672x810x672 in 64x64 tiles, one workgroup per CU, parts
+// left out in turn): 18 of 33 us are the MFMAs themselves, 6 the barrier per
+// slice, 2 the loads, 3 the fragment reads, the rest start and end.  So the
+// slices are deep (32) and the tiles small enough for several workgroups per
+// CU (gemm_tile): 57 us register-staged -> 24 us in 32x32 tiles, 977x1301
+// 115 -> 56 us, 288x384 in the mirror form 14.7 -> 5.8 us.
+//
+// Large problems take 96 x 128 tiles of 16 waves (48 x 16 each, one
+// workgroup per CU; 96 x 64 tiles of 8 waves, two per CU, measured the same
+// within 2%) with K-slices of 24 (144 KB of LDS for the three stages;
+// 16-deep slices measured 4-8% slower).  The 1536 x 2048 transforms of the
+// 2048x1536-cell grid give 256 workgroups, one per CU (84.4 us alone in the
+// mirror form; 92 in the step, with the operands out of the caches and the
+// fused chunk pass); workgroups are
 // dispatched to the 8 XCDs round-robin, so when the grid is a multiple of 256
 // tiles in 8 x 4 patches the tile indices are permuted to give each XCD
 // compact patches (its L2 then serves 8 A- and 4 B-tiles to 32 workgroups).
+//
+// k_gemm_nt (operands of any alignment, and the batch's shape 2): BK = 16
+// with two LDS buffers, the next slice fetched into registers while the
+// current one is multiplied, then stored into the other buffer.  LDS rows are
+// padded to 16 (mod 32) doubles; in the NN form (the transforms along y,
+// whose B operand is the field itself, k-contiguous) the B slice is read as
+// 16-double runs of each column and stored with a row pitch of BN+1, which
+// spreads the transposing LDS stores over the banks.
 #include "fribo_ychunk.h"
 #include "fribo_batch.h"
 #include <hip/hip_ext.h>
@@ -89,16 +100,16 @@ __device__ inline void gauge_partial(const f64x4 (&acc)[RM][RN], int grow, doubl
 {
     double v = 0.0;
 #pragma unroll
-    for (int c = 0; c < RN; ++c) {
-        const int col = n0 + wn * TN + c * 16 + (lane & 15);
+    for (int c = 0; c < RN; ++c)
 #pragma unroll
-        for (int r = 0; r < RM; ++r)
+        for (int q = 0; q < 4; ++q) {
+            const int col = n0 + wn * TN + c * 16 + (lane >> 4) + 4 * q;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = i0 + wm * TM + r * 16 + (lane >> 4) + 4 * q;
+            for (int r = 0; r < RM; ++r) {
+                const int row = i0 + wm * TM + r * 16 + (lane & 15);
                 if (row == grow && col < N) v = v + zg[col] * acc[r][c][q];
             }
-    }
+        }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
     if (lane == 0) sh[wave] = v;
@@ -110,38 +121,57 @@ __device__ inline void gauge_partial(const f64x4 (&acc)[RM][RN], int grow, doubl
     }
 }
 
-// Gauge partials of a tile with rows [i0, i0 + BM), tile column by of gy.
-// Plain form: C(M-1, :) into part[by].  Mirror form (ks > 0, C before the
-// pair butterfly, whose row M-1 is C(0, :) - C(M-1, :)): C(0, :) into
-// part[by] and -C(M-1, :) into part[gy + by].
-template <int RM, int RN, int TM, int TN, int NW, int BM>
-__device__ inline void gauge_partials(const f64x4 (&acc)[RM][RN], int ks, int M, int N, int i0, int n0, int wm,
-                                      int wn, int lane, int wave, int by, int gy, const double* __restrict__ zg,
-                                      double* part, double* sh)
+// Rows and K range of one tile row of C.  Plain form (ks = 0): tile bx holds
+// rows [bx * BM, ..), all of K.  Mirror form (ks > 0, A block-diagonal with
+// blocks [0, ks) and [ks, K) in both indices): the tile rows of the first
+// block come first, those of the second start at ks, so no tile holds rows
+// of both and each multiplies its own half of K only (a tile across the
+// split would run over all of K: twice the time of the others).  The second
+// block's loads start at the even row below ks (16-byte loads) and at the
+// multiple of four below it along k: the row is not stored, the k-rows meet
+// zeros of A.  Rows [lo, hi) are stored.
+struct TileRows {
+    int i0, lo, hi, kb, ke;
+};
+__host__ __device__ inline int tiles_m(int M, int ks, int BM)
 {
-    const bool last = M - 1 >= i0 && M - 1 < i0 + BM;
-    if (ks > 0 && i0 == 0) {
-        gauge_partial<RM, RN, TM, TN, NW>(acc, 0, 1.0, N, i0, n0, wm, wn, lane, wave, zg, part + by, sh);
-        if (last) lds_barrier();
+    if (ks <= 0) return (M + BM - 1) / BM;
+    return (ks + BM - 1) / BM + (M - (ks & ~1) + BM - 1) / BM;
+}
+__device__ inline TileRows tile_rows(int bx, int M, int K, int ks, int BM)
+{
+    const int nb0 = ks > 0 ? (ks + BM - 1) / BM : 0;
+    TileRows t;
+    if (ks > 0 && bx >= nb0) {
+        t.i0 = (ks & ~1) + (bx - nb0) * BM;
+        t.lo = t.i0 > ks ? t.i0 : ks;
+        t.hi = min(t.i0 + BM, M);
+        t.kb = ks & ~3;
+        t.ke = K;
+    } else {
+        t.i0 = bx * BM;
+        t.lo = t.i0;
+        t.hi = min(t.i0 + BM, ks > 0 ? ks : M);
+        t.kb = 0;
+        t.ke = ks > 0 ? ks : K;
     }
-    if (last)
-        gauge_partial<RM, RN, TM, TN, NW>(acc, M - 1, ks > 0 ? -1.0 : 1.0, N, i0, n0, wm, wn, lane, wave, zg,
-                                          part + (ks > 0 ? gy + by : by), sh);
+    return t;
 }
 
-// K range of an output tile with rows [i0, i0 + BM).  Plain form (ks = 0):
-// all of K.  Mirror form (ks > 0, A block-diagonal with blocks [0, ks) and
-// [ks, K) in both indices): rows below ks take k in [0, ks), rows from ks on
-// take [ks, K), a tile holding both takes all of K (the zero blocks add
-// exact zeros).  The start is rounded down to a multiple of BK: the k-rows
-// it adds meet zeros of A.
-__device__ inline void tile_krange(int ks, int K, int i0, int BM, int BK, int& kb, int& ke)
+// Gauge partials of a tile, tile column by of gy.  Plain form: C(M-1, :)
+// into part[by].  Mirror form (ks > 0, C before the pair butterfly, whose
+// row M-1 is C(0, :) - C(M-1, :)): C(0, :) into part[by] and -C(M-1, :) into
+// part[gy + by].
+template <int RM, int RN, int TM, int TN, int NW>
+__device__ inline void gauge_partials(const f64x4 (&acc)[RM][RN], int ks, int M, int N, const TileRows& tr, int n0,
+                                      int wm, int wn, int lane, int wave, int by, int gy,
+                                      const double* __restrict__ zg, double* part, double* sh)
 {
-    kb = 0;
-    ke = K;
-    if (ks <= 0) return;
-    if (i0 >= ks) kb = ks / BK * BK;
-    if (i0 + BM <= ks) ke = ks;
+    if (ks > 0 && tr.i0 == 0)
+        gauge_partial<RM, RN, TM, TN, NW>(acc, 0, 1.0, N, tr.i0, n0, wm, wn, lane, wave, zg, part + by, sh);
+    if (tr.hi == M)
+        gauge_partial<RM, RN, TM, TN, NW>(acc, M - 1, ks > 0 ? -1.0 : 1.0, N, tr.i0, n0, wm, wn, lane, wave, zg,
+                                          part + (ks > 0 ? gy + by : by), sh);
 }
 
 template <int BM, int BN, int WM, int WN, bool NN>
@@ -161,9 +191,9 @@ __device__ __forceinline__ void gemm_nt_body(int M, int N, int K, const double* 
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
     const int wm = wave % WM, wn = wave / WM;
-    const int i0 = vb.x * BM, n0 = vb.y * BN;
-    int kb, ke;
-    tile_krange(ks, K, i0, BM, GBK, kb, ke);
+    const int n0 = vb.y * BN;
+    const TileRows tr = tile_rows(vb.x, M, K, ks, BM);
+    const int i0 = tr.i0, kb = tr.kb, ke = tr.ke;
     double ra[NA], rb[NB];
 
     auto load = [&](int k0) {
@@ -223,7 +253,7 @@ __device__ __forceinline__ void gemm_nt_body(int M, int N, int K, const double* 
             for (int r = 0; r < RM; ++r)
 #pragma unroll
                 for (int c = 0; c < RN; ++c)
-                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b[c], acc[r][c], 0, 0, 0);
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[c], a[r], acc[r][c], 0, 0, 0);
         }
         if (more) store(buf ^ 1);
         __syncthreads();
@@ -233,17 +263,17 @@ __device__ __forceinline__ void gemm_nt_body(int M, int N, int K, const double* 
     for (int r = 0; r < RM; ++r)
 #pragma unroll
         for (int c = 0; c < RN; ++c) {
-            const int col = n0 + wn * TN + c * 16 + (lane & 15);
+            const int row = i0 + wm * TM + r * 16 + (lane & 15);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int row = i0 + wm * TM + r * 16 + (lane >> 4) + 4 * v;
-                if (row < M && col < N) C[(size_t)col * ldc + row] = acc[r][c][v];
+                const int col = n0 + wn * TN + c * 16 + (lane >> 4) + 4 * v;
+                if (row >= tr.lo && row < tr.hi && col < N) C[(size_t)col * ldc + row] = acc[r][c][v];
             }
         }
     if (zg) {
         __shared__ double gsh[WM * WN];
-        gauge_partials<RM, RN, TM, TN, WM * WN, BM>(acc, ks, M, N, i0, n0, wm, wn, lane, wave, vb.y, vb.gy, zg,
-                                                    gpart, gsh);
+        gauge_partials<RM, RN, TM, TN, WM * WN>(acc, ks, M, N, tr, n0, wm, wn, lane, wave, vb.y, vb.gy, zg, gpart,
+                                                gsh);
     }
 }
 template <int BM, int BN, int WM, int WN, bool NN>
@@ -267,51 +297,56 @@ __global__ __launch_bounds__(64 * WM * WN) void kb_gemm_nt(const BGrid<GemmProb>
 #ifndef GEMM_PRIO
 #define GEMM_PRIO 2
 #endif
-#ifndef GEMM_ASM_DMA
-#define GEMM_ASM_DMA 1
-#endif
+// Wait until at most n of the wave's vector memory accesses are outstanding.
+template <int n>
+__device__ inline void wait_vm()
+{
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+}
+
 // One 16-byte-per-lane global -> LDS load (global_load_lds_dwordx4: lane l
-// writes dst + 16 l).  Issued as inline assembly, the compiler does not track
-// the LDS write, so it adds no wait for it before later LDS reads of other
+// reads base + off and writes LDS byte lds + 16 l; base and lds are the same
+// in every lane).  Issued as inline assembly, the compiler does not track the
+// LDS write, so it adds no wait for it before later LDS reads of other
 // stages; the kernel's own vmcnt wait and barrier order every read after the
 // loads of its slice.
-__device__ inline void dma16(const double* src, double* dst)
+__device__ inline void dma16(const double* base, unsigned off, unsigned lds)
 {
-#if GEMM_ASM_DMA
-    const unsigned lds = __builtin_amdgcn_readfirstlane(
-        (unsigned)(uintptr_t)(__attribute__((address_space(3))) double*)dst);
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
-#else
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-#endif
+    const unsigned long long b = (unsigned long long)base;
+    const unsigned long long sb =
+        ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(b >> 32)) << 32) |
+        (unsigned)__builtin_amdgcn_readfirstlane((unsigned)b);
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+                 "v"(off), "s"(sb)
+                 : "memory");
 }
 
 template <int BK, bool NN, int WM = 2, int WN = 8, int BN = 128, int BM = 96>
 __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double* __restrict__ A, int lda, const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc, const DevScalars* S, const double* __restrict__ zg, double* gpart, YFuse yf, int ks, const VBlock& vb)
 {
+    constexpr int NST = 3;                                  // stages
     constexpr int NW = WM * WN;
     constexpr int TM = BM / WM, TN = BN / WN, RM = TM / 16, RN = TN / 16;
-    constexpr int LA = BM + 16, SLA = LA / 2;               // A: k-rows, BM / 2 of SLA slots used
-    constexpr int LB = NN ? BK + 2 : BN + 16, SLB = LB / 2; // B: n-rows (NN) or k-rows (NT)
+    // A: k-rows of BM doubles.  B: k-rows of BN doubles (NT) or n-rows of BK
+    // k-values (NN; 24 of them in a pitch of 26)
+    constexpr bool PADB = NN && BK == 24;
+    constexpr int LA = BM, SLA = LA / 2;
+    constexpr int LB = NN ? BK + (PADB ? 2 : 0) : BN, SLB = LB / 2;
     constexpr int SA = BK * LA, SB = NN ? BN * LB : BK * LB;   // doubles per stage
-    constexpr int IA = SA / 128, IB0 = SB / 128;            // 1 KB loads per stage
+    constexpr int IA = SA / 128, IB0 = (SB + 127) / 128;    // 1 KB loads per stage
     // every wave issues NI loads per stage; spare loads land past SB
     constexpr int NI = (IA + IB0 + NW - 1) / NW, IB = NI * NW - IA;
     constexpr int SBP = IB * 128;                           // B stage with the spare slots
-    static_assert(SA % 128 == 0 && SB % 128 == 0, "stage size");
-    static_assert(NI < 16, "load count per wave");
+    static_assert(SA % 128 == 0, "stage size");
+    static_assert(NI * (NST - 2) < 64, "loads in flight per wave");
     static_assert(TM % 16 == 0 && TN % 16 == 0 && BM % WM == 0 && BN % WN == 0, "wave tile");
-    static_assert(BM % 32 == 0, "A pitch 16 (mod 32)");
+    static_assert(BK == 16 || BK == 24 || BK == 32, "k-slices");
     if (S && S->err) return;
-    // the three stages in one block, which the fused epilogue of the NN form
+    // the stages in one block, which the fused epilogue of the NN form
     // reuses for the tile (BN rows of pitch BM + 1)
-    constexpr int SMN = 3 * (SA + SBP), STN = NN ? BN * (BM + 1) : 0;
+    constexpr int SMN = NST * (SA + SBP), STN = NN && BM == 96 ? BN * (BM + 1) : 0;
     __shared__ __attribute__((aligned(1024))) double SM[SMN > STN ? SMN : STN];
-    double* const S0 = SM;
-    double* const S1 = SM + (SA + SBP);
-    double* const S2 = SM + 2 * (SA + SBP);
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave % WM, wn = wave / WM;
     int bx = vb.x, by = vb.y;
     constexpr int PM = GEMM_PATCH_M, PN = 32 / GEMM_PATCH_M;
@@ -324,30 +359,55 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
         bx = (patch % npm) * PM + ll % PM;
         by = (patch / npm) * PN + ll / PM;
     }
-    const int i0 = bx * BM, n0 = by * BN;
-    int kb, ke;
-    tile_krange(ks, K, i0, BM, BK, kb, ke);
-    const int mlast = M - 2 + (M & 1), klast = K - 2 + (K & 1), nlast = N - 2 + (N & 1);
+    const int n0 = by * BN;
+    const TileRows tr = tile_rows(bx, M, K, ks, BM);
+    const int i0 = tr.i0, kb = tr.kb, ke = tr.ke;
+    const int mlast = M - 2 + (M & 1), nlast = N - 2 + (N & 1);
 
-    auto issue = [&](int k0, double* As, double* Bs) {
+    // A direct LDS write lands lane by lane, so the bank layout is made by
+    // which elements a lane fetches: 16-byte slot q of a row holds pair
+    // q ^ swz.  k-rows of a multiple of 32 doubles swap neighbouring runs of
+    // 16 doubles on odd rows (the two k-rows a half-wave reads then lie in
+    // different bank halves); the n-rows of the NN form spread the 16 rows a
+    // fragment reads over all banks.
+    auto swz_k = [](int k, int w) { return w % 32 == 0 ? (k & 1) << 3 : 0; };
+    auto swz_n = [](int n) { return PADB ? 0 : BK == 16 ? (n >> 1) & 7 : n & 15; };
+    // Load r of this wave is the 1 KB unit wave + NW * r of a stage (the A
+    // units first).  Its lane offsets from the slice's first element of A or B
+    // are the same for every slice, so a slice costs no address arithmetic
+    // per lane; only a slice that crosses K gets offsets of its own (kc: the
+    // k-rows the slice has inside the matrix).
+    unsigned voff[NI];
+    auto set_off = [&](int kc) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < NI; ++r) {
             const int ii = wave + NW * r;
-            const double* src;
-            double* dst;
-            if (ii < IA) {
-                const int slot = ii * 64 + lane, kk = slot / SLA, q = slot % SLA;
-                src = A + (size_t)min(k0 + kk, K - 1) * lda + min(i0 + 2 * q, mlast);
-                dst = As + ii * 128;
-            } else {
-                const int jj = ii - IA, slot = jj * 64 + lane, row = slot / SLB, q = slot % SLB;
-                // rows past the tile (the spare slots) read clamped addresses
-                if (NN) src = B + (size_t)min(n0 + row, N - 1) * ldb + min(k0 + 2 * q, klast);
-                else src = B + (size_t)min(k0 + min(row, BK - 1), K - 1) * ldb + min(n0 + 2 * q, nlast);
-                dst = Bs + jj * 128;
-            }
-            dma16(src, dst);
+            const int sa = ii * 64 + lane, ka = sa / SLA, qa = (sa % SLA) ^ swz_k(ka, BM);
+            const unsigned oa = (unsigned)(min(ka, kc - 1) * lda + min(i0 + 2 * qa, mlast)) * 8u;
+            // rows past the tile (the spare slots) and the pad pair of a row
+            // read other elements of the slice
+            const int sb = (ii - IA) * 64 + lane, rb = sb / SLB, qb = (sb % SLB) ^ (NN ? swz_n(rb) : swz_k(rb, BN));
+            const unsigned ob = NN ? (unsigned)((min(n0 + rb, N - 1) - n0) * ldb + min(2 * qb < BK ? 2 * qb : 0, (kc - 1) & ~1)) * 8u
+                                   : (unsigned)(min(rb, min(BK, kc) - 1) * ldb + min(n0 + 2 * qb, nlast)) * 8u;
+            voff[r] = ii < IA ? oa : ob;
         }
+    };
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) double*)SM;
+    constexpr int ST = SA + SBP;                            // doubles per stage
+    const double* pa = A + (size_t)kb * lda;
+    const double* pb = NN ? B + (size_t)n0 * ldb + kb : B + (size_t)kb * ldb;
+    int kleft = K - kb;                                     // k-rows of the matrix from the next slice to load on
+    set_off(min(BK, kleft));
+    // loads the next slice into the stage at element `st` of SM
+    auto issue = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < NI; ++r) {
+            const int ii = wave + NW * r;
+            dma16(ii < IA ? pa : pb, voff[r], lds0 + (unsigned)st * 8u + ii * 1024);
+        }
+        pa += (size_t)BK * lda;
+        pb += NN ? (size_t)BK : (size_t)BK * ldb;
+        kleft -= BK;
     };
 
     f64x4 acc[RM][RN];
@@ -357,29 +417,47 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
         for (int c = 0; c < RN; ++c) acc[r][c] = (f64x4){0.0, 0.0, 0.0, 0.0};
 
     const int nk = (ke - kb + BK - 1) / BK;
-    // slice s is in stage (As, Bs); slice s+2 goes into (An, Bn), the stage of slice s-1
-    auto step = [&](int s, double* As, double* Bs, double* An, double* Bn) {
-        if (s + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0F70 | NI);   // vmcnt(NI): only slice s+1 in flight
-        else __builtin_amdgcn_s_waitcnt(0x0F70);                    // vmcnt(0)
+    const int rem = (ke - kb) - (nk - 1) * BK;              // valid k-rows of the last slice
+#pragma unroll
+    for (int q = 0; q < NST - 1; ++q)
+        if (q < nk) {
+            if (q > 0 && kleft < BK) set_off(kleft);
+            issue(q * ST);
+        }
+    // slice s is in the stage at cur; slice s + NST - 1 goes into the stage of
+    // slice s - 1, at nxt
+    int cur = 0, nxt = (NST - 1) * ST;
+    for (int s = 0; s < nk; ++s) {
+        // slice s has landed: only the slices after it may be in flight
+        if (s + NST - 2 < nk) wait_vm<NI * (NST - 2)>();
+        else wait_vm<0>();
         raw_barrier();
-        const int kv = ke - kb - s * BK;      // valid k-rows of this slice
-        if (kv < BK) {
-            for (int e = t; e < (BK - kv) * LA; e += 64 * NW) As[kv * LA + e] = 0.0;
+#if GEMM_PRIO == 2
+        __builtin_amdgcn_s_setprio(1);
+#endif
+        if (s + NST - 1 < nk) {
+            if (kleft < BK) set_off(kleft);
+            issue(nxt);
+        }
+#if GEMM_PRIO == 2
+        __builtin_amdgcn_s_setprio(0);
+#endif
+        double* const As = SM + cur;
+        double* const Bs = As + SA;
+        if (s == nk - 1 && rem < BK) {
+            // k-rows past the range: cleared before use
+            for (int e = t; e < (BK - rem) * LA; e += 64 * NW) As[rem * LA + e] = 0.0;
             if (NN) {
-                for (int e = t; e < BN * (BK - kv); e += 64 * NW) Bs[(e / (BK - kv)) * LB + kv + e % (BK - kv)] = 0.0;
+                for (int e = t; e < BN * (BK - rem); e += 64 * NW) {
+                    const int n = e / (BK - rem), k = rem + e % (BK - rem);
+                    Bs[n * LB + (k ^ (swz_n(n) << 1))] = 0.0;
+                }
             } else {
-                for (int e = t; e < (BK - kv) * LB; e += 64 * NW) Bs[kv * LB + e] = 0.0;
+                for (int e = t; e < (BK - rem) * LB; e += 64 * NW) Bs[rem * LB + e] = 0.0;
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
             raw_barrier();
         }
-#if GEMM_PRIO == 2
-        __builtin_amdgcn_s_setprio(1);
-#endif
-        if (s + 2 < nk) issue(kb + (s + 2) * BK, An, Bn);
-#if GEMM_PRIO == 2
-        __builtin_amdgcn_s_setprio(0);
-#endif
 #if GEMM_PRIO == 1
         __builtin_amdgcn_s_setprio(1);
 #endif
@@ -388,43 +466,41 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
             const int kr = k4 + (lane >> 4);
             double a[RM], b[RN];
 #pragma unroll
-            for (int r = 0; r < RM; ++r) a[r] = As[kr * LA + wm * TM + r * 16 + (lane & 15)];
+            for (int r = 0; r < RM; ++r) a[r] = As[kr * LA + ((wm * TM + r * 16 + (lane & 15)) ^ (swz_k(lane >> 4, BM) << 1))];
 #pragma unroll
-            for (int c = 0; c < RN; ++c)
-                b[c] = NN ? Bs[(wn * TN + c * 16 + (lane & 15)) * LB + kr] : Bs[kr * LB + wn * TN + c * 16 + (lane & 15)];
+            for (int c = 0; c < RN; ++c) {
+                const int n = wn * TN + c * 16 + (lane & 15);
+                b[c] = NN ? Bs[n * LB + (kr ^ (swz_n(lane & 15) << 1))] : Bs[kr * LB + (n ^ (swz_k(lane >> 4, BN) << 1))];
+            }
 #pragma unroll
             for (int r = 0; r < RM; ++r)
 #pragma unroll
                 for (int c = 0; c < RN; ++c)
-                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b[c], acc[r][c], 0, 0, 0);
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[c], a[r], acc[r][c], 0, 0, 0);
         }
 #if GEMM_PRIO == 1
         __builtin_amdgcn_s_setprio(0);
 #endif
-    };
-    issue(kb, S0, S0 + SA);
-    if (nk > 1) issue(kb + BK, S1, S1 + SA);
-    for (int s = 0; s < nk; s += 3) {
-        step(s, S0, S0 + SA, S2, S2 + SA);
-        if (s + 1 < nk) step(s + 1, S1, S1 + SA, S0, S0 + SA);
-        if (s + 2 < nk) step(s + 2, S2, S2 + SA, S1, S1 + SA);
+        cur = cur + ST == NST * ST ? 0 : cur + ST;
+        nxt = nxt + ST == NST * ST ? 0 : nxt + ST;
     }
 #pragma unroll
     for (int r = 0; r < RM; ++r)
 #pragma unroll
         for (int c = 0; c < RN; ++c) {
-            const int col = n0 + wn * TN + c * 16 + (lane & 15);
+            const int row = i0 + wm * TM + r * 16 + (lane & 15);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int row = i0 + wm * TM + r * 16 + (lane >> 4) + 4 * v;
-                if (row < M && col < N) C[(size_t)col * ldc + row] = acc[r][c][v];
+                const int col = n0 + wn * TN + c * 16 + (lane >> 4) + 4 * v;
+                if (row >= tr.lo && row < tr.hi && col < N) C[(size_t)col * ldc + row] = acc[r][c][v];
             }
         }
     if (zg) {
         __shared__ double gsh[NW];
-        gauge_partials<RM, RN, TM, TN, NW, BM>(acc, ks, M, N, i0, n0, wm, wn, lane, wave, by, vb.gy, zg, gpart, gsh);
+        gauge_partials<RM, RN, TM, TN, NW>(acc, ks, M, N, tr, n0, wm, wn, lane, wave, by, vb.gy, zg, gpart, gsh);
     }
-    if (NN && yf.csz > 0) {
+    if constexpr (NN && BM == 96)
+    if (yf.csz > 0) {
         // chunk elimination of the y-mode z-lines on this tile: rows i are
         // y-modes, columns n the z rows; the tile holds BN / csz whole chunks
         constexpr int LT = BM + 1;   // LDS row pitch of the staged tile (one z row per LDS row)
@@ -435,7 +511,7 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
             for (int c = 0; c < RN; ++c)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    SM[(wn * TN + c * 16 + (lane & 15)) * LT + wm * TM + r * 16 + (lane >> 4) + 4 * v] = acc[r][c][v];
+                    SM[(wn * TN + c * 16 + (lane >> 4) + 4 * v) * LT + wm * TM + r * 16 + (lane & 15)] = acc[r][c][v];
         lds_barrier();
         constexpr int WPC = (BM + 63) / 64;   // waves per chunk
         const int csz = yf.csz, cc = wave / WPC, iw = (wave % WPC) * 64 + lane;
@@ -451,7 +527,7 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
             double yl, vl, ys, vs, ws, wl;
             ychunk_rows<32, false>(yf.amphk, yf.acphk, yf.apphk, s, m, w, dv, nullptr, nullptr, nullptr, yl, vl,
                                    ys, vs, ws, wl);
-            if (iw < BM && i0 + iw < M)
+            if (iw < BM && i0 + iw >= tr.lo && i0 + iw < tr.hi)
                 ysum_store(yf.ysum, yf.n2m, i0 + iw + 1, p, yf.amphk, yf.acphk, s + m, w, col[m * LT], yl, vl, wl,
                            ys, vs, ws);
         }
@@ -492,44 +568,70 @@ static void launch_timed(Kern kern, dim3 g, dim3 b, hipStream_t st, hipEvent_t e
     else hipLaunchKernelGGL(kern, g, b, 0, st, args...);
 }
 
+// Tile shape of one transform on the direct-to-LDS kernel.  The unit of time
+// is one 16x16 block per SIMD over all of K: a workgroup of 4 waves with one
+// block each (32x32) costs 1, one of 32x64 costs 2, one of 96x128 costs 12,
+// and a CU works through ceil(workgroups / 256) of them.  Per unit the larger
+// tiles are the faster ones (fewer loads and barriers per block): measured
+// with 12 units each, 1536x2048x1536 in the mirror form takes 84.4 us in
+// 96x128 tiles, 89.8 in 32x64 and 97.6 in 32x32, hence the weights 1, 0.94
+// and 0.87; but smaller tiles round up less (977x1301x977: 56.0 us with 5
+// units of 32x32, 62.1 with 6 of 32x64, 105 with 12 of 96x128).  With fewer
+// than 4 units the time is latency and the shorter tiles win ties (600x480
+// NT: 13.3 against 14.0 us).
+enum { TILE_32x32, TILE_32x64, TILE_96x128 };
+static int gemm_tile(int M, int N, int ks)
+{
+    const auto rounds = [](long t) { return (t + 255) / 256; };
+    const long u32 = rounds((long)tiles_m(M, ks, 32) * cdiv(N, 32));
+    const long u64 = 2 * rounds((long)tiles_m(M, ks, 32) * cdiv(N, 64));
+    const long u96 = 12 * rounds((long)tiles_m(M, ks, 96) * cdiv(N, 128));
+    if (100 * u96 <= 106 * u64 && 100 * u96 <= 115 * u32) return TILE_96x128;
+    return u32 >= 4 && 100 * u64 <= 108 * u32 ? TILE_32x64 : TILE_32x32;
+}
+
 template <bool NN>
 static int launch_gemm(int M, int N, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc,
                        const DevScalars* S, hipStream_t st, const double* zg, double* gpart, bool plan,
                        hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, const YFuse* yfp = nullptr,
                        bool* fused = nullptr, int ks = 0)
 {
-    YFuse yf{};
-    // the fused chunk pass needs whole chunks of at most 33 rows in every
-    // output tile of the direct-to-LDS kernel, and no more chunks per tile
-    // than the epilogue has wave groups (one group of (96 + 63) / 64 waves
-    // per chunk)
-    constexpr int kChunkGroups = (GEMM_DMA_WM * GEMM_DMA_WN) / ((96 + 63) / 64);
-    if (NN && yfp && yfp->csz > 1 && yfp->csz <= 33 && GEMM_DMA_BN % yfp->csz == 0 && N % GEMM_DMA_BN == 0 &&
-        GEMM_DMA_BN / yfp->csz <= kChunkGroups)
-        yf = *yfp;
     if (fused) *fused = false;
-    if ((long)cdiv(M, 96) * cdiv(N, 128) >= 192 && dma_ok<NN>(M, N, K, A, lda, B, ldb)) {
+    if (!dma_ok<NN>(M, N, K, A, lda, B, ldb)) {
+        // operands without 16-byte alignment (host callers' own leading dimensions)
+        if (!plan)
+            launch_timed(k_gemm_nt<32, 32, 2, 2, NN>, dim3(tiles_m(M, ks, 32), cdiv(N, 32)), dim3(256), st, e0, e1, M,
+                         N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
+        return cdiv(N, 32);
+    }
+    YFuse yf{};
+    switch (gemm_tile(M, N, ks)) {
+    case TILE_96x128: {
+        // the fused chunk pass needs whole chunks of at most 33 rows in every
+        // output tile, and no more chunks per tile than the epilogue has wave
+        // groups (one group of (96 + 63) / 64 waves per chunk)
+        constexpr int kChunkGroups = (GEMM_DMA_WM * GEMM_DMA_WN) / ((96 + 63) / 64);
+        if (NN && yfp && yfp->csz > 1 && yfp->csz <= 33 && GEMM_DMA_BN % yfp->csz == 0 && N % GEMM_DMA_BN == 0 &&
+            GEMM_DMA_BN / yfp->csz <= kChunkGroups)
+            yf = *yfp;
         if (!plan)
             launch_timed(k_gemm_dma<GEMM_DMA_BK, NN, GEMM_DMA_WM, GEMM_DMA_WN, GEMM_DMA_BN>,
-                         dim3(cdiv(M, 96), cdiv(N, GEMM_DMA_BN)), dim3(64 * GEMM_DMA_WM * GEMM_DMA_WN), st, e0, e1, M,
-                         N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks);
+                         dim3(tiles_m(M, ks, 96), cdiv(N, GEMM_DMA_BN)), dim3(64 * GEMM_DMA_WM * GEMM_DMA_WN), st, e0,
+                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks);
         if (fused) *fused = yf.csz > 0;
         return cdiv(N, GEMM_DMA_BN);
-    } else if ((long)cdiv(M, 96) * cdiv(N, 128) >= 192) {
-        if (!plan)
-            launch_timed(k_gemm_nt<96, 128, 2, 4, NN>, dim3(cdiv(M, 96), cdiv(N, 128)), dim3(512), st, e0, e1, M, N,
-                         K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
-        return cdiv(N, 128);
-    } else if ((long)cdiv(M, 64) * cdiv(N, 64) >= 96) {
-        if (!plan)
-            launch_timed(k_gemm_nt<64, 64, 2, 2, NN>, dim3(cdiv(M, 64), cdiv(N, 64)), dim3(256), st, e0, e1, M, N,
-                         K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
-        return cdiv(N, 64);
     }
-    if (!plan)
-        launch_timed(k_gemm_nt<32, 32, 2, 2, NN>, dim3(cdiv(M, 32), cdiv(N, 32)), dim3(256), st, e0, e1, M, N, K,
-                     A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
-    return cdiv(N, 32);
+    case TILE_32x64:
+        if (!plan)
+            launch_timed(k_gemm_dma<32, NN, 2, 4, 64, 32>, dim3(tiles_m(M, ks, 32), cdiv(N, 64)), dim3(512), st, e0,
+                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks);
+        return cdiv(N, 64);
+    default:
+        if (!plan)
+            launch_timed(k_gemm_dma<32, NN, 2, 2, 32, 32>, dim3(tiles_m(M, ks, 32), cdiv(N, 32)), dim3(256), st, e0,
+                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks);
+        return cdiv(N, 32);
+    }
 }
 
 void launch_gemm_nt(int M, int N, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc,
@@ -549,9 +651,10 @@ bool launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double*
 
 // Tile columns of the C = A * B launch these arguments get (the number of
 // gauge partials it writes).
-int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double* B, int ldb)
+int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double* B, int ldb, int ks)
 {
-    return launch_gemm<true>(M, N, K, A, lda, B, ldb, nullptr, 0, nullptr, 0, nullptr, nullptr, true);
+    return launch_gemm<true>(M, N, K, A, lda, B, ldb, nullptr, 0, nullptr, 0, nullptr, nullptr, true, nullptr, nullptr,
+                             nullptr, nullptr, ks);
 }
 
 // ---------------------------------------------------------------------------
@@ -561,6 +664,9 @@ int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double*
 // output element over k in the same order, so the transform results do not
 // depend on the shape; the gauge partials are one per tile column of the
 // shape in use (gemm_cfg_tile_n).
+// Shapes 0 and 1 are the direct-to-LDS kernel with 32 x 32 tiles of 4 waves
+// (the tiles of small single instances) and 64 x 64 tiles of 16, shape 2 the
+// register-staged kernel with 96 x 128 tiles.
 // Shapes 3 and 4 are the direct-to-LDS kernel with 96 x GEMM_DMA_BN tiles of
 // 16 waves (the single-instance transforms' shape, K-slices of GEMM_DMA_BK)
 // and 96 x 64 tiles of 8 waves, two workgroups per CU, with K-slices of 16
@@ -575,7 +681,7 @@ int gemm_cfg_tile_n(int cfg)
 // The shapes every instance of the batch can run: bit c set for cfg c.
 int gemm_cfg_mask(const FluidDev& F)
 {
-    int m = 7;
+    int m = 4;
     const bool yax = F.taxis == 1;
     const double* A = yax ? F.ymmi : F.dph + fidx(F, 1, 1);
     const double* Bm = yax ? F.dph + fidx(F, 1, 1) : F.zmmt;
@@ -585,7 +691,7 @@ int gemm_cfg_mask(const FluidDev& F)
     const double* A2 = yax ? F.ymm : F.hmn;
     const double* B2 = yax ? F.hmn : F.zmm;
     const bool ok2 = yax ? dma_ok<true>(F.n2m, F.n3m, K, A2, lda, B2, ldb) : dma_ok<false>(F.n2m, F.n3m, K, A2, F.P, B2, ldb);
-    if (ok1 && ok2) m |= 8 | 16;
+    if (ok1 && ok2) m |= 1 | 2 | 8 | 16;
     return m;
 }
 
@@ -605,7 +711,7 @@ static void launch_gemm_b(BatchSet& B, int key, const std::vector<GemmProb>& pr,
     default: break;
     }
     for (int i = 0; i < B.n; ++i) {
-        d[3 * i] = cdiv(pr[i].M, bm);
+        d[3 * i] = tiles_m(pr[i].M, pr[i].ks, bm);
         d[3 * i + 1] = cdiv(pr[i].N, bn);
         d[3 * i + 2] = 1;
     }
@@ -619,8 +725,8 @@ static void launch_gemm_b(BatchSet& B, int key, const std::vector<GemmProb>& pr,
         break;
     case 4: hipLaunchKernelGGL((kb_gemm_dma<16, NN, 2, 4, 64>), dim3(tot), dim3(512), 0, st, G); break;
     case 2: hipLaunchKernelGGL((kb_gemm_nt<96, 128, 2, 4, NN>), dim3(tot), dim3(512), 0, st, G); break;
-    case 1: hipLaunchKernelGGL((kb_gemm_nt<64, 64, 2, 2, NN>), dim3(tot), dim3(256), 0, st, G); break;
-    default: hipLaunchKernelGGL((kb_gemm_nt<32, 32, 2, 2, NN>), dim3(tot), dim3(256), 0, st, G); break;
+    case 1: hipLaunchKernelGGL((kb_gemm_dma<32, NN, 4, 4, 64, 64>), dim3(tot), dim3(1024), 0, st, G); break;
+    default: hipLaunchKernelGGL((kb_gemm_dma<32, NN, 2, 2, 32, 32>), dim3(tot), dim3(256), 0, st, G); break;
     }
 }
 

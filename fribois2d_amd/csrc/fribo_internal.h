@@ -252,7 +252,7 @@ bool launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double*
                     double* C, int ldc, const DevScalars* S, hipStream_t st, const double* zg = nullptr,
                     double* gpart = nullptr, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr,
                     const YFuse* yf = nullptr, int ks = 0);
-int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double* B, int ldb);
+int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double* B, int ldb, int ks);
 // first_done: the chunk pass already ran in the forward transform's epilogue
 void launch_ysolve(const FluidDev& F, hipStream_t st, bool first_done = false);
 void launch_loads(const FluidDev& F, double hpr, hipStream_t st);
