@@ -327,6 +327,7 @@ static void apply_ysh(fribo_ctx* c)
     FluidDev& F = c->F;
     F.ysh = (c->ymirror_on && c->ysh_avail > 0 && F.taxis == 1 && F.refine < 0) ? c->ysh_avail : 0;
     if (F.taxis == 1) F.ngpart = ngpart_for(c);
+    set_marching(F);
 }
 
 // Eigen-system of the y pressure operator (fribo_eig.hip) and the gauge
@@ -534,8 +535,10 @@ extern "C" int fribo_init(const fribo_params* p, const double* rc, const double*
     }
     F.ncfl = fribo_ncfl(F.n2m, F.n3m);
     if (!e) e = dalloc(c, &F.cfl_part, 2 * (size_t)F.ncfl);
-    F.npr_part = fribo_npr_part(F.n2m, F.n3m);
-    if (!e) e = dalloc(c, &F.pr_part, F.npr_part);
+    set_marching(F);
+    // room for the partials of either form (the mirror form's tiles cover the
+    // top half with its mirror image and may be shorter)
+    if (!e) e = dalloc(c, &F.pr_part, fribo_npr_part(F.n2m, F.n3m, 1));
     if (!e) e = setup_ksys(c, F.ks[0], F.n3m, 1, 0, 0);
     if (!e) e = setup_ksys(c, F.ks[1], F.n3m - 1, 2, 0, 0);
     if (!e) e = setup_ksys(c, F.js[0], F.n2 - 2, 2, 1, 1);
@@ -1791,6 +1794,7 @@ static int batch_refresh(fribo_batch_ctx* b)
         B.hF[i] = F;
         b->gen[i] = b->inst[i]->mk_gen;
     }
+    set_marching_batch(B.hF);
     HIPCHK(hipMemcpyAsync(B.dF, B.hF.data(), B.n * sizeof(FluidDev), hipMemcpyHostToDevice, b->st));
     HIPCHK(hipStreamSynchronize(b->st));
     if (b->gexec) {

@@ -171,6 +171,7 @@ enum {
     BK_COUNT
 };
 
+void set_marching_batch(std::vector<FluidDev>& F);
 void launch_cfl_b(BatchSet& B, hipStream_t st);
 void launch_bc_b(BatchSet& B, int n, bool mean, hipStream_t st);
 void launch_rhs_b(BatchSet& B, hipStream_t st);

@@ -20,20 +20,14 @@ inline int fribo_ncfl(int n2m, int n3m) { return ((n2m + 255) / 256) * ((n3m + F
 #define FRIBO_STATIC_LOADS_MAX_NLM 8192   // markers fribo_loads_transfer_static serves
 
 // Marching tiles of the stencil kernels (k_rhs, k_div, k_upd): a wave owns
-// FRIBO_WJ output columns (plus a halo lane each side) and MK planes
-// (FRIBO_MK_RHS for k_rhs, whose register window limits its occupancy;
-// FRIBO_MK for k_div and k_upd, whose shorter tiles put more waves in
-// flight).  k_upd writes one pressure partial per tile.
-#ifndef FRIBO_MK
-#define FRIBO_MK 8
-#endif
-#ifndef FRIBO_MK_RHS
-#define FRIBO_MK_RHS 16
-#endif
+// FRIBO_WJ output columns (plus a halo lane each side) and a number of planes
+// set by set_marching.  k_upd writes one pressure partial per tile.
+#define FRIBO_MK 8           // most planes of a tile of k_div and k_upd
+#define FRIBO_MK_RHS 16      // most planes of a tile of k_rhs, whose register window limits its occupancy
 #define FRIBO_WJ 62
-__host__ __device__ inline int fribo_npr_part(int n2m, int n3m)
+__host__ __device__ inline int fribo_npr_part(int ncol, int n3m, int mk)
 {
-    return ((n2m + FRIBO_WJ - 1) / FRIBO_WJ) * ((n3m + FRIBO_MK - 1) / FRIBO_MK);
+    return ((ncol + FRIBO_WJ - 1) / FRIBO_WJ) * ((n3m + mk - 1) / mk);
 }
 
 struct DevScalars {
@@ -132,7 +126,9 @@ struct FluidDev {
     double *cfl_part;        // [2*ncfl]
     int ncfl;                // CFL partials (workgroups of k_cfl)
     double *pr_part;         // [npr_part]
-    int npr_part;            // partials of k_upd (those of the mirror form's k_upd: npr_count)
+    int npr_part;            // partials of k_upd in the form in use
+    int mkr, mkd, mku;       // planes per tile of k_rhs, k_div, k_upd (set_marching)
+    int mkp;                 // planes per pressure partial of k_upd (mku is a multiple)
     // Helmholtz systems: ks[0] q2 along k, ks[1] q3 along k,
     // js[0] q2 along j, js[1] q3 along j; Poisson j-lines
     KSys ks[2];
@@ -275,6 +271,9 @@ int ytransform_mirror(int n, const double* am, const double* ac, const double* a
                       double* wys, double tol);
 int phini_sym(int n3, const double* zz, double alx3, int ld, double* zmm, double* zmmt, double* wr,
               bool device = false);
+// Planes per tile of the marching kernels and the number of pressure partials
+// for the form in use (F.ysh): one instance, and the instances of a batch.
+void set_marching(FluidDev& F);
 int jsolve_stride(const FluidDev& F);
 size_t jsolve_lds_bytes(const FluidDev& F);
 size_t sysprep_lds_bytes(const FluidDev& F);

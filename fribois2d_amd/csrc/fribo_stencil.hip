@@ -360,13 +360,6 @@ size_t sysprep_lds_bytes(const FluidDev& F)
     return (size_t)3 * (n + (n >> 5) + 1) * sizeof(double);
 }
 
-// Pressure partials k_upd leaves: one per tile (the mirror form's tiles
-// cover the top half with its mirror image, half as many).
-__device__ inline int npr_count(const FluidDev& F)
-{
-    return F.ysh > 0 ? fribo_npr_part(F.n2m / 2, F.n3m) : F.npr_part;
-}
-
 // The first PR_PRE pressure partials of thread t (entries t, t+1024, ...,
 // clamped to the last), loaded ahead so that they travel with the kernel's
 // other loads (8192 partials: the 2048x1536 grid has 6400, 3328 in the
@@ -374,7 +367,7 @@ __device__ inline int npr_count(const FluidDev& F)
 #define PR_PRE 8
 __device__ inline void pr_load(const FluidDev& F, double* v)
 {
-    const int t = threadIdx.x, n = npr_count(F);
+    const int t = threadIdx.x, n = F.npr_part;
 #pragma unroll
     for (int u = 0; u < PR_PRE; ++u) v[u] = F.pr_part[min(t + 1024 * u, n - 1)];
 }
@@ -385,7 +378,7 @@ __device__ inline void pr_load(const FluidDev& F, double* v)
 // flight at a time), then block_sum.  Fixed order.
 __device__ inline double pr_partial(const FluidDev& F, const double* v0)
 {
-    const int t = threadIdx.x, n = npr_count(F);
+    const int t = threadIdx.x, n = F.npr_part;
     double s = 0.0;
 #pragma unroll
     for (int u = 0; u < PR_PRE; ++u)
@@ -677,11 +670,8 @@ void launch_bc_b(BatchSet& B, int n, bool mean, hipStream_t st)
 // ---------------------------------------------------------------------------
 // Marching layout shared by k_rhs, k_div and k_upd: one 64-lane wave owns
 // columns j = 62*bx + lane (lanes 1..62 produce output, lanes 0 and 63 are
-// the j-1 / j+1 halo) and marches MK planes k = MK*by+1 .. MK*by+MK (MKR for
-// k_rhs), keeping a register window of the planes it needs; j-neighbours come
+// the j-1 / j+1 halo) and marches mk planes k = mk*by+1 .. mk*by+mk, keeping a register window of the planes it needs; j-neighbours come
 // from the adjacent lanes, so every field value is read from HBM once.
-#define MK FRIBO_MK
-#define MKR FRIBO_MK_RHS
 #define WJ FRIBO_WJ
 // Waves (tiles) per workgroup: adjacent tiles in j share their boundary
 // cache lines, which then come from the one L2 of the workgroup's XCD; the
@@ -699,7 +689,7 @@ void launch_bc_b(BatchSet& B, int n, bool mean, hipStream_t st)
 #ifndef SW_UPD
 #define SW_UPD 1
 #endif
-static_assert(MK <= 64 && MKR <= 64, "one plane of a tile per lane");
+static_assert(FRIBO_MK <= 64 && FRIBO_MK_RHS <= 64, "one plane of a tile per lane");
 
 // Single-instance launches of the marching kernels: the hardware hands
 // workgroups to the 8 XCDs round-robin by linear id, so the launch grid is
@@ -725,6 +715,55 @@ static inline dim3 xcd_pad(dim3 g)
     return dim3(g.x, (g.y + 7) / 8 * 8);
 }
 
+// Planes per tile: the most (whose halo planes are the smallest share) that
+// still give kMarchWaves waves, two per SIMD.  A wave's planes follow each
+// other at the latency of a load, so on small grids the tile's height sets
+// the time.  Times with 2048 waves wanted, against the tallest tiles (k_rhs
+// 16 planes, k_div and k_upd 8): 64x48 4.3/3.0/5.1 against 18.6/6.0/10.9 us,
+// 384x288 5.9/4.8/6.5 against 16.5/6.2/10.6, 810x672 11.9/5.3/11.3 against
+// 22.5/6.5/13.7; at 2048x1536 the tallest tiles give 3200 waves and shorter
+// ones lose (52.5/15.1/40.2 against 49.5/14.7/38.6).
+static constexpr int kMarchWaves = 2048;
+
+static int march_waves(const FluidDev& F, int ncol, int mk) { return fribo_npr_part(ncol, F.n3m, mk); }
+static int march_half(const FluidDev& F) { return F.ysh > 0 ? F.n2m / 2 : F.n2m; }
+
+void set_marching(FluidDev& F)
+{
+    const auto planes = [&](int ncol, int most) {
+        int mk = most;
+        while (mk > 1 && march_waves(F, ncol, mk) < kMarchWaves) mk /= 2;
+        return mk;
+    };
+    F.mkr = planes(F.n2m, FRIBO_MK_RHS);
+    F.mkd = F.mku = F.mkp = planes(march_half(F), FRIBO_MK);
+    F.npr_part = fribo_npr_part(march_half(F), F.n3m, F.mkp);
+}
+
+// The instances of a batch fill the chip together, so their tiles are as tall
+// as the batch's waves allow (24 instances of 96..448 x 70..380: k_upd 22.8
+// us against 42 with each instance's own height); the pressure partials stay
+// those of the instance alone, so its mean is the same bits.
+void set_marching_batch(std::vector<FluidDev>& F)
+{
+    const auto planes = [&](int most, bool whole) {
+        int mk = most;
+        for (; mk > 1; mk /= 2) {
+            long w = 0;
+            for (const auto& f : F) w += march_waves(f, whole ? f.n2m : march_half(f), mk);
+            if (w >= kMarchWaves) break;
+        }
+        return mk;
+    };
+    for (auto& f : F) set_marching(f);
+    const int mr = planes(FRIBO_MK_RHS, true), md = planes(FRIBO_MK, false);
+    for (auto& f : F) {
+        f.mkr = std::max(f.mkr, mr);
+        f.mkd = std::max(f.mkd, md);
+        f.mku = std::max(f.mkp, md);
+    }
+}
+
 __device__ inline double up1(double v) { return __shfl_up(v, 1, 64); }
 __device__ inline double dn1(double v) { return __shfl_down(v, 1, 64); }
 
@@ -739,10 +778,10 @@ __device__ __forceinline__ void rhs_body(const FluidDev& F, const VBlock& vb)
     const int ntj = (F.n2m + WJ - 1) / WJ, bx = (int)vb.x * SW_RHS + (int)(threadIdx.x >> 6);
     if (bx >= ntj) return;
     const int j = WJ * bx + lane;
-    const int k0 = MKR * vb.y + 1;
+    const int k0 = F.mkr * vb.y + 1;
     const int n2m = F.n2m, n3m = F.n3m;
     if (k0 > n3m) return;
-    const int k1 = min(k0 + MKR - 1, n3m);
+    const int k1 = min(k0 + F.mkr - 1, n3m);
     const bool inj = (j >= 1 && j <= F.n2);
     const bool out = (lane >= 1 && lane <= WJ && j <= n2m);
     const double dt = S->dt, ga = S->ga, ro = S->ro, al = S->al, alre = S->alre, pend = S->pend;
@@ -895,7 +934,7 @@ __device__ __forceinline__ void rhs_body(const FluidDev& F, const VBlock& vb)
 __global__ __launch_bounds__(64 * SW_RHS) void k_rhs(const FluidDev F)
 {
     VBlock vb = vb_hw();
-    if (vb_xcd_band(vb, (F.n3m + MKR - 1) / MKR)) rhs_body(F, vb);
+    if (vb_xcd_band(vb, (F.n3m + F.mkr - 1) / F.mkr)) rhs_body(F, vb);
 }
 __global__ __launch_bounds__(64 * SW_RHS) void kb_rhs(const BGrid<FluidDev> G)
 {
@@ -907,7 +946,7 @@ __global__ __launch_bounds__(64 * SW_RHS) void kb_rhs(const BGrid<FluidDev> G)
 static dim3 grid_rhs(const FluidDev& F)
 {
     const int ntj = (F.n2m + WJ - 1) / WJ;
-    return dim3((ntj + SW_RHS - 1) / SW_RHS, (F.n3m + MKR - 1) / MKR);
+    return dim3((ntj + SW_RHS - 1) / SW_RHS, (F.n3m + F.mkr - 1) / F.mkr);
 }
 
 void launch_rhs(const FluidDev& F, hipStream_t st)
@@ -938,9 +977,9 @@ __device__ __forceinline__ void div_body(const FluidDev& F, const VBlock& vb)
     const int ntj = (jtop + WJ - 1) / WJ, bx = (int)vb.x * SW_DIV + (int)(threadIdx.x >> 6);
     if (bx >= ntj) return;
     const int j = WJ * bx + lane;
-    const int k0 = MK * vb.y + 1;
+    const int k0 = F.mkd * vb.y + 1;
     if (k0 > F.n3m) return;
-    const int k1 = min(k0 + MK - 1, F.n3m);
+    const int k1 = min(k0 + F.mkd - 1, F.n3m);
     const bool inj = (j >= 1 && j <= F.n2);
     const bool out = (lane >= 1 && lane <= WJ && j <= jtop);
     const double usdtal = 1.0 / (S->dt * S->al);
@@ -993,7 +1032,7 @@ template <bool MIRROR>
 __global__ __launch_bounds__(64 * SW_DIV) void k_div(const FluidDev F)
 {
     VBlock vb = vb_hw();
-    if (vb_xcd_band(vb, (F.n3m + MK - 1) / MK)) div_body<MIRROR>(F, vb);
+    if (vb_xcd_band(vb, (F.n3m + F.mkd - 1) / F.mkd)) div_body<MIRROR>(F, vb);
 }
 __global__ __launch_bounds__(64 * SW_DIV) void kb_div(const BGrid<FluidDev> G)
 {
@@ -1007,7 +1046,7 @@ __global__ __launch_bounds__(64 * SW_DIV) void kb_div(const BGrid<FluidDev> G)
 static dim3 grid_div(const FluidDev& F)
 {
     const int ntj = ((F.ysh > 0 ? F.n2m / 2 : F.n2m) + WJ - 1) / WJ;
-    return dim3((ntj + SW_DIV - 1) / SW_DIV, (F.n3m + MK - 1) / MK);
+    return dim3((ntj + SW_DIV - 1) / SW_DIV, (F.n3m + F.mkd - 1) / F.mkd);
 }
 
 // The single-instance step passes F.ysh = 0 unless the mirror form runs
@@ -1045,10 +1084,11 @@ __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
     const int ntj = (jtop + WJ - 1) / WJ, bx = (int)vb.x * SW_UPD + (int)(threadIdx.x >> 6);
     if (bx >= ntj) return;
     const int j = WJ * bx + lane;
-    const int k0 = MK * vb.y + 1;
-    double part = 0.0;
+    const int k0 = F.mku * vb.y + 1;
     if (k0 <= F.n3m) {
-        const int k1 = min(k0 + MK - 1, F.n3m);
+        double part = 0.0;
+        const int mkp = F.mkp;
+        const int k1 = min(k0 + F.mku - 1, F.n3m);
         const bool inj = (j >= 1 && j <= F.n2);
         const bool out = (lane >= 1 && lane <= WJ && j <= jtop);
         const double al = S->al, dt = S->dt, pend = S->pend, be = al * S->beta;
@@ -1163,17 +1203,20 @@ __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
             dc = dp;
             dm_m = dc_m;
             dc_m = dp_m;
+            // end of a partial's planes: wave reduction (fixed order)
+            if (k % mkp == 0 || k == n3m) {
+                for (int off = 32; off > 0; off >>= 1) part = part + __shfl_xor(part, off, 64);
+                if (lane == 0) F.pr_part[(k - 1) / mkp * ntj + bx] = part;
+                part = 0.0;
+            }
         }
     }
-    // wave reduction (fixed order) -> one partial per workgroup
-    for (int off = 32; off > 0; off >>= 1) part = part + __shfl_xor(part, off, 64);
-    if (lane == 0) F.pr_part[vb.y * ntj + bx] = part;
 }
 template <bool MIRROR>
 __global__ __launch_bounds__(64 * SW_UPD) void k_upd(const FluidDev F)
 {
     VBlock vb = vb_hw();
-    if (vb_xcd_band(vb, (F.n3m + MK - 1) / MK)) upd_body<MIRROR>(F, vb);
+    if (vb_xcd_band(vb, (F.n3m + F.mku - 1) / F.mku)) upd_body<MIRROR>(F, vb);
 }
 __global__ __launch_bounds__(64 * SW_UPD) void kb_upd(const BGrid<FluidDev> G)
 {
@@ -1187,7 +1230,7 @@ __global__ __launch_bounds__(64 * SW_UPD) void kb_upd(const BGrid<FluidDev> G)
 static dim3 grid_upd(const FluidDev& F)
 {
     const int ntj = ((F.ysh > 0 ? F.n2m / 2 : F.n2m) + WJ - 1) / WJ;
-    return dim3((ntj + SW_UPD - 1) / SW_UPD, (F.n3m + MK - 1) / MK);
+    return dim3((ntj + SW_UPD - 1) / SW_UPD, (F.n3m + F.mku - 1) / F.mku);
 }
 
 void launch_upd(const FluidDev& F, hipStream_t st)
