@@ -188,7 +188,7 @@ def run_ensemble(args):
     mirror = [g.ymirror for g in gs]
     mk = EnsembleMarkers(cs)
     b = FluidBatch(gs)
-    best, tune_ms, tune_total = b.autotune(5)
+    best, tune_ms, _ = b.autotune(5)
     b.set_graph(args.launch == "graph")
     t = np.zeros(n)
     dt = np.array([c.params.dt0 for c in cs])
@@ -259,9 +259,7 @@ def run_ensemble(args):
                      "kernel": "kb_gemm (grouped forward transform)", "avg_ms": round(gemm_ms, 4),
                      "members_in_mirror_form": int(sum(mirror))},
         "autotune": {"shape": shapes.get(best, best),
-                     "ms_per_launch": {shapes[k]: round(float(v), 4) for k, v in enumerate(tune_ms) if v > 0},
-                     "ms_with_unfused_chunk_pass": {shapes[k]: round(float(v), 4)
-                                                    for k, v in enumerate(tune_total) if v > 0}},
+                     "ms_per_launch": {shapes[k]: round(float(v), 4) for k, v in enumerate(tune_ms) if v > 0}},
         "init_s": round(t_init, 1),
     }
     print(json.dumps(out))
@@ -487,17 +485,10 @@ def main():
                for k, v in prof_all.items() if v[1]}
     # HBM fraction of the memory-bound classes: compulsory FP64 field values
     # per cell per launch (reads + writes), at the 8 TB/s MI355X peak
-    # (the per-mode Poisson lines: along z one read and one write of hmn; along
-    # y the two chunk passes read it twice and write it once, unless the first
-    # pass runs in the forward transform's epilogue: equal chunks of at most
-    # 33 rows dividing its 64-column tiles, which the direct-to-LDS kernel
-    # takes at >= 192 tiles of 96x128)
-    nch = max(1, min(n3m // 2, 64))
-    csz = n3m // nch
-    fused = (axis == "y" and n3m % nch == 0 and 1 < csz <= 33 and 64 % csz == 0 and n3m % 64 == 0
-             and -(-n2m // 96) * -(-n3m // 128) >= 192)
+    # (the per-mode Poisson lines: one read and one write of hmn; along y the
+    # lines of more than 2048 rows take three passes, which read it twice)
     values = {"rhs": 9, "jsolve_helm": 4, "ksolve": 6, "div": 3,
-              "jsolve_poisson": (2 if fused else 3) if axis == "y" else 2,
+              "jsolve_poisson": 3 if axis == "y" and n3m > 2048 else 2,
               "upd": 7, "cfl": 2}
     for k, nv in values.items():
         if k in kernels and kernels[k]["ms_per_step"] > 0:

@@ -917,7 +917,7 @@ static void enqueue_poisson(fribo_ctx* c)
                 launch_gemm32(F.n2m, F.n3m, F.n2m, F.ymmi, F.ldy, d, F.P, F.hmn, F.P, nullptr, F.S, st, nullptr,
                               nullptr, a, b);
             });
-            run(c, PC_JP, [&] { launch_ysolve(F, st, false); });
+            run(c, PC_JP, [&] { launch_ysolve(F, st); });
             const bool last = it == F.refine;
             run_ev(c, PC_GEMM, [&](hipEvent_t a, hipEvent_t b) {
                 launch_gemm32(F.n2m, F.n3m, F.n2m, F.ymm, F.ldy, F.hmn, F.P, last ? d : xa, F.P,
@@ -936,33 +936,25 @@ static void enqueue_poisson(fribo_ctx* c)
         FluidDev Fm = F;
         Fm.wy = F.wys;
         Fm.ynull = F.ynulls;
-        YFuse yf{F.wys, F.amphk, F.acphk, F.apphk, F.ysum, F.n2m, 0};
-        if (F.n3m % F.ks[0].nch == 0) yf.csz = F.n3m / F.ks[0].nch;
-        bool fused = false;
         run_ev(c, PC_GEMM, [&](hipEvent_t a, hipEvent_t b) {
-            fused = launch_gemm_nn(F.n2m, F.n3m, F.n2m, F.ysmi, F.ldy, d, F.P, F.hmn, F.P, F.S, st, nullptr, nullptr,
-                                   a, b, &yf, F.ysh);
+            launch_gemm_nn(F.n2m, F.n3m, F.n2m, F.ysmi, F.ldy, d, F.P, F.hmn, F.P, F.S, st, nullptr, nullptr, a, b,
+                           F.ysh);
         });
-        run(c, PC_JP, [&] { launch_ysolve(Fm, st, fused); });
+        run(c, PC_JP, [&] { launch_ysolve(Fm, st); });
         run_ev(c, PC_GEMM, [&](hipEvent_t a, hipEvent_t b) {
             launch_gemm_nn(F.n2m, F.n3m, F.n2m, F.ysm, F.ldy, F.hmn, F.P, d, F.P, F.S, st, F.zg, F.gpart, a, b,
-                           nullptr, F.ysh);
+                           F.ysh);
         });
         c->dph_mirror = true;
         return;
     }
     if (F.taxis == 1) {
         c->dph_mirror = false;
-        // the chunk pass of the per-mode z-lines runs in the forward
-        // transform's epilogue when the line partition has equal chunks
-        YFuse yf{F.wy, F.amphk, F.acphk, F.apphk, F.ysum, F.n2m, 0};
-        if (F.n3m % F.ks[0].nch == 0) yf.csz = F.n3m / F.ks[0].nch;
-        bool fused = false;
         run_ev(c, PC_GEMM, [&](hipEvent_t a, hipEvent_t b) {
-            fused = launch_gemm_nn(F.n2m, F.n3m, F.n2m, F.ymmi, F.ldy, F.dph + fidx(F, 1, 1), F.P, F.hmn, F.P, F.S,
-                                   st, nullptr, nullptr, a, b, &yf);
+            launch_gemm_nn(F.n2m, F.n3m, F.n2m, F.ymmi, F.ldy, F.dph + fidx(F, 1, 1), F.P, F.hmn, F.P, F.S, st,
+                           nullptr, nullptr, a, b);
         });
-        run(c, PC_JP, [&] { launch_ysolve(F, st, fused); });
+        run(c, PC_JP, [&] { launch_ysolve(F, st); });
         run_ev(c, PC_GEMM, [&](hipEvent_t a, hipEvent_t b) {
             launch_gemm_nn(F.n2m, F.n3m, F.n2m, F.ymm, F.ldy, F.hmn, F.P, F.dph + fidx(F, 1, 1), F.P, F.S, st, F.zg,
                            F.gpart, a, b);
@@ -1702,9 +1694,7 @@ static BGrid<FluidDev> batch_grid(BatchSet* B, int key, const std::vector<int>& 
 static bool same_prob(const GemmProb& a, const GemmProb& b)
 {
     return a.M == b.M && a.N == b.N && a.K == b.K && a.lda == b.lda && a.ldb == b.ldb && a.ldc == b.ldc &&
-           a.A == b.A && a.B == b.B && a.C == b.C && a.S == b.S && a.zg == b.zg && a.gpart == b.gpart &&
-           a.yf.wy == b.yf.wy && a.yf.amphk == b.yf.amphk && a.yf.acphk == b.yf.acphk && a.yf.apphk == b.yf.apphk &&
-           a.yf.ysum == b.yf.ysum && a.yf.n2m == b.yf.n2m && a.yf.csz == b.yf.csz && a.ks == b.ks;
+           a.A == b.A && a.B == b.B && a.C == b.C && a.S == b.S && a.zg == b.zg && a.gpart == b.gpart && a.ks == b.ks;
 }
 
 static bool same_probs(const std::vector<GemmProb>& a, const std::vector<GemmProb>& b)
@@ -1778,9 +1768,6 @@ static int batch_refresh(fribo_batch_ctx* b)
 {
     BatchSet& B = b->B;
     B.gemm_cfg = b->gemm_fixed >= 0 ? b->gemm_fixed : batch_default_gemm(b);
-    bool fuse = B.gemm_cfg == 3 || B.gemm_cfg == 4;
-    for (auto h : b->inst) fuse = fuse && gemm_fuse_ok(h->F, B.gemm_cfg);
-    B.ysolve_fused = fuse;
     for (int i = 0; i < B.n; ++i) {
         FluidDev F = b->inst[i]->F;
         F.jstride = jsolve_stride_for(F, b->jclass);
@@ -1988,8 +1975,8 @@ static void batch_enqueue(fribo_batch_ctx* b)
         launch_jsolve_helm_b(B, st);
         launch_ksolve_b(B, st);
         launch_div_b(B, st);
-        const bool fused = launch_poisson_gemm_b(B, true, st);
-        if (B.hF[0].taxis == 1) launch_ysolve_b(B, st, fused);
+        launch_poisson_gemm_b(B, true, st);
+        if (B.hF[0].taxis == 1) launch_ysolve_b(B, st);
         else launch_jsolve_poisson_b(B, st);
         launch_poisson_gemm_b(B, false, st);
         launch_upd_b(B, st);
@@ -2092,8 +2079,8 @@ extern "C" int fribo_batch_get_gemm_shape(fribo_batch b)
 // every instance (its output hmn is scratch between steps; nothing of the
 // state changes) with each shape all instances can run, reps timed launches
 // after one untimed, on the batch's own problems; the fastest shape is kept.
-// ms[5] receives the mean time per grouped launch of shapes 0..4 (0 where a
-// shape is not available).
+// ms[10] receives the mean time per grouped launch of shapes 0..4 twice (0
+// where a shape is not available).
 extern "C" int fribo_batch_autotune(fribo_batch b, int32_t reps, double* ms, int32_t* best_out)
 {
     if (!b || reps < 1) return set_err(FRIBO_ERR_ARG, "bad autotune arguments");
@@ -2114,29 +2101,18 @@ extern "C" int fribo_batch_autotune(fribo_batch b, int32_t reps, double* ms, int
             b->gemm_fixed = keep;
             return e;
         }
-        // the forward transform alone, then with the chunk pass of the
-        // per-mode z-lines where this shape does not run it in the
-        // transform's epilogue (the time that decides)
-        float tt[2] = {0.0f, 0.0f};
-        for (int pass = 0; pass < 2; ++pass) {
-            auto fwd = [&] {
-                const bool fused = launch_poisson_gemm_b(b->B, true, b->st);
-                if (pass == 1 && !fused && b->B.hF[0].taxis == 1) launch_ysolve1_b(b->B, b->st);
-            };
-            fwd();
-            HIPCHK(hipEventRecord(e0, b->st));
-            for (int r = 0; r < reps; ++r) fwd();
-            HIPCHK(hipEventRecord(e1, b->st));
-            HIPCHK(hipEventSynchronize(e1));
-            HIPCHK(hipGetLastError());
-            HIPCHK(hipEventElapsedTime(&tt[pass], e0, e1));
-            tt[pass] /= (float)reps;
-        }
-        const float t = tt[1];
-        if (ms) {
-            ms[cfg] = tt[0];
-            ms[5 + cfg] = tt[1];
-        }
+        float t = 0.0f;
+        launch_poisson_gemm_b(b->B, true, b->st);
+        HIPCHK(hipEventRecord(e0, b->st));
+        for (int r = 0; r < reps; ++r) launch_poisson_gemm_b(b->B, true, b->st);
+        HIPCHK(hipEventRecord(e1, b->st));
+        HIPCHK(hipEventSynchronize(e1));
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipEventElapsedTime(&t, e0, e1));
+        t /= (float)reps;
+        // no shape leaves a pass of the z-lines to another kernel, so both
+        // figures of a shape are the transform's
+        if (ms) ms[cfg] = ms[5 + cfg] = t;
         if (best < 0 || t < best_ms) {
             best = cfg;
             best_ms = t;

@@ -94,7 +94,6 @@ struct GemmProb {
     const DevScalars* S;
     const double* zg;
     double* gpart;
-    YFuse yf;
     int ks;   // mirror form: split point of the block-diagonal A (0: plain)
 };
 
@@ -112,7 +111,6 @@ struct BatchSet {
     void* owner = nullptr;
     // choices shared by all instances (largest size class over the batch)
     int gemm_cfg = 0;        // 0: 32x32 tiles, 1: 64x64, 2: 96x128, 3: direct-to-LDS 96x128, 4: direct-to-LDS 96x64
-    bool ysolve_fused = false;
 
     BGrid<FluidDev> grid(int key, const std::vector<int>& dims) { return grid_fn(this, key, dims); }
     BGrid<GemmProb> gemm(int key, const std::vector<GemmProb>& p, const std::vector<int>& dims)
@@ -167,7 +165,7 @@ inline void blaunch_xcd(BatchSet& B, int key, const std::vector<int>& dims, Kern
 // Stage keys of the launch tables.
 enum {
     BK_CFL, BK_BC, BK_RHS, BK_DIV, BK_UPD, BK_MEAN, BK_MLS_IDX, BK_MLS_SUP, BK_MLS_ORDER, BK_MLS_INTERP,
-    BK_MLS_SPREAD, BK_JH, BK_JP, BK_K1, BK_K2, BK_K3, BK_KF, BK_Y1, BK_Y2, BK_Y3, BK_GEMM_F, BK_GEMM_B, BK_IO,
+    BK_MLS_SPREAD, BK_JH, BK_JP, BK_K1, BK_K2, BK_K3, BK_KF, BK_Y1, BK_Y2, BK_Y3, BK_YF, BK_GEMM_F, BK_GEMM_B, BK_IO,
     BK_COUNT
 };
 
@@ -183,16 +181,13 @@ void launch_mls_force_b(BatchSet& B, hipStream_t st);
 void launch_jsolve_helm_b(BatchSet& B, hipStream_t st);
 void launch_jsolve_poisson_b(BatchSet& B, hipStream_t st);
 void launch_ksolve_b(BatchSet& B, hipStream_t st);
-void launch_ysolve_b(BatchSet& B, hipStream_t st, bool first_done);
-// the first (chunk) pass of the batched per-mode z-lines alone
-void launch_ysolve1_b(BatchSet& B, hipStream_t st);
+void launch_ysolve_b(BatchSet& B, hipStream_t st);
 // transforms of the Poisson solve: forward (fwd) or backward, the axis of
-// the instances (all alike); returns true when the fused chunk pass ran
-bool launch_poisson_gemm_b(BatchSet& B, bool fwd, hipStream_t st);
+// the instances (all alike)
+void launch_poisson_gemm_b(BatchSet& B, bool fwd, hipStream_t st);
 int jsolve_class_h(const FluidDev& F);
 int gemm_cfg_mask(const FluidDev& F);
 int gemm_cfg_parts(const FluidDev& F, int cfg);
-bool gemm_fuse_ok(const FluidDev& F, int cfg);
 int jsolve_stride_for(const FluidDev& F, int mh);
 // true when every instance can use the counting-sort marker order
 bool mls_batchable(const FluidDev& F);

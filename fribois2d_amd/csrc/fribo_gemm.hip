@@ -62,7 +62,6 @@
 // whose B operand is the field itself, k-contiguous) the B slice is read as
 // 16-double runs of each column and stored with a row pitch of BN+1, which
 // spreads the transposing LDS stores over the banks.
-#include "fribo_ychunk.h"
 #include "fribo_batch.h"
 #include <hip/hip_ext.h>
 
@@ -322,7 +321,7 @@ __device__ inline void dma16(const double* base, unsigned off, unsigned lds)
 }
 
 template <int BK, bool NN, int WM = 2, int WN = 8, int BN = 128, int BM = 96>
-__device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double* __restrict__ A, int lda, const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc, const DevScalars* S, const double* __restrict__ zg, double* gpart, YFuse yf, int ks, const VBlock& vb)
+__device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double* __restrict__ A, int lda, const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc, const DevScalars* S, const double* __restrict__ zg, double* gpart, int ks, const VBlock& vb)
 {
     constexpr int NST = 3;                                  // stages
     constexpr int NW = WM * WN;
@@ -342,10 +341,7 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
     static_assert(TM % 16 == 0 && TN % 16 == 0 && BM % WM == 0 && BN % WN == 0, "wave tile");
     static_assert(BK == 16 || BK == 24 || BK == 32, "k-slices");
     if (S && S->err) return;
-    // the stages in one block, which the fused epilogue of the NN form
-    // reuses for the tile (BN rows of pitch BM + 1)
-    constexpr int SMN = NST * (SA + SBP), STN = NN && BM == 96 ? BN * (BM + 1) : 0;
-    __shared__ __attribute__((aligned(1024))) double SM[SMN > STN ? SMN : STN];
+    __shared__ __attribute__((aligned(1024))) double SM[NST * (SA + SBP)];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave % WM, wn = wave / WM;
     int bx = vb.x, by = vb.y;
@@ -499,51 +495,18 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
         __shared__ double gsh[NW];
         gauge_partials<RM, RN, TM, TN, NW>(acc, ks, M, N, tr, n0, wm, wn, lane, wave, by, vb.gy, zg, gpart, gsh);
     }
-    if constexpr (NN && BM == 96)
-    if (yf.csz > 0) {
-        // chunk elimination of the y-mode z-lines on this tile: rows i are
-        // y-modes, columns n the z rows; the tile holds BN / csz whole chunks
-        constexpr int LT = BM + 1;   // LDS row pitch of the staged tile (one z row per LDS row)
-        lds_barrier();   // no DMA is in flight after the last slice
-#pragma unroll
-        for (int r = 0; r < RM; ++r)
-#pragma unroll
-            for (int c = 0; c < RN; ++c)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    SM[(wn * TN + c * 16 + (lane >> 4) + 4 * v) * LT + wm * TM + r * 16 + (lane & 15)] = acc[r][c][v];
-        lds_barrier();
-        constexpr int WPC = (BM + 63) / 64;   // waves per chunk
-        const int csz = yf.csz, cc = wave / WPC, iw = (wave % WPC) * 64 + lane;
-        if (cc < BN / csz) {                  // wave-uniform
-            const int il = iw < BM ? iw : BM - 1;
-            const int ic = min(i0 + il, M - 1);
-            const int p = (n0 + cc * csz) / csz, s = p * csz, m = csz - 1;
-            const double* col = SM + (size_t)(cc * csz) * LT + il;
-            double dv[32];
-#pragma unroll
-            for (int q = 0; q < 32; ++q) dv[q] = col[(q < m ? q : 0) * LT];
-            const double w = yf.wy[ic];
-            double yl, vl, ys, vs, ws, wl;
-            ychunk_rows<32, false>(yf.amphk, yf.acphk, yf.apphk, s, m, w, dv, nullptr, nullptr, nullptr, yl, vl,
-                                   ys, vs, ws, wl);
-            if (iw < BM && i0 + iw >= tr.lo && i0 + iw < tr.hi)
-                ysum_store(yf.ysum, yf.n2m, i0 + iw + 1, p, yf.amphk, yf.acphk, s + m, w, col[m * LT], yl, vl, wl,
-                           ys, vs, ws);
-        }
-    }
 }
 template <int BK, bool NN, int WM = 2, int WN = 8, int BN = 128, int BM = 96>
-__global__ __launch_bounds__(64 * WM * WN) void k_gemm_dma(int M, int N, int K, const double* __restrict__ A, int lda, const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc, const DevScalars* S, const double* __restrict__ zg, double* gpart, YFuse yf, int ks)
+__global__ __launch_bounds__(64 * WM * WN) void k_gemm_dma(int M, int N, int K, const double* __restrict__ A, int lda, const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc, const DevScalars* S, const double* __restrict__ zg, double* gpart, int ks)
 {
-    gemm_dma_body<BK, NN, WM, WN, BN, BM>(M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks, vb_hw());
+    gemm_dma_body<BK, NN, WM, WN, BN, BM>(M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks, vb_hw());
 }
 template <int BK, bool NN, int WM = 2, int WN = 8, int BN = 128, int BM = 96>
 __global__ __launch_bounds__(64 * WM * WN) void kb_gemm_dma(const BGrid<GemmProb> G)
 {
     VBlock vb;
     const GemmProb& P = *bg_block(G, vb);
-    gemm_dma_body<BK, NN, WM, WN, BN, BM>(P.M, P.N, P.K, P.A, P.lda, P.B, P.ldb, P.C, P.ldc, P.S, P.zg, P.gpart, P.yf, P.ks, vb);
+    gemm_dma_body<BK, NN, WM, WN, BN, BM>(P.M, P.N, P.K, P.A, P.lda, P.B, P.ldb, P.C, P.ldc, P.S, P.zg, P.gpart, P.ks, vb);
 }
 
 static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -593,10 +556,8 @@ static int gemm_tile(int M, int N, int ks)
 template <bool NN>
 static int launch_gemm(int M, int N, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc,
                        const DevScalars* S, hipStream_t st, const double* zg, double* gpart, bool plan,
-                       hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, const YFuse* yfp = nullptr,
-                       bool* fused = nullptr, int ks = 0)
+                       hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, int ks = 0)
 {
-    if (fused) *fused = false;
     if (!dma_ok<NN>(M, N, K, A, lda, B, ldb)) {
         // operands without 16-byte alignment (host callers' own leading dimensions)
         if (!plan)
@@ -604,32 +565,22 @@ static int launch_gemm(int M, int N, int K, const double* A, int lda, const doub
                          N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
         return cdiv(N, 32);
     }
-    YFuse yf{};
     switch (gemm_tile(M, N, ks)) {
-    case TILE_96x128: {
-        // the fused chunk pass needs whole chunks of at most 33 rows in every
-        // output tile, and no more chunks per tile than the epilogue has wave
-        // groups (one group of (96 + 63) / 64 waves per chunk)
-        constexpr int kChunkGroups = (GEMM_DMA_WM * GEMM_DMA_WN) / ((96 + 63) / 64);
-        if (NN && yfp && yfp->csz > 1 && yfp->csz <= 33 && GEMM_DMA_BN % yfp->csz == 0 && N % GEMM_DMA_BN == 0 &&
-            GEMM_DMA_BN / yfp->csz <= kChunkGroups)
-            yf = *yfp;
+    case TILE_96x128:
         if (!plan)
             launch_timed(k_gemm_dma<GEMM_DMA_BK, NN, GEMM_DMA_WM, GEMM_DMA_WN, GEMM_DMA_BN>,
                          dim3(tiles_m(M, ks, 96), cdiv(N, GEMM_DMA_BN)), dim3(64 * GEMM_DMA_WM * GEMM_DMA_WN), st, e0,
-                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks);
-        if (fused) *fused = yf.csz > 0;
+                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
         return cdiv(N, GEMM_DMA_BN);
-    }
     case TILE_32x64:
         if (!plan)
             launch_timed(k_gemm_dma<32, NN, 2, 4, 64, 32>, dim3(tiles_m(M, ks, 32), cdiv(N, 64)), dim3(512), st, e0,
-                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks);
+                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
         return cdiv(N, 64);
     default:
         if (!plan)
             launch_timed(k_gemm_dma<32, NN, 2, 2, 32, 32>, dim3(tiles_m(M, ks, 32), cdiv(N, 32)), dim3(256), st, e0,
-                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, yf, ks);
+                         e1, M, N, K, A, lda, B, ldb, C, ldc, S, zg, gpart, ks);
         return cdiv(N, 32);
     }
 }
@@ -640,13 +591,11 @@ void launch_gemm_nt(int M, int N, int K, const double* A, int lda, const double*
     launch_gemm<false>(M, N, K, A, lda, B, ldb, C, ldc, S, st, nullptr, nullptr, false, e0, e1);
 }
 
-bool launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc,
+void launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc,
                     const DevScalars* S, hipStream_t st, const double* zg, double* gpart, hipEvent_t e0,
-                    hipEvent_t e1, const YFuse* yf, int ks)
+                    hipEvent_t e1, int ks)
 {
-    bool fused = false;
-    launch_gemm<true>(M, N, K, A, lda, B, ldb, C, ldc, S, st, zg, gpart, false, e0, e1, yf, &fused, ks);
-    return fused;
+    launch_gemm<true>(M, N, K, A, lda, B, ldb, C, ldc, S, st, zg, gpart, false, e0, e1, ks);
 }
 
 // Tile columns of the C = A * B launch these arguments get (the number of
@@ -654,7 +603,7 @@ bool launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double*
 int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double* B, int ldb, int ks)
 {
     return launch_gemm<true>(M, N, K, A, lda, B, ldb, nullptr, 0, nullptr, 0, nullptr, nullptr, true, nullptr, nullptr,
-                             nullptr, nullptr, ks);
+                             ks);
 }
 
 // ---------------------------------------------------------------------------
@@ -730,11 +679,10 @@ static void launch_gemm_b(BatchSet& B, int key, const std::vector<GemmProb>& pr,
     }
 }
 
-bool launch_poisson_gemm_b(BatchSet& B, bool fwd, hipStream_t st)
+void launch_poisson_gemm_b(BatchSet& B, bool fwd, hipStream_t st)
 {
     const bool yax = B.hF[0].taxis == 1;
     std::vector<GemmProb> pr(B.n);
-    bool fused = false;
     for (int i = 0; i < B.n; ++i) {
         const FluidDev& F = B.hF[i];
         GemmProb& q = pr[i];
@@ -755,9 +703,6 @@ bool launch_poisson_gemm_b(BatchSet& B, bool fwd, hipStream_t st)
             if (!fwd) {
                 q.zg = F.zg;
                 q.gpart = F.gpart;
-            } else if (B.ysolve_fused) {
-                q.yf = YFuse{F.wy, F.amphk, F.acphk, F.apphk, F.ysum, F.n2m, F.n3m / F.ks[0].nch};
-                fused = true;
             }
         } else {
             q.K = F.n3m;
@@ -771,21 +716,6 @@ bool launch_poisson_gemm_b(BatchSet& B, bool fwd, hipStream_t st)
     }
     if (yax) launch_gemm_b<true>(B, fwd ? BK_GEMM_F : BK_GEMM_B, pr, st);
     else launch_gemm_b<false>(B, fwd ? BK_GEMM_F : BK_GEMM_B, pr, st);
-    return fused;
-}
-
-// The fused chunk pass is possible for an instance when its line partition
-// has equal chunks that fill the direct-to-LDS kernel's output tiles of batch
-// shape cfg (3 or 4), and the tile has a group of (96 + 63) / 64 waves per
-// chunk.
-bool gemm_fuse_ok(const FluidDev& F, int cfg)
-{
-    if (cfg != 3 && cfg != 4) return false;
-    const int bn = gemm_cfg_tile_n(cfg), waves = cfg == 3 ? GEMM_DMA_WM * GEMM_DMA_WN : 8;
-    const int groups = waves / ((96 + 63) / 64);
-    if (F.taxis != 1 || F.n3m % F.ks[0].nch != 0) return false;
-    const int csz = F.n3m / F.ks[0].nch;
-    return csz > 1 && csz <= 33 && bn % csz == 0 && F.n3m % bn == 0 && bn / csz <= groups;
 }
 
 // ---------------------------------------------------------------------------

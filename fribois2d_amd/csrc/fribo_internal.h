@@ -183,6 +183,27 @@ __device__ inline double lane_bcast(double v, int l)
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// Raw buffer access to a field: a uniform descriptor plus one 32-bit byte
+// offset per lane (a 64-bit address would take two registers per row).
+typedef unsigned int kf_u32x2 __attribute__((ext_vector_type(2)));
+__device__ inline __amdgpu_buffer_rsrc_t kf_rsrc(const double* base)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(base), 0, 0x7fffffff, 0x00020000);
+}
+// voff: per-lane byte offset; soff: uniform byte offset (a scalar register)
+__device__ inline double kf_load(__amdgpu_buffer_rsrc_t r, int voff, int soff = 0)
+{
+    const kf_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+    return __hiloint2double((int)v.y, (int)v.x);
+}
+__device__ inline void kf_store(__amdgpu_buffer_rsrc_t r, int voff, double d, int soff = 0)
+{
+    kf_u32x2 v;
+    v.x = (unsigned)__double2loint(d);
+    v.y = (unsigned)__double2hiint(d);
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, soff, 0);
+}
+
 // 1/x from the hardware estimate refined by two Newton steps (within an ulp
 // of the rounded quotient for the pivots of the diagonally dominant line
 // systems, far from zero and from the denormal range).  A fraction of the
@@ -228,29 +249,16 @@ void launch_jsolve_poisson(const FluidDev& F, hipStream_t st);
 void launch_ksolve(const FluidDev& F, hipStream_t st);
 // true when both k-systems have chunks of at most 32 rows (the one-pass form)
 bool ksolve_fused_fits(const FluidDev& F);
-// First pass of the y-order z-lines (chunk elimination, fribo_ychunk.h) run
-// by the epilogue of the forward transform on its own output tile, when
-// every 64-column tile holds whole chunks of the line partition (csz rows
-// each, csz - 1 <= 32).  csz = 0: no fused pass.
-struct YFuse {
-    const double *wy, *amphk, *acphk, *apphk;
-    double* ysum;
-    int n2m, csz;
-};
-
 // e0/e1 (optional): events the dispatch records at its start and end
 void launch_gemm_nt(int M, int N, int K, const double* A, int lda, const double* B, int ldb,
                     double* C, int ldc, const DevScalars* S, hipStream_t st, hipEvent_t e0 = nullptr,
                     hipEvent_t e1 = nullptr);
-// Returns true when the fused chunk pass of yf ran (yf->csz > 0 and the
-// direct-to-LDS kernel with 64-column tiles took the launch).
-bool launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double* B, int ldb,
+void launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double* B, int ldb,
                     double* C, int ldc, const DevScalars* S, hipStream_t st, const double* zg = nullptr,
-                    double* gpart = nullptr, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr,
-                    const YFuse* yf = nullptr, int ks = 0);
+                    double* gpart = nullptr, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, int ks = 0);
 int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double* B, int ldb, int ks);
-// first_done: the chunk pass already ran in the forward transform's epilogue
-void launch_ysolve(const FluidDev& F, hipStream_t st, bool first_done = false);
+// The per-mode z-lines of the y-order Poisson solve, hmn in place.
+void launch_ysolve(const FluidDev& F, hipStream_t st);
 void launch_loads(const FluidDev& F, double hpr, hipStream_t st);
 // mixed-precision Poisson solve: r = rhs - (A_y + A_z) x (r may alias rhs),
 // and the FP32 transform C = X0 + A * B (X0 optional, may alias C)

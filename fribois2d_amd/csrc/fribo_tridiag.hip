@@ -1008,27 +1008,6 @@ __device__ inline void kf_unroll(std::integer_sequence<int, I...>, Fn fn)
     (fn(std::integral_constant<int, I>{}), ...);
 }
 
-// Raw buffer access to a field: a uniform descriptor plus one 32-bit byte
-// offset per lane (a 64-bit address would take two registers per row).
-typedef unsigned int kf_u32x2 __attribute__((ext_vector_type(2)));
-__device__ inline __amdgpu_buffer_rsrc_t kf_rsrc(const double* base)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(base), 0, 0x7fffffff, 0x00020000);
-}
-// voff: per-lane byte offset; soff: uniform byte offset (a scalar register)
-__device__ inline double kf_load(__amdgpu_buffer_rsrc_t r, int voff, int soff = 0)
-{
-    const kf_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-    return __hiloint2double((int)v.y, (int)v.x);
-}
-__device__ inline void kf_store(__amdgpu_buffer_rsrc_t r, int voff, double d, int soff = 0)
-{
-    kf_u32x2 v;
-    v.x = (unsigned)__double2loint(d);
-    v.y = (unsigned)__double2hiint(d);
-    __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, soff, 0);
-}
-
 template <int MAXM>
 __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBlock& vb)
 {

@@ -1,8 +1,6 @@
 // Chunk elimination of the per-y-mode z-lines of the y-order Poisson solve
 // (the shifted operator A_z + wy(j) of phcalc_outflow.F90:34-56 restated
-// along z), shared by the line kernels of fribo_ysolve.hip and by the
-// epilogue of the forward transform GEMM, which runs the first pass on its
-// own output tile.
+// along z) in the three-pass form of fribo_ysolve.hip.
 #pragma once
 #include "fribo_internal.h"
 

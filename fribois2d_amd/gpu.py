@@ -509,8 +509,8 @@ class FluidBatch:
 
     def autotune(self, reps=5):
         """Pick the transform tile shape by timing; returns (best, ms per
-        shape of the transform alone, ms per shape with the chunk pass of
-        the per-mode z-lines that the shape does not fuse, which decides)."""
+        shape of the transform, and the same again: the figure that
+        decides)."""
         ms = np.zeros(10)
         best = C.c_int32(-1)
         _check(load().fribo_batch_autotune(self.b, int(reps), _dp(ms), C.byref(best)))

@@ -49,3 +49,26 @@ def test_mirror_form_projects(n2m):
     g.fluid_tsch(0, p.dt0)
     assert g.diagnostics()["divmax"] <= 1e-10
     g.close()
+
+
+@pytest.mark.parametrize("n3m", [6, 127, 129, 512, 513, 1024, 1025, 2048, 2049])
+@pytest.mark.parametrize("n2m", [5, 14])
+def test_mode_lines_project(n3m, n2m):
+    """The per-mode z-lines at the edges of their chunk classes (chunks of 2
+    to 8, 9 to 16 and 17 to 32 rows in one pass, longer ones in three).  A
+    step ends divergence-free to rounding: the condition number of the Poisson
+    operator times 2^-53 of the divergence the step starts from, and 2^-53
+    over the spacing; 16 times that is allowed."""
+    from fribois2d_amd import cases
+    from fribois2d_amd.gpu import FluidStep
+    rc, zz = np.linspace(0.0, 6.0, n2m + 1), np.linspace(0.0, 8.0, n3m + 1)
+    p = cases.FluidParams(n2=n2m + 1, n3=n3m + 1, alx3=8.0, rext2=6.0, visc=0.02, ibact=False)
+    g = FluidStep(p, rc, zz)
+    assert g.transform == ("y" if n2m < n3m else "z")
+    g.set_state(cases.initial_state(p, 9))
+    div0 = g.diagnostics()["divmax"]
+    g.fluid_tsch(0, p.dt0)
+    hy, hz = 6.0 / n2m, 8.0 / n3m
+    kappa = (4.0 / hy ** 2 + 4.0 / hz ** 2) / (np.pi / 8.0) ** 2
+    assert g.diagnostics()["divmax"] <= 16.0 * 2.0 ** -53 * (kappa * div0 + 1.0 / min(hy, hz))
+    g.close()
