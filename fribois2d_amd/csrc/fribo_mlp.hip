@@ -6,26 +6,37 @@
 // the network only proposes where it starts.
 //
 // Network: NI inputs -> H tanh -> H tanh -> NO linear outputs (H = 64), FP32
-// parameters laid out as [W1 (H x NI, row-major), b1 (H), W2 (H x H), b2 (H),
-// W3 (NO x H), b3 (NO)].
+// parameters [W1 (H x NI, row-major), b1 (H), W2 (H x H), b2 (H), W3 (NO x H),
+// b3 (NO)] at the C ABI.  On the device W1 and W2 are stored transposed (input
+// by input, the 64 units side by side), so that every access of 64 lanes, one
+// per unit, is one run; fribo_mlp_create and the read-backs convert.
 //
-// Training (FP32): one step over a minibatch of B samples is three launches:
-//   k_mlp_fwd   one workgroup per sample: the two hidden layers and the
-//               outputs, kept for the backward pass;
-//   k_mlp_bwd   one workgroup per sample: output error of the mean squared
-//               loss and the back-propagated errors of both hidden layers;
-//   k_mlp_adam  one thread per parameter: its gradient summed over the
-//               minibatch in sample order (deterministic) and the Adam update.
+// Training (FP32): the samples of a call go to the device once; one step over
+// a minibatch is two launches and no synchronisation:
+//   k_mlp_step  workgroups of MLP_NS samples: both hidden layers, the outputs,
+//               the back-propagated errors of the mean squared loss, and the
+//               workgroup's part of the gradient, with the weights in LDS;
+//   k_mlp_adam  one thread per parameter: the parts added in workgroup order
+//               (deterministic) and the Adam update.
+// A minibatch of 256 at NI = 45: 94 -> 16.7 us a step (65 us of the 94 one
+// kernel that added 256 samples per parameter one after the other, the rest
+// two pageable copies and a synchronisation).
 // Inference (BF16): k_mlp_infer rounds inputs, weights and hidden
-// activations to bfloat16 and accumulates in FP32; one workgroup per sample.
+// activations to bfloat16 and accumulates in FP32.  Small sets are read from
+// and written to pinned host memory by the kernel itself: one proposal 33 -> 21 us.
 #include "fribo_internal.h"
 
 #include <algorithm>
 #include <cmath>
-#include <string>
+#include <cstring>
+#include <new>
 #include <vector>
 
 #define MLP_H 64
+#define MLP_NS 8             // samples per workgroup, one per wave
+#define MLP_NT (64 * MLP_NS) // threads per workgroup
+#define MLP_PARTS 128        // most gradient parts of a minibatch
+#define MLP_LDW (MLP_H + 1)  // LDS row pitch of W2: read along rows and columns
 
 struct MlpDims {
     int ni, no;
@@ -55,128 +66,227 @@ __device__ inline float bf16r(float x)
     return __uint_as_float(u & 0xffff0000u);
 }
 
-__global__ __launch_bounds__(MLP_H) void k_mlp_fwd(MlpDims d, const float* __restrict__ p, const float* __restrict__ X,
-                                                   float* __restrict__ H1, float* __restrict__ H2,
-                                                   float* __restrict__ Y)
+// Weights and samples of a workgroup in LDS (dynamic; floats).
+struct MlpLds {
+    float *w1, *b1, *w2, *b2, *w3, *b3, *x, *h1, *h2, *y, *d1, *d2;
+};
+__host__ __device__ inline size_t mlp_lds_floats(const MlpDims& d)
 {
-    __shared__ float xs[256], h1[MLP_H], h2[MLP_H];
-    const int b = blockIdx.x, u = threadIdx.x;
-    for (int i = u; i < d.ni; i += MLP_H) xs[i] = X[(size_t)b * d.ni + i];
-    __syncthreads();
-    float s = p[d.b1 + u];
-    for (int i = 0; i < d.ni; ++i) s += p[d.w1 + u * d.ni + i] * xs[i];
-    h1[u] = tanhf(s);
-    H1[(size_t)b * MLP_H + u] = h1[u];
-    __syncthreads();
-    s = p[d.b2 + u];
-    for (int i = 0; i < MLP_H; ++i) s += p[d.w2 + u * MLP_H + i] * h1[i];
-    h2[u] = tanhf(s);
-    H2[(size_t)b * MLP_H + u] = h2[u];
-    __syncthreads();
-    if (u < d.no) {
-        s = p[d.b3 + u];
-        for (int i = 0; i < MLP_H; ++i) s += p[d.w3 + u * MLP_H + i] * h2[i];
-        Y[(size_t)b * d.no + u] = s;
+    return (size_t)MLP_H * d.ni + MLP_H + MLP_H * MLP_LDW + MLP_H + (size_t)d.no * MLP_H + 16 +
+           (size_t)MLP_NS * d.ni + 4 * MLP_NS * MLP_H + MLP_NS * 16;
+}
+__device__ inline MlpLds mlp_lds(const MlpDims& d, float* l)
+{
+    MlpLds m;
+    m.x = l;                       l += MLP_NS * d.ni;   // [ni][MLP_NS]: first, for 16-byte reads
+    m.w1 = l;                      l += MLP_H * d.ni;    // [ni][H]
+    m.b1 = l;                      l += MLP_H;
+    m.w2 = l;                      l += MLP_H * MLP_LDW; // [H inputs][MLP_LDW]
+    m.b2 = l;                      l += MLP_H;
+    m.w3 = l;                      l += d.no * MLP_H;    // [no][H]
+    m.b3 = l;                      l += 16;
+    m.h1 = l;                      l += MLP_NS * MLP_H;  // [MLP_NS][H]
+    m.h2 = l;                      l += MLP_NS * MLP_H;
+    m.d1 = l;                      l += MLP_NS * MLP_H;
+    m.d2 = l;                      l += MLP_NS * MLP_H;
+    m.y = l;                                             // [MLP_NS][16]
+    return m;
+}
+
+// Stages the parameters (rounded to bfloat16 for inference); every array of
+// the device layout but b3 starts and ends on 16 bytes.
+template <bool BF16>
+__device__ inline void mlp_stage(const MlpDims& d, const float* __restrict__ p, const MlpLds& m)
+{
+    const int t = threadIdx.x;
+    auto r4 = [](float4 v) {
+        return BF16 ? make_float4(bf16r(v.x), bf16r(v.y), bf16r(v.z), bf16r(v.w)) : v;
+    };
+    const float4* const w1 = (const float4*)(p + d.w1);
+    const float4* const w2 = (const float4*)(p + d.w2);
+    const float4* const w3 = (const float4*)(p + d.w3);
+#pragma unroll 4
+    for (int q = t; q < MLP_H / 4 * d.ni; q += MLP_NT) ((float4*)m.w1)[q] = r4(w1[q]);
+#pragma unroll
+    for (int q = t; q < MLP_H * MLP_H / 4; q += MLP_NT) {
+        const float4 v = r4(w2[q]);
+        float* const o = m.w2 + (q >> 4) * MLP_LDW + 4 * (q & 15);
+        o[0] = v.x;
+        o[1] = v.y;
+        o[2] = v.z;
+        o[3] = v.w;
+    }
+    if (t < MLP_H / 4 * d.no) ((float4*)m.w3)[t] = r4(w3[t]);
+    if (t < MLP_H) {
+        m.b1[t] = BF16 ? bf16r(p[d.b1 + t]) : p[d.b1 + t];
+        m.b2[t] = BF16 ? bf16r(p[d.b2 + t]) : p[d.b2 + t];
+    }
+    if (t < d.no) m.b3[t] = BF16 ? bf16r(p[d.b3 + t]) : p[d.b3 + t];
+}
+
+// Inputs of the samples [b0, b0 + MLP_NS) below B, zeros past them; wave g
+// takes sample g.
+template <bool BF16>
+__device__ inline void mlp_inputs(const MlpDims& d, const float* __restrict__ X, int b0, int B, const MlpLds& m)
+{
+    const int s = threadIdx.x >> 6;
+    for (int i = threadIdx.x & 63; i < d.ni; i += 64) {
+        const float x = b0 + s < B ? X[(size_t)(b0 + s) * d.ni + i] : 0.0f;
+        m.x[i * MLP_NS + s] = BF16 ? bf16r(x) : x;
     }
 }
 
-// Errors of the loss L = (1 / (B NO)) sum (Y - T)^2 with respect to the
-// pre-activations: D3 = dL/dY, D2 and D1 of the hidden layers.
-__global__ __launch_bounds__(MLP_H) void k_mlp_bwd(MlpDims d, const float* __restrict__ p, int B,
-                                                   const float* __restrict__ T, const float* __restrict__ H1,
-                                                   const float* __restrict__ H2, const float* __restrict__ Y,
-                                                   float* __restrict__ D1, float* __restrict__ D2,
-                                                   float* __restrict__ D3)
+// Both hidden layers and the outputs (m.y) of the staged samples: wave g
+// takes sample g, lane u unit u; sums in input order from the bias on.
+template <bool BF16>
+__device__ inline void mlp_forward(const MlpDims& d, const MlpLds& m)
 {
-    __shared__ float d3[16], d2[MLP_H];
-    const int b = blockIdx.x, u = threadIdx.x;
+    const int t = threadIdx.x, u = t & 63, s = t >> 6;
+    float a = m.b1[u];
+#pragma unroll 8
+    for (int i = 0; i < d.ni; ++i) a = fmaf(m.w1[i * MLP_H + u], m.x[i * MLP_NS + s], a);
+    a = tanhf(a);
+    m.h1[s * MLP_H + u] = BF16 ? bf16r(a) : a;
+    __syncthreads();
+    a = m.b2[u];
+#pragma unroll 16
+    for (int i = 0; i < MLP_H; ++i) a = fmaf(m.w2[i * MLP_LDW + u], m.h1[s * MLP_H + i], a);
+    a = tanhf(a);
+    m.h2[s * MLP_H + u] = BF16 ? bf16r(a) : a;
+    __syncthreads();
+    if (u < d.no) {
+        float y = m.b3[u];
+#pragma unroll 16
+        for (int i = 0; i < MLP_H; ++i) y = fmaf(m.w3[u * MLP_H + i], m.h2[s * MLP_H + i], y);
+        m.y[s * 16 + u] = y;
+    }
+    __syncthreads();
+}
+
+// Forward and backward of a minibatch of B samples, loss
+// L = (1 / (B NO)) sum (Y - T)^2: workgroup g takes the groups of MLP_NS
+// samples g, g + parts, ... and leaves its part of the gradient (device
+// layout) in G + g * np; Y (optional) receives the outputs.
+__global__ __launch_bounds__(MLP_NT) void k_mlp_step(MlpDims d, const float* __restrict__ p, int B,
+                                                     const float* __restrict__ X, const float* __restrict__ T,
+                                                     float* __restrict__ G, float* __restrict__ Y)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const MlpLds m = mlp_lds(d, lds);
+    const int u = threadIdx.x & 63, g = threadIdx.x >> 6;
     const float sc = 2.0f / (float)(B * d.no);
-    if (u < d.no) {
-        d3[u] = sc * (Y[(size_t)b * d.no + u] - T[(size_t)b * d.no + u]);
-        D3[(size_t)b * d.no + u] = d3[u];
+    float* const part = G + (size_t)blockIdx.x * d.np;
+    mlp_stage<false>(d, p, m);
+    for (int b0 = blockIdx.x * MLP_NS; b0 < B; b0 += gridDim.x * MLP_NS) {
+        const bool first = b0 == (int)blockIdx.x * MLP_NS;
+        const int b = b0 + g;   // the wave's sample
+        mlp_inputs<false>(d, X, b0, B, m);
+        const float tgt = u < d.no && b < B ? T[(size_t)b * d.no + u] : 0.0f;
+        __syncthreads();
+        mlp_forward<false>(d, m);
+        // output errors in place of the outputs
+        if (u < d.no) {
+            const float y = m.y[g * 16 + u];
+            if (b < B && Y) Y[(size_t)b * d.no + u] = y;
+            m.y[g * 16 + u] = b < B ? sc * (y - tgt) : 0.0f;
+        }
+        __syncthreads();
+        float a = 0.0f;
+        for (int o = 0; o < d.no; ++o) a = fmaf(m.w3[o * MLP_H + u], m.y[g * 16 + o], a);
+        float h = m.h2[g * MLP_H + u];
+        m.d2[g * MLP_H + u] = a * (1.0f - h * h);
+        __syncthreads();
+        a = 0.0f;
+        // unit o's weight of input u
+#pragma unroll 16
+        for (int o = 0; o < MLP_H; ++o) a = fmaf(m.w2[u * MLP_LDW + o], m.d2[g * MLP_H + o], a);
+        h = m.h1[g * MLP_H + u];
+        m.d1[g * MLP_H + u] = a * (1.0f - h * h);
+        __syncthreads();
+        // gradient parts: lane u, wave g takes every MLP_NS-th input
+        float e1[MLP_NS], e2[MLP_NS];
+#pragma unroll
+        for (int s = 0; s < MLP_NS; ++s) {
+            e1[s] = m.d1[s * MLP_H + u];
+            e2[s] = m.d2[s * MLP_H + u];
+        }
+        auto put = [&](int q, float v) { part[q] = first ? v : part[q] + v; };
+#pragma unroll 4
+        for (int i = g; i < d.ni; i += MLP_NS) {
+            float v = 0.0f;
+#pragma unroll
+            for (int s = 0; s < MLP_NS; ++s) v = fmaf(e1[s], m.x[i * MLP_NS + s], v);
+            put(d.w1 + i * MLP_H + u, v);
+        }
+#pragma unroll
+        for (int i = g; i < MLP_H; i += MLP_NS) {
+            float v = 0.0f;
+#pragma unroll
+            for (int s = 0; s < MLP_NS; ++s) v = fmaf(e2[s], m.h1[s * MLP_H + i], v);
+            put(d.w2 + i * MLP_H + u, v);
+        }
+        for (int o = g; o < d.no; o += MLP_NS) {
+            float v = 0.0f;
+#pragma unroll
+            for (int s = 0; s < MLP_NS; ++s) v = fmaf(m.y[s * 16 + o], m.h2[s * MLP_H + u], v);
+            put(d.w3 + o * MLP_H + u, v);
+        }
+        if (g == 0) {
+            float v1 = 0.0f, v2 = 0.0f;
+#pragma unroll
+            for (int s = 0; s < MLP_NS; ++s) {
+                v1 += e1[s];
+                v2 += e2[s];
+            }
+            put(d.b1 + u, v1);
+            put(d.b2 + u, v2);
+            if (u < d.no) {
+                float v3 = 0.0f;
+#pragma unroll
+                for (int s = 0; s < MLP_NS; ++s) v3 += m.y[s * 16 + u];
+                put(d.b3 + u, v3);
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    float s = 0.0f;
-    for (int o = 0; o < d.no; ++o) s += p[d.w3 + o * MLP_H + u] * d3[o];
-    const float h2 = H2[(size_t)b * MLP_H + u];
-    d2[u] = s * (1.0f - h2 * h2);
-    D2[(size_t)b * MLP_H + u] = d2[u];
-    __syncthreads();
-    s = 0.0f;
-    for (int o = 0; o < MLP_H; ++o) s += p[d.w2 + o * MLP_H + u] * d2[o];
-    const float h1 = H1[(size_t)b * MLP_H + u];
-    D1[(size_t)b * MLP_H + u] = s * (1.0f - h1 * h1);
 }
 
-// Gradient of parameter q (summed over the B samples in order) and, when
-// lr > 0, the Adam step t (bias-corrected moments); grad (optional) receives
-// the gradient.
-__device__ inline float mlp_grad(const MlpDims& d, int q, int B, const float* X, const float* H1, const float* H2,
-                                 const float* D1, const float* D2, const float* D3)
-{
-    float g = 0.0f;
-    if (q < d.b1) {
-        const int u = (q - d.w1) / d.ni, i = (q - d.w1) % d.ni;
-        for (int b = 0; b < B; ++b) g += D1[(size_t)b * MLP_H + u] * X[(size_t)b * d.ni + i];
-    } else if (q < d.w2) {
-        const int u = q - d.b1;
-        for (int b = 0; b < B; ++b) g += D1[(size_t)b * MLP_H + u];
-    } else if (q < d.b2) {
-        const int u = (q - d.w2) / MLP_H, i = (q - d.w2) % MLP_H;
-        for (int b = 0; b < B; ++b) g += D2[(size_t)b * MLP_H + u] * H1[(size_t)b * MLP_H + i];
-    } else if (q < d.w3) {
-        const int u = q - d.b2;
-        for (int b = 0; b < B; ++b) g += D2[(size_t)b * MLP_H + u];
-    } else if (q < d.b3) {
-        const int o = (q - d.w3) / MLP_H, i = (q - d.w3) % MLP_H;
-        for (int b = 0; b < B; ++b) g += D3[(size_t)b * d.no + o] * H2[(size_t)b * MLP_H + i];
-    } else {
-        const int o = q - d.b3;
-        for (int b = 0; b < B; ++b) g += D3[(size_t)b * d.no + o];
-    }
-    return g;
-}
-
-__global__ __launch_bounds__(256) void k_mlp_adam(MlpDims d, float* __restrict__ p, float* __restrict__ m1,
-                                                  float* __restrict__ m2, int B, const float* __restrict__ X,
-                                                  const float* __restrict__ H1, const float* __restrict__ H2,
-                                                  const float* __restrict__ D1, const float* __restrict__ D2,
-                                                  const float* __restrict__ D3, float lr, float c1, float c2,
-                                                  float* __restrict__ grad)
+// Gradient of every parameter (the parts in workgroup order) and, when
+// lr > 0, the Adam step t (c1, c2: bias corrections); grad (optional)
+// receives the gradient.
+__global__ __launch_bounds__(256) void k_mlp_adam(int np, float* __restrict__ p, float* __restrict__ m1,
+                                                  float* __restrict__ m2, int parts, const float* __restrict__ G,
+                                                  float lr, float c1, float c2, float* __restrict__ grad)
 {
     const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= d.np) return;
-    const float g = mlp_grad(d, q, B, X, H1, H2, D1, D2, D3);
+    if (q >= np) return;
+    float g = 0.0f;
+    const float a1 = m1[q], a2 = m2[q], pq = p[q];
+#pragma unroll 16
+    for (int w = 0; w < parts; ++w) g += G[(size_t)w * np + q];
     if (grad) grad[q] = g;
     if (lr <= 0.0f) return;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float a = b1 * m1[q] + (1.0f - b1) * g;
-    const float v = b2 * m2[q] + (1.0f - b2) * g * g;
+    const float a = b1 * a1 + (1.0f - b1) * g;
+    const float v = b2 * a2 + (1.0f - b2) * g * g;
     m1[q] = a;
     m2[q] = v;
-    p[q] -= lr * (a * c1) / (sqrtf(v * c2) + eps);
+    p[q] = pq - lr * (a * c1) / (sqrtf(v * c2) + eps);
 }
 
-__global__ __launch_bounds__(MLP_H) void k_mlp_infer(MlpDims d, const float* __restrict__ p,
-                                                     const float* __restrict__ X, float* __restrict__ Y)
+// BF16 inference of n samples (products of two bfloat16 values are exact in
+// FP32, so the fused accumulation rounds as a separate one does).
+__global__ __launch_bounds__(MLP_NT) void k_mlp_infer(MlpDims d, const float* __restrict__ p, int n,
+                                                      const float* __restrict__ X, float* __restrict__ Y)
 {
-    __shared__ float xs[256], h1[MLP_H], h2[MLP_H];
-    const int b = blockIdx.x, u = threadIdx.x;
-    for (int i = u; i < d.ni; i += MLP_H) xs[i] = bf16r(X[(size_t)b * d.ni + i]);
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const MlpLds m = mlp_lds(d, lds);
+    const int u = threadIdx.x & 63, b = blockIdx.x * MLP_NS + (threadIdx.x >> 6);
+    mlp_inputs<true>(d, X, blockIdx.x * MLP_NS, n, m);
+    mlp_stage<true>(d, p, m);
     __syncthreads();
-    float s = bf16r(p[d.b1 + u]);
-    for (int i = 0; i < d.ni; ++i) s += bf16r(p[d.w1 + u * d.ni + i]) * xs[i];
-    h1[u] = bf16r(tanhf(s));
-    __syncthreads();
-    s = bf16r(p[d.b2 + u]);
-    for (int i = 0; i < MLP_H; ++i) s += bf16r(p[d.w2 + u * MLP_H + i]) * h1[i];
-    h2[u] = bf16r(tanhf(s));
-    __syncthreads();
-    if (u < d.no) {
-        s = bf16r(p[d.b3 + u]);
-        for (int i = 0; i < MLP_H; ++i) s += bf16r(p[d.w3 + u * MLP_H + i]) * h2[i];
-        Y[(size_t)b * d.no + u] = s;
-    }
+    mlp_forward<true>(d, m);
+    if (u < d.no && b < n) Y[(size_t)b * d.no + u] = m.y[(threadIdx.x >> 6) * 16 + u];
 }
 
 // ---------------------------------------------------------------------------
@@ -184,38 +294,44 @@ __global__ __launch_bounds__(MLP_H) void k_mlp_infer(MlpDims d, const float* __r
 struct fribo_mlp_ctx {
     MlpDims d;
     hipStream_t st = nullptr;
-    float *p = nullptr, *m1 = nullptr, *m2 = nullptr;
-    int cap = 0;    // samples the work buffers hold
-    float *X = nullptr, *T = nullptr, *H1 = nullptr, *H2 = nullptr, *Y = nullptr, *D1 = nullptr, *D2 = nullptr,
-          *D3 = nullptr, *G = nullptr;
-    long step = 0;  // Adam steps taken
+    float *p = nullptr, *m1 = nullptr, *m2 = nullptr, *g = nullptr;   // one allocation, device layout
+    float* work = nullptr;       // device work space of `cap` floats
+    size_t cap = 0;
+    float* pin = nullptr;        // pinned host memory: MLP_PIN floats and the staged parameters
+    long step = 0;               // Adam steps taken
 };
 typedef fribo_mlp_ctx* fribo_mlp;
 
-static void mlp_free_work(fribo_mlp m)
+// Floats of pinned memory a network keeps (64 KB): the largest set whose
+// inputs and outputs the inference kernel reads and writes on the host.
+#define MLP_PIN 16384
+
+static int mlp_reserve(fribo_mlp m, size_t floats)
 {
-    float** w[] = {&m->X, &m->T, &m->H1, &m->H2, &m->Y, &m->D1, &m->D2, &m->D3};
-    for (auto q : w) {
-        if (*q) hipFree(*q);
-        *q = nullptr;
-    }
+    if (floats <= m->cap) return 0;
+    if (m->work) hipFree(m->work);
+    m->work = nullptr;
     m->cap = 0;
+    if (hipMalloc(&m->work, floats * sizeof(float)) != hipSuccess) return FRIBO_E_HIP;
+    m->cap = floats;
+    return 0;
 }
 
-static int mlp_reserve(fribo_mlp m, int n)
+// Device layout <-> C ABI layout of parameters and gradients.
+static void mlp_layout(const MlpDims& d, const float* src, float* dst, bool to_device)
 {
-    if (n <= m->cap) return 0;
-    mlp_free_work(m);
-    const size_t ni = m->d.ni, no = m->d.no, H = MLP_H;
-    const size_t sz[] = {ni, no, H, H, no, H, H, no};
-    float** w[] = {&m->X, &m->T, &m->H1, &m->H2, &m->Y, &m->D1, &m->D2, &m->D3};
-    for (int i = 0; i < 8; ++i)
-        if (hipMalloc(w[i], (size_t)n * sz[i] * sizeof(float)) != hipSuccess) {
-            mlp_free_work(m);
-            return FRIBO_E_HIP;
-        }
-    m->cap = n;
-    return 0;
+    auto turn = [&](int o, int ncol) {   // H x ncol rows at the ABI, ncol x H on the device
+        for (int u = 0; u < MLP_H; ++u)
+            for (int i = 0; i < ncol; ++i) {
+                const int a = o + u * ncol + i, b = o + i * MLP_H + u;
+                if (to_device) dst[b] = src[a];
+                else dst[a] = src[b];
+            }
+    };
+    turn(d.w1, d.ni);
+    std::copy(src + d.b1, src + d.w2, dst + d.b1);
+    turn(d.w2, MLP_H);
+    std::copy(src + d.b2, src + d.np, dst + d.b2);
 }
 
 // Network with ni inputs (<= 256) and no outputs (<= 16); parameters from
@@ -226,9 +342,10 @@ extern "C" int fribo_mlp_create(int32_t ni, int32_t no, const float* init, uint6
     if (!out || ni < 1 || ni > 256 || no < 1 || no > 16) return FRIBO_E_ARG;
     fribo_mlp m = new fribo_mlp_ctx();
     m->d = mlp_dims(ni, no);
-    std::vector<float> p0(m->d.np, 0.0f);
+    const MlpDims& d = m->d;
+    std::vector<float> p0(d.np, 0.0f);
     if (init) {
-        std::copy(init, init + m->d.np, p0.begin());
+        std::copy(init, init + d.np, p0.begin());
     } else {
         uint64_t s = seed ? seed : 0x9e3779b97f4a7c15ull;
         auto uni = [&s]() {   // splitmix64 -> [-1, 1)
@@ -240,23 +357,27 @@ extern "C" int fribo_mlp_create(int32_t ni, int32_t no, const float* init, uint6
         };
         const float a1 = std::sqrt(6.0f / (ni + MLP_H)), a2 = std::sqrt(6.0f / (2 * MLP_H)),
                     a3 = std::sqrt(6.0f / (MLP_H + no));
-        for (int q = m->d.w1; q < m->d.b1; ++q) p0[q] = a1 * uni();
-        for (int q = m->d.w2; q < m->d.b2; ++q) p0[q] = a2 * uni();
-        for (int q = m->d.w3; q < m->d.b3; ++q) p0[q] = a3 * uni();
+        for (int q = d.w1; q < d.b1; ++q) p0[q] = a1 * uni();
+        for (int q = d.w2; q < d.b2; ++q) p0[q] = a2 * uni();
+        for (int q = d.w3; q < d.b3; ++q) p0[q] = a3 * uni();
     }
-    const size_t nb = (size_t)m->d.np * sizeof(float);
-    if (hipStreamCreate(&m->st) != hipSuccess || hipMalloc(&m->p, nb) != hipSuccess ||
-        hipMalloc(&m->m1, nb) != hipSuccess || hipMalloc(&m->m2, nb) != hipSuccess ||
-        hipMalloc(&m->G, nb) != hipSuccess || hipMemcpy(m->p, p0.data(), nb, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(m->m1, 0, nb) != hipSuccess || hipMemset(m->m2, 0, nb) != hipSuccess) {
+    // parameters, both moments (zero) and the gradient in one allocation; the
+    // upload is staged past the pinned memory of the inference and not waited for
+    const size_t nb = (size_t)d.np * sizeof(float);
+    if (hipStreamCreate(&m->st) != hipSuccess || hipMalloc(&m->p, 4 * nb) != hipSuccess ||
+        hipHostMalloc((void**)&m->pin, MLP_PIN * sizeof(float) + nb, hipHostMallocDefault) != hipSuccess ||
+        (mlp_layout(d, p0.data(), m->pin + MLP_PIN, true), false) ||
+        hipMemcpyAsync(m->p, m->pin + MLP_PIN, nb, hipMemcpyHostToDevice, m->st) != hipSuccess ||
+        hipMemsetAsync(m->p + d.np, 0, 2 * nb, m->st) != hipSuccess) {
         if (m->p) hipFree(m->p);
-        if (m->m1) hipFree(m->m1);
-        if (m->m2) hipFree(m->m2);
-        if (m->G) hipFree(m->G);
+        if (m->pin) hipHostFree(m->pin);
         if (m->st) hipStreamDestroy(m->st);
         delete m;
         return FRIBO_E_HIP;
     }
+    m->m1 = m->p + d.np;
+    m->m2 = m->m1 + d.np;
+    m->g = m->m2 + d.np;
     *out = m;
     return 0;
 }
@@ -265,11 +386,9 @@ extern "C" int fribo_mlp_destroy(fribo_mlp m)
 {
     if (!m) return FRIBO_E_ARG;
     hipStreamSynchronize(m->st);
-    mlp_free_work(m);
+    if (m->work) hipFree(m->work);
     hipFree(m->p);
-    hipFree(m->m1);
-    hipFree(m->m2);
-    hipFree(m->G);
+    hipHostFree(m->pin);
     hipStreamDestroy(m->st);
     delete m;
     return 0;
@@ -280,56 +399,78 @@ extern "C" int fribo_mlp_size(fribo_mlp m)
     return m ? m->d.np : -1;
 }
 
-extern "C" int fribo_mlp_get_params(fribo_mlp m, float* out)
+// A device array of np floats in the ABI's layout.
+static int mlp_fetch(fribo_mlp m, const float* dev, float* out)
 {
-    if (!m || !out) return FRIBO_E_ARG;
-    if (hipMemcpy(out, m->p, (size_t)m->d.np * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
+    std::vector<float> v(m->d.np);
+    if (hipMemcpyAsync(v.data(), dev, v.size() * sizeof(float), hipMemcpyDeviceToHost, m->st) != hipSuccess ||
+        hipStreamSynchronize(m->st) != hipSuccess)
         return FRIBO_E_HIP;
+    mlp_layout(m->d, v.data(), out, false);
     return 0;
 }
 
-// One pass over n samples (X n x ni, T n x no, row-major): forward, backward
-// and, with lr > 0, one Adam step of the whole set as the minibatch.  grad
-// (optional, np floats) receives the gradient of the mean squared loss,
-// loss (optional) its value.
-static int mlp_pass(fribo_mlp m, int n, const float* X, const float* T, float lr, float* grad, float* loss)
+extern "C" int fribo_mlp_get_params(fribo_mlp m, float* out)
 {
-    if (!m || n < 1 || !X || !T) return FRIBO_E_ARG;
-    if (mlp_reserve(m, n)) return FRIBO_E_HIP;
+    if (!m || !out) return FRIBO_E_ARG;
+    return mlp_fetch(m, m->p, out);
+}
+
+// Passes over n samples (X n x ni, T n x no, row-major) in minibatches of
+// `batch`, `epochs` times: forward, backward and, with lr > 0, one Adam step
+// per minibatch.  grad (optional, np floats) receives the last minibatch's
+// gradient of the mean squared loss, loss (optional) its value.
+static int mlp_run(fribo_mlp m, int n, const float* X, const float* T, int epochs, int batch, float lr, float* grad,
+                   float* loss)
+{
     const MlpDims& d = m->d;
-    if (hipMemcpyAsync(m->X, X, (size_t)n * d.ni * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess ||
-        hipMemcpyAsync(m->T, T, (size_t)n * d.no * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess)
+    batch = std::min(batch, n);
+    const int most = std::min((batch + MLP_NS - 1) / MLP_NS, MLP_PARTS);
+    const size_t nx = (size_t)n * d.ni, nt = (size_t)n * d.no, ny = loss ? (size_t)batch * d.no : 0;
+    if (mlp_reserve(m, nx + nt + ny + (size_t)most * d.np)) return FRIBO_E_HIP;
+    float *dX = m->work, *dT = dX + nx, *dY = dT + nt, *dG = dY + ny;
+    if (hipMemcpyAsync(dX, X, nx * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess ||
+        hipMemcpyAsync(dT, T, nt * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess)
         return FRIBO_E_HIP;
-    hipLaunchKernelGGL(k_mlp_fwd, dim3(n), dim3(MLP_H), 0, m->st, d, (const float*)m->p, (const float*)m->X, m->H1,
-                       m->H2, m->Y);
-    hipLaunchKernelGGL(k_mlp_bwd, dim3(n), dim3(MLP_H), 0, m->st, d, (const float*)m->p, n, (const float*)m->T,
-                       (const float*)m->H1, (const float*)m->H2, (const float*)m->Y, m->D1, m->D2, m->D3);
-    float c1 = 1.0f, c2 = 1.0f;
-    if (lr > 0.0f) {
-        ++m->step;
-        c1 = 1.0f / (1.0f - std::pow(0.9f, (float)m->step));
-        c2 = 1.0f / (1.0f - std::pow(0.999f, (float)m->step));
-    }
-    hipLaunchKernelGGL(k_mlp_adam, dim3((d.np + 255) / 256), dim3(256), 0, m->st, d, m->p, m->m1, m->m2, n,
-                       (const float*)m->X, (const float*)m->H1, (const float*)m->H2, (const float*)m->D1,
-                       (const float*)m->D2, (const float*)m->D3, lr, c1, c2, grad ? m->G : (float*)nullptr);
+    const size_t lds = mlp_lds_floats(d) * sizeof(float);
+    int b = 0, s = 0;
+    for (int e = 0; e < epochs; ++e)
+        for (s = 0; s < n; s += batch) {
+            b = std::min(batch, n - s);
+            const bool last = e == epochs - 1 && s + batch >= n;
+            const int parts = std::min((b + MLP_NS - 1) / MLP_NS, MLP_PARTS);
+            hipLaunchKernelGGL(k_mlp_step, dim3(parts), dim3(MLP_NT), lds, m->st, d, (const float*)m->p, b,
+                               (const float*)dX + (size_t)s * d.ni, (const float*)dT + (size_t)s * d.no, dG,
+                               last && loss ? dY : (float*)nullptr);
+            float c1 = 1.0f, c2 = 1.0f;
+            if (lr > 0.0f) {
+                ++m->step;
+                c1 = 1.0f / (1.0f - std::pow(0.9f, (float)m->step));
+                c2 = 1.0f / (1.0f - std::pow(0.999f, (float)m->step));
+            }
+            hipLaunchKernelGGL(k_mlp_adam, dim3((d.np + 255) / 256), dim3(256), 0, m->st, d.np, m->p, m->m1, m->m2,
+                               parts, (const float*)dG, lr, c1, c2, grad && last ? m->g : (float*)nullptr);
+            if (last) break;
+        }
     if (hipGetLastError() != hipSuccess) return FRIBO_E_HIP;
-    if (grad && hipMemcpyAsync(grad, m->G, (size_t)d.np * sizeof(float), hipMemcpyDeviceToHost, m->st) != hipSuccess)
-        return FRIBO_E_HIP;
     std::vector<float> y;
     if (loss) {
-        y.resize((size_t)n * d.no);
-        if (hipMemcpyAsync(y.data(), m->Y, y.size() * sizeof(float), hipMemcpyDeviceToHost, m->st) != hipSuccess)
+        y.resize((size_t)b * d.no);
+        if (hipMemcpyAsync(y.data(), dY, y.size() * sizeof(float), hipMemcpyDeviceToHost, m->st) != hipSuccess)
             return FRIBO_E_HIP;
     }
     if (hipStreamSynchronize(m->st) != hipSuccess) return FRIBO_E_HIP;
+    if (grad) {
+        const int rc = mlp_fetch(m, m->g, grad);
+        if (rc) return rc;
+    }
     if (loss) {
-        double s = 0.0;
+        double v = 0.0;
         for (size_t i = 0; i < y.size(); ++i) {
-            const double e = (double)y[i] - (double)T[i];
-            s += e * e;
+            const double e = (double)y[i] - (double)T[(size_t)s * d.no + i];
+            v += e * e;
         }
-        *loss = (float)(s / (double)y.size());
+        *loss = (float)(v / (double)y.size());
     }
     return 0;
 }
@@ -337,7 +478,8 @@ static int mlp_pass(fribo_mlp m, int n, const float* X, const float* T, float lr
 // Gradient of the mean squared loss over the n samples (no update).
 extern "C" int fribo_mlp_grad(fribo_mlp m, int32_t n, const float* X, const float* T, float* grad, float* loss)
 {
-    return mlp_pass(m, n, X, T, 0.0f, grad, loss);
+    if (!m || n < 1 || !X || !T) return FRIBO_E_ARG;
+    return mlp_run(m, n, X, T, 1, n, 0.0f, grad, loss);
 }
 
 // Adam training: epochs passes over the n samples in minibatches of
@@ -346,29 +488,33 @@ extern "C" int fribo_mlp_grad(fribo_mlp m, int32_t n, const float* X, const floa
 extern "C" int fribo_mlp_train(fribo_mlp m, int32_t n, const float* X, const float* T, int32_t epochs,
                                int32_t batch, float lr, float* loss)
 {
-    if (!m || n < 1 || epochs < 1 || batch < 1 || !(lr > 0.0f)) return FRIBO_E_ARG;
-    for (int e = 0; e < epochs; ++e)
-        for (int s = 0; s < n; s += batch) {
-            const int b = std::min(batch, n - s);
-            const bool last = e == epochs - 1 && s + batch >= n;
-            int rc = mlp_pass(m, b, X + (size_t)s * m->d.ni, T + (size_t)s * m->d.no, lr, nullptr,
-                              last ? loss : nullptr);
-            if (rc) return rc;
-        }
-    return 0;
+    if (!m || n < 1 || epochs < 1 || batch < 1 || !(lr > 0.0f) || !X || !T) return FRIBO_E_ARG;
+    return mlp_run(m, n, X, T, epochs, batch, lr, nullptr, loss);
 }
 
 // Inference in BF16 (FP32 accumulation) of n samples: Y = net(X).
 extern "C" int fribo_mlp_predict(fribo_mlp m, int32_t n, const float* X, float* Y)
 {
     if (!m || n < 1 || !X || !Y) return FRIBO_E_ARG;
-    if (mlp_reserve(m, n)) return FRIBO_E_HIP;
     const MlpDims& d = m->d;
-    if (hipMemcpyAsync(m->X, X, (size_t)n * d.ni * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess)
-        return FRIBO_E_HIP;
-    hipLaunchKernelGGL(k_mlp_infer, dim3(n), dim3(MLP_H), 0, m->st, d, (const float*)m->p, (const float*)m->X, m->Y);
+    const size_t nx = (size_t)n * d.ni, ny = (size_t)n * d.no;
+    const size_t lds = mlp_lds_floats(d) * sizeof(float);
+    const dim3 g((n + MLP_NS - 1) / MLP_NS);
+    if (nx + ny <= MLP_PIN) {
+        // the kernel reads and writes the pinned memory itself: no copies
+        memcpy(m->pin, X, nx * sizeof(float));
+        hipLaunchKernelGGL(k_mlp_infer, g, dim3(MLP_NT), lds, m->st, d, (const float*)m->p, n, (const float*)m->pin,
+                           m->pin + nx);
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->st) != hipSuccess) return FRIBO_E_HIP;
+        memcpy(Y, m->pin + nx, ny * sizeof(float));
+        return 0;
+    }
+    if (mlp_reserve(m, nx + ny)) return FRIBO_E_HIP;
+    if (hipMemcpyAsync(m->work, X, nx * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess) return FRIBO_E_HIP;
+    hipLaunchKernelGGL(k_mlp_infer, g, dim3(MLP_NT), lds, m->st, d, (const float*)m->p, n, (const float*)m->work,
+                       m->work + nx);
     if (hipGetLastError() != hipSuccess) return FRIBO_E_HIP;
-    if (hipMemcpyAsync(Y, m->Y, (size_t)n * d.no * sizeof(float), hipMemcpyDeviceToHost, m->st) != hipSuccess ||
+    if (hipMemcpyAsync(Y, m->work + nx, ny * sizeof(float), hipMemcpyDeviceToHost, m->st) != hipSuccess ||
         hipStreamSynchronize(m->st) != hipSuccess)
         return FRIBO_E_HIP;
     return 0;
