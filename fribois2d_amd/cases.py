@@ -327,17 +327,15 @@ def createnorm(verts, orient=-1.0):
     """rigid.F90:468-495: unit normal of every segment from the cross product
     of the segment (x=0 plane) with the vector to its midpoint lifted to x=or."""
     v = np.asarray(verts, dtype=np.float64)
-    nlm = v.shape[0] - 1
-    out = np.zeros((nlm, 2))
-    for i in range(nlm):
-        t1 = np.array([0.0, v[i, 0], v[i, 1]])
-        t2 = np.array([0.0, v[i + 1, 0], v[i + 1, 1]])
-        t3 = np.array([orient, (v[i, 0] + v[i + 1, 0]) * 0.5, (v[i, 1] + v[i + 1, 1]) * 0.5])
-        a, b = t2 - t1, t3 - t1
-        cr = np.array([a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]])
-        cr = cr / math.sqrt(float(np.sum(cr ** 2)))
-        out[i] = cr[1:]
-    return out
+    t1, t2 = v[:-1], v[1:]
+    mid = (t1 + t2) * 0.5
+    # a = t2 - t1 and b = t3 - t1 with a leading x component (0 and orient);
+    # every segment at once, each with the operations of the scalar formulas
+    ay, az = t2[:, 0] - t1[:, 0], t2[:, 1] - t1[:, 1]
+    by, bz = mid[:, 0] - t1[:, 0], mid[:, 1] - t1[:, 1]
+    c0, c1, c2 = ay * bz - az * by, az * orient - 0.0 * bz, 0.0 * by - ay * orient
+    cn = np.sqrt((c0 ** 2 + c1 ** 2) + c2 ** 2)
+    return np.stack([c1 / cn, c2 / cn], axis=1)
 
 
 def _heave(amp, freq):
