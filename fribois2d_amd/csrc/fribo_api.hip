@@ -49,7 +49,9 @@ struct fribo_ctx {
     std::vector<void*> mk_allocs;
     // marker upload: lmcc, lmvel, lmA staged together in pinned memory and
     // sent in one copy; ev_mk marks the copy so the staging is reused only
-    // after it has been read
+    // after it has been read.  Behind the 5 nlm doubles: 7 nlm + 1 that the
+    // load kernels read and write (LoadsIO) and 2 nlm + 2 that k_checkbcs
+    // writes
     double* mk_stage = nullptr;
     hipEvent_t ev_mk = nullptr;
     DevScalars hs;
@@ -66,7 +68,9 @@ struct fribo_ctx {
     // step inputs staged in pinned memory: {dt, dt_o, ns, err=0}
     struct StepIn { double dt, dto; int ns, err; };
     StepIn* in = nullptr;
-    DevScalars* hsp = nullptr;   // pinned landing buffer of the scalars read back after a step
+    // pinned landing buffer of the scalars read back after a step, followed by
+    // the nine results of the diagnostics
+    DevScalars* hsp = nullptr;
     hipEvent_t ev_rb = nullptr;  // the read-back copy of those scalars
     XferRing xfer;               // staging ring of the state transfers
     // k_cfl of the next step already enqueued behind the read-back of this
@@ -77,8 +81,7 @@ struct fribo_ctx {
     bool use_graph = false;
     bool yavail = false;     // transform along y set up
     double dmin = 0.0;       // smallest node spacing of the grid (cordin.F90:217-231)
-    double* nb = nullptr;    // device: the two checkbcs norms
-    double* dpart = nullptr; // device: diagnostics partials [8][256] and results [9]
+    double* dpart = nullptr; // device: diagnostics partials [8][256]
     // rollback copy of the prognostic state for iterated coupling
     double* snap = nullptr;
     bool snap_valid = false;
@@ -399,14 +402,12 @@ static int setup_ytransform(fribo_ctx* c, const double* zmmt, int ldz)
     return FRIBO_OK;
 }
 
-// Static device scratch of fribo_loads_transfer_static: the probe inputs
-// lmnor, lmacc (2 nlm each), the outputs press (nlm) and tau (2 nlm) and the
-// per-marker work records (FRIBO_LWORK nlm) for up to
-// FRIBO_STATIC_LOADS_MAX_NLM markers, 1.8 MB held on every device the
-// library runs on until the process ends.  Host code never passes the
+// Static device scratch of fribo_loads_transfer_static: the per-marker work
+// records (FRIBO_LWORK nlm) for up to FRIBO_STATIC_LOADS_MAX_NLM markers,
+// 1.3 MB held on every device the library runs on until the process ends.  Host code never passes the
 // array's name to a kernel or a copy: it uses the device address that
 // hipGetSymbolAddress returns, once per device, kept in g_scratch_addr.
-static __device__ __align__(256) double scratch[(size_t)FRIBO_STATIC_LOADS_MAX_NLM * (7 + FRIBO_LWORK)];
+static __device__ __align__(256) double scratch[(size_t)FRIBO_STATIC_LOADS_MAX_NLM * FRIBO_LWORK];
 
 static constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
@@ -557,8 +558,7 @@ extern "C" int fribo_init(const fribo_params* p, const double* rc, const double*
     if (!e) e = dalloc(c, &F.kDe, (size_t)2 * FRIBO_KMAXCH * F.n2m);
     if (!e) e = dalloc(c, &F.kX, (size_t)2 * FRIBO_KMAXCH * F.n2m);
     if (!e) e = dalloc(c, &F.S, 1);
-    if (!e) e = dalloc(c, &c->nb, 2);
-    if (!e) e = dalloc(c, &c->dpart, 8 * 256 + 16);
+    if (!e) e = dalloc(c, &c->dpart, 8 * 256);
     {
         // utils_proc.F90:600-602: first node nearest to z = 18.5
         int indz = 1;
@@ -588,7 +588,8 @@ extern "C" int fribo_init(const fribo_params* p, const double* rc, const double*
     memset(&c->hs, 0, sizeof(c->hs));
     {
         hipError_t he = hipHostMalloc((void**)&c->in, sizeof(fribo_ctx::StepIn), hipHostMallocDefault);
-        if (he == hipSuccess) he = hipHostMalloc((void**)&c->hsp, sizeof(DevScalars), hipHostMallocDefault);
+        if (he == hipSuccess) 
+            he = hipHostMalloc((void**)&c->hsp, sizeof(DevScalars) + 9 * sizeof(double), hipHostMallocDefault);
         if (he == hipSuccess) he = hipEventCreateWithFlags(&c->ev_rb, hipEventDisableTiming);
         if (he != hipSuccess) {
             for (void* q : c->allocs) hipFree(q);
@@ -756,14 +757,10 @@ extern "C" int fribo_set_markers(fribo_handle h, int32_t nlm, const double* lmcc
         if (!e) e = dalloc(h, &F.contrib, 2 * FRIBO_DIMSD * (size_t)nlm, L);
         if (!e) e = dalloc(h, &F.keys, 2 * (size_t)maxkeys, L);
         if (!e) e = dalloc(h, &F.segval, 2 * (size_t)maxkeys, L);
-        if (!e) e = dalloc(h, &F.lmnor, 2 * (size_t)nlm, L);
-        if (!e) e = dalloc(h, &F.lmacc, 2 * (size_t)nlm, L);
-        if (!e) e = dalloc(h, &F.press, (size_t)nlm, L);
-        if (!e) e = dalloc(h, &F.tau, 2 * (size_t)nlm, L);
         if (!e) e = dalloc(h, &F.lwork, FRIBO_LWORK * (size_t)nlm, L);
-        if (!e) e = dalloc(h, &F.bcerr, 2 * (size_t)nlm, L);
         if (!e && nlm > 0) {
-            hipError_t he = hipHostMalloc((void**)&h->mk_stage, 5 * (size_t)nlm * sizeof(double), hipHostMallocDefault);
+            hipError_t he = hipHostMalloc((void**)&h->mk_stage, (14 * (size_t)nlm + 3) * sizeof(double),
+                                          hipHostMallocDefault);
             if (he == hipSuccess && !h->ev_mk) he = hipEventCreateWithFlags(&h->ev_mk, hipEventDisableTiming);
             if (he != hipSuccess) e = set_err(FRIBO_ERR_HIP, hipGetErrorString(he));
         }
@@ -1340,30 +1337,40 @@ extern "C" int fribo_test_copy(int64_t bytes, int32_t reps, double* ms_per_copy)
 
 // loads_transfer_c (loads_transfer.F90:4-162) on the state the last step
 // left: probes at hpr = ddmin*kprobe along lmnor, where cordin already scaled
-// ddmin by kprobe (cordin.F90:231-233, loads_transfer.F90:41).
+// ddmin by kprobe (cordin.F90:231-233, loads_transfer.F90:41).  lwork: the
+// per-marker work records.  Inputs and results pass through the handle's
+// pinned marker staging, so the call is two launches and one wait.
+static int run_loads(fribo_ctx* h, double* lwork, double kprobe, const double* lmnor, const double* lmacc,
+                     double* press, double* tau)
+{
+    FluidDev F = h->F;
+    F.lwork = lwork;
+    const size_t n = (size_t)F.nlm, nb = n * sizeof(double);
+    double* io = h->mk_stage + 5 * n;
+    const LoadsIO L = {io, io + 2 * n, io + 4 * n, io + 5 * n, (int*)(io + 7 * n)};
+    memcpy(io, lmnor, 2 * nb);
+    memcpy(io + 2 * n, lmacc, 2 * nb);
+    const double hpr = (h->dmin * kprobe) * kprobe;
+    launch_loads(F, L, hpr, h->st);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(h->st));
+    h->hs.err = *L.err;
+    if (h->hs.err) return set_err(h->hs.err, "MLS partition of unity violated at a load probe");
+    memcpy(press, L.press, nb);
+    memcpy(tau, L.tau, 2 * nb);
+    return FRIBO_OK;
+}
+
 extern "C" int fribo_loads_transfer(fribo_handle h, double kprobe, const double* lmnor, const double* lmacc,
                                     double* press, double* tau)
 {
     if (!h || !lmnor || !lmacc || !press || !tau) return set_err(FRIBO_ERR_ARG, "null argument");
-    FluidDev& F = h->F;
-    if (F.nlm <= 0) return set_err(FRIBO_ERR_ARG, "no markers set");
-    const size_t nb = (size_t)F.nlm * sizeof(double);
-    HIPCHK(hipMemcpyAsync(F.lmnor, lmnor, 2 * nb, hipMemcpyHostToDevice, h->st));
-    HIPCHK(hipMemcpyAsync(F.lmacc, lmacc, 2 * nb, hipMemcpyHostToDevice, h->st));
-    const double hpr = (h->dmin * kprobe) * kprobe;
-    launch_loads(F, hpr, h->st);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(press, F.press, nb, hipMemcpyDeviceToHost, h->st));
-    HIPCHK(hipMemcpyAsync(tau, F.tau, 2 * nb, hipMemcpyDeviceToHost, h->st));
-    int e = read_scalars(h);
-    if (e) return e;
-    if (h->hs.err) return set_err(h->hs.err, "MLS partition of unity violated at a load probe");
-    return FRIBO_OK;
+    if (h->F.nlm <= 0) return set_err(FRIBO_ERR_ARG, "no markers set");
+    return run_loads(h, h->F.lwork, kprobe, lmnor, lmacc, press, tau);
 }
 
-// fribo_loads_transfer with every device buffer of the call (probe inputs,
-// loads, per-marker work records) in the static scratch of the handle's
-// device: no allocation.  Same kernels, same results.
+// fribo_loads_transfer with its work records in the static scratch of the
+// handle's device: no allocation.  Same kernels, same results.
 extern "C" int fribo_loads_transfer_static(fribo_handle h, double kprobe, const double* lmnor, const double* lmacc,
                                            double* press, double* tau)
 {
@@ -1374,43 +1381,23 @@ extern "C" int fribo_loads_transfer_static(fribo_handle h, double kprobe, const 
                                             " markers, the static scratch holds at most " +
                                             std::to_string(FRIBO_STATIC_LOADS_MAX_NLM));
     if (!h->scratch) return set_err(FRIBO_ERR_HIP, "static scratch address not set");
-    FluidDev G = h->F;
-    const size_t n = (size_t)G.nlm;
-    G.lmnor = h->scratch;
-    G.lmacc = G.lmnor + 2 * n;
-    G.press = G.lmacc + 2 * n;
-    G.tau = G.press + n;
-    G.lwork = G.tau + 2 * n;
-    const size_t nb = n * sizeof(double);
-    HIPCHK(hipMemcpyAsync(G.lmnor, lmnor, 2 * nb, hipMemcpyHostToDevice, h->st));
-    HIPCHK(hipMemcpyAsync(G.lmacc, lmacc, 2 * nb, hipMemcpyHostToDevice, h->st));
-    const double hpr = (h->dmin * kprobe) * kprobe;
-    launch_loads(G, hpr, h->st);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(press, G.press, nb, hipMemcpyDeviceToHost, h->st));
-    HIPCHK(hipMemcpyAsync(tau, G.tau, 2 * nb, hipMemcpyDeviceToHost, h->st));
-    int e = read_scalars(h);
-    if (e) return e;
-    if (h->hs.err) return set_err(h->hs.err, "MLS partition of unity violated at a load probe");
-    return FRIBO_OK;
+    return run_loads(h, h->scratch, kprobe, lmnor, lmacc, press, tau);
 }
 
 // checkbcs (ckbcs.F90:5-86) on the state the last step left.
 extern "C" int fribo_checkbcs(fribo_handle h, double* bcerrv, double* bcerrw, double* nbcv, double* nbcw)
 {
     if (!h) return set_err(FRIBO_ERR_ARG, "null handle");
-    FluidDev& F = h->F;
-    if (F.nlm <= 0) return set_err(FRIBO_ERR_ARG, "no markers set");
-    launch_checkbcs(F, h->nb, h->st);
+    if (h->F.nlm <= 0) return set_err(FRIBO_ERR_ARG, "no markers set");
+    const size_t n = (size_t)h->F.nlm;
+    double* out = h->mk_stage + 12 * n + 1;
+    launch_checkbcs(h->F, out, h->st);
     HIPCHK(hipGetLastError());
-    const size_t nb = (size_t)F.nlm * sizeof(double);
-    if (bcerrv) HIPCHK(hipMemcpyAsync(bcerrv, F.bcerr, nb, hipMemcpyDeviceToHost, h->st));
-    if (bcerrw) HIPCHK(hipMemcpyAsync(bcerrw, F.bcerr + F.nlm, nb, hipMemcpyDeviceToHost, h->st));
-    double v[2];
-    HIPCHK(hipMemcpyAsync(v, h->nb, sizeof(v), hipMemcpyDeviceToHost, h->st));
     HIPCHK(hipStreamSynchronize(h->st));
-    if (nbcv) *nbcv = v[0];
-    if (nbcw) *nbcw = v[1];
+    if (bcerrv) memcpy(bcerrv, out, n * sizeof(double));
+    if (bcerrw) memcpy(bcerrw, out + n, n * sizeof(double));
+    if (nbcv) *nbcv = out[2 * n];
+    if (nbcw) *nbcw = out[2 * n + 1];
     return FRIBO_OK;
 }
 
@@ -1418,11 +1405,11 @@ extern "C" int fribo_checkbcs(fribo_handle h, double* bcerrv, double* bcerrw, do
 extern "C" int fribo_diagnostics(fribo_handle h, double* out)
 {
     if (!h || !out) return set_err(FRIBO_ERR_ARG, "null argument");
-    double* res = h->dpart + 8 * 256;
+    double* res = (double*)(h->hsp + 1);
     launch_diag(h->F, h->dpart, h->vort_k, res, h->st);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out, res, 9 * sizeof(double), hipMemcpyDeviceToHost, h->st));
     HIPCHK(hipStreamSynchronize(h->st));
+    memcpy(out, res, 9 * sizeof(double));
     return FRIBO_OK;
 }
 
@@ -1440,18 +1427,11 @@ static size_t snap_doubles(const FluidDev& F)
 static int snap_copy(fribo_ctx* h, bool save)
 {
     FluidDev& F = h->F;
-    const size_t fsz = (size_t)F.P * F.nk * sizeof(double), bsz = (size_t)(F.n2 + 2) * sizeof(double);
-    double* fl[5] = {F.q2, F.q3, F.pr, F.ru2, F.ru3};
-    double* bc[10] = {F.qb2s, F.qb3s, F.qb2n, F.qb3n, F.dqb2s, F.dqb3s, F.dqb2n, F.dqb3n, F.dq2x2o, F.dq3x2o};
-    char* p = (char*)h->snap;
-    for (int i = 0; i < 5; ++i, p += fsz)
-        HIPCHK(hipMemcpyAsync(save ? (void*)p : (void*)fl[i], save ? (void*)fl[i] : (void*)p, fsz,
-                              hipMemcpyDeviceToDevice, h->st));
-    for (int i = 0; i < 10; ++i, p += bsz)
-        HIPCHK(hipMemcpyAsync(save ? (void*)p : (void*)bc[i], save ? (void*)bc[i] : (void*)p, bsz,
-                              hipMemcpyDeviceToDevice, h->st));
-    HIPCHK(hipMemcpyAsync(save ? (void*)p : (void*)F.S, save ? (void*)F.S : (void*)p, sizeof(DevScalars),
-                          hipMemcpyDeviceToDevice, h->st));
+    const SnapTab T = {{F.q2, F.q3, F.pr, F.ru2, F.ru3},
+                       {F.qb2s, F.qb3s, F.qb2n, F.qb3n, F.dqb2s, F.dqb3s, F.dqb2n, F.dqb3n, F.dq2x2o, F.dq3x2o},
+                       (size_t)F.P * F.nk, (size_t)(F.n2 + 2)};
+    launch_snap(T, F.S, h->snap, save, h->st);
+    HIPCHK(hipGetLastError());
     return FRIBO_OK;
 }
 

@@ -148,13 +148,35 @@ struct FluidDev {
     unsigned long long *keys;      // [2][maxkeys]
     double *segval;                // [2][maxkeys] cell value at segment heads
     int maxkeys;
-    // loads on the body (loads_transfer_c) and the forcing check (checkbcs)
-    double *lmnor, *lmacc;         // (nlm,2) column-major, from the host
-    double *press, *tau;           // (nlm), (nlm,2)
-    double *lwork;                 // [nlm][FRIBO_LWORK] per-marker probe data
-    double *bcerr;                 // (nlm,2)
+    double *lwork;                 // [nlm][FRIBO_LWORK] per-marker probe data of the loads (loads_transfer_c)
     DevScalars* S;
 };
+
+// Host side of a load computation, in pinned memory the kernels read and write
+// directly: normals and accelerations (nlm,2) in, pressure (nlm), friction
+// stress (nlm,2) and the error flag out.
+struct LoadsIO {
+    const double *nor, *acc;
+    double *press, *tau;
+    int* err;
+};
+
+// Arrays of the rollback copy: fields of flen doubles each (an even number),
+// boundary arrays of blen doubles.
+struct SnapTab {
+    double *field[5], *bnd[10];
+    size_t flen, blen;
+};
+
+// Lane n of each 16-lane row of the wave, broadcast to the row (DPP
+// row_newbcast), for a double.
+template <int N>
+__device__ inline double row_bcast(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + N, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + N, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
 
 // s_barrier without the memory fence of __syncthreads (whose release waits
 // for every outstanding global access of the wave, loads into LDS and
@@ -259,7 +281,7 @@ void launch_gemm_nn(int M, int N, int K, const double* A, int lda, const double*
 int gemm_nn_tiles_n(int M, int N, int K, const double* A, int lda, const double* B, int ldb, int ks);
 // The per-mode z-lines of the y-order Poisson solve, hmn in place.
 void launch_ysolve(const FluidDev& F, hipStream_t st);
-void launch_loads(const FluidDev& F, double hpr, hipStream_t st);
+void launch_loads(const FluidDev& F, const LoadsIO& io, double hpr, hipStream_t st);
 // mixed-precision Poisson solve: r = rhs - (A_y + A_z) x (r may alias rhs),
 // and the FP32 transform C = X0 + A * B (X0 optional, may alias C)
 void launch_pres_residual(const FluidDev& F, const double* x, const double* rhs, double* r, hipStream_t st);
@@ -267,7 +289,8 @@ void launch_gemm32(int M, int N, int K, const double* A, int lda, const double* 
                    const double* X0, const DevScalars* S, hipStream_t st, const double* zg, double* gpart,
                    hipEvent_t e0, hipEvent_t e1);
 int gemm32_tiles_n(int N);
-void launch_checkbcs(const FluidDev& F, double* nb, hipStream_t st);
+void launch_checkbcs(const FluidDev& F, double* out, hipStream_t st);
+void launch_snap(const SnapTab& T, DevScalars* S, double* snap, bool save, hipStream_t st);
 void launch_diag(const FluidDev& F, double* part, int kv, double* out, hipStream_t st);
 // device: the symmetrised eigen-problem on the GPU (rocSOLVER STEDC) instead
 // of the host QL

@@ -116,47 +116,65 @@ __global__ __launch_bounds__(64) void kb_mls_idx(const BGrid<FluidDev> G)
     mls_idx_body(*Fp, vb);
 }
 
-// utils_math.f90:637-725, 3x3 scaled partial pivoting; returns info
-__device__ int gesolve3(const double ai[3][3], const double bi[3], double x[3])
+// utils_math.f90:637-725, 3x3 scaled partial pivoting; returns info.  The
+// row exchange names its rows by constants (a row index known only at run
+// time would put the matrix in scratch memory, and the solve would wait for
+// memory at every step of a chain that is serial anyway).
+__device__ __forceinline__ int gesolve3(const double ai[3][3], const double bi[3], double x[3])
 {
     double a[3][3], b[3], sc[3];
+#pragma unroll
     for (int i = 0; i < 3; ++i) {
         b[i] = bi[i];
+#pragma unroll
         for (int j = 0; j < 3; ++j) a[i][j] = ai[i][j];
     }
+#pragma unroll
     for (int k = 0; k < 2; ++k) {
+#pragma unroll
         for (int i = k; i < 3; ++i) {
             sc[i] = 0.0;
+#pragma unroll
             for (int j = k; j < 3; ++j) sc[i] = fmax(sc[i], fabs(a[i][j]));
         }
         double pivot = fabs(a[k][k] / sc[k]);
         int l = k;
-        for (int j = k + 1; j < 3; ++j)
-            if (fabs(a[j][k] / sc[j]) > pivot) {
-                pivot = fabs(a[j][k] / sc[j]);
+#pragma unroll
+        for (int j = k + 1; j < 3; ++j) {
+            const double v = fabs(a[j][k] / sc[j]);
+            if (v > pivot) {
+                pivot = v;
                 l = j;
             }
-        if (pivot == 0.0) return 0;
-        if (l != k) {
-            for (int j = k; j < 3; ++j) {
-                double st = a[k][j];
-                a[k][j] = a[l][j];
-                a[l][j] = st;
-            }
-            double st = b[k];
-            b[k] = b[l];
-            b[l] = st;
         }
+        if (pivot == 0.0) return 0;
+#pragma unroll
+        for (int r = k + 1; r < 3; ++r) {
+            const bool sw = l == r;
+#pragma unroll
+            for (int j = k; j < 3; ++j) {
+                const double st = a[k][j];
+                a[k][j] = sw ? a[r][j] : st;
+                a[r][j] = sw ? st : a[r][j];
+            }
+            const double st = b[k];
+            b[k] = sw ? b[r] : st;
+            b[r] = sw ? st : b[r];
+        }
+#pragma unroll
         for (int i = k + 1; i < 3; ++i) {
             double c = a[i][k] / a[k][k];
             a[i][k] = 0.0;
             b[i] = b[i] - c * b[k];
+#pragma unroll
             for (int j = k + 1; j < 3; ++j) a[i][j] = a[i][j] - c * a[k][j];
         }
     }
     x[2] = b[2] / a[2][2];
+#pragma unroll
     for (int i = 1; i >= 0; --i) {
         double c = 0.0;
+#pragma unroll
         for (int j = i + 1; j < 3; ++j) c = c + a[i][j] * x[j];
         x[i] = (b[i] - c) / a[i][i];
     }
@@ -800,8 +818,6 @@ void launch_mls_force_b(BatchSet& B, hipStream_t st)
 // ---------------------------------------------------------------------------
 // Loads on the body (loads_transfer.F90:4-162) and the forcing check.
 
-#define LMNOR(n, c) F.lmnor[(size_t)((n) - 1) + (size_t)((c) - 1) * F.nlm]
-#define LMACC(n, c) F.lmacc[(size_t)((n) - 1) + (size_t)((c) - 1) * F.nlm]
 #define LW(n, q) F.lwork[(size_t)((n) - 1) * FRIBO_LWORK + (q)]
 
 // MLSint.F90:492-585 (weight_function_d), one direction: value and derivative
@@ -847,15 +863,17 @@ __device__ inline void weight1d_d(double difc, double sdd, int wfun, double radi
     }
 }
 
-// first minimum of |x(i) - v| over i = c-5..c+5 inside 1..n (probeind)
+// first minimum of |x(i) - v| over i = c-5..c+5 inside 1..n (probeind); the
+// reads of indices outside are clamped, so that all are in flight together
 __device__ inline int window_minloc(const double* x, int n, int c, double v)
 {
     int best = 0;
     double bv = 0.0;
-    for (int i = c - 5; i <= c + 5; ++i) {
-        if (i < 1 || i > n) continue;
-        const double a = fabs(x[i] - v);
-        if (best == 0 || a < bv) {
+#pragma unroll
+    for (int q = 0; q < 11; ++q) {
+        const int i = c - 5 + q;
+        const double a = fabs(x[min(max(i, 1), n)] - v);
+        if (i >= 1 && i <= n && (best == 0 || a < bv)) {
             bv = a;
             best = i;
         }
@@ -864,181 +882,179 @@ __device__ inline int window_minloc(const double* x, int n, int c, double v)
 }
 
 // Probe values: ucy/ucz/pc (loads_transfer.F90:210-267) need f(j-1,k) at j=1,
-// which the reference's column-major storage resolves to f(n2,k-1).
-__device__ inline double fat(const FluidDev& F, const double* f, int j, int k)
-{
-    if (j == 0) {
-        j = F.n2;
-        k = k - 1;
-    }
-    return f[fidx(F, j, k)];
-}
-
-__device__ inline double prat(const FluidDev& F, const DevScalars* S, int j, int k)
+// which the reference's column-major storage resolves to f(n2,k-1).  The
+// pressure's pending means are applied as it is read.
+__device__ inline double fat(const FluidDev& F, const double* f, bool prs, int j, int k)
 {
     if (j == 0) {
         j = F.n2;
         k = k - 1;
     }
     const bool edge = (j == F.n2) || k < 1 || k > F.n3m;
-    return F.pr[fidx(F, j, k)] - (edge ? S->goff : S->pend);
+    const double v = f[fidx(F, j, k)];
+    return prs ? v - (edge ? F.S->goff : F.S->pend) : v;
 }
 
-// One thread per marker: probes, MLS_SF_d, getpbup and the pressure; the
-// velocity-derivative combinations are left in lwork for the friction stress,
-// which needs the tangent of the previous marker when this one has none.
-__global__ __launch_bounds__(64) void k_loads(const FluidDev F, double hpr)
+// Sum over lanes 0..8 of each 16-lane row in that order, in every lane.
+__device__ inline double row_sum9(double v)
+{
+    double s = 0.0;
+    s = s + row_bcast<0>(v);
+    s = s + row_bcast<1>(v);
+    s = s + row_bcast<2>(v);
+    s = s + row_bcast<3>(v);
+    s = s + row_bcast<4>(v);
+    s = s + row_bcast<5>(v);
+    s = s + row_bcast<6>(v);
+    s = s + row_bcast<7>(v);
+    s = s + row_bcast<8>(v);
+    return s;
+}
+
+// One wave per marker, one 16-lane row per grid (q2, q3, pressure; the fourth
+// row repeats the third and stores nothing), lane m < 9 owning support m:
+// probe, MLS_SF_d, getpbup and the pressure; the velocity-derivative
+// combinations are left in lwork for the friction stress, which needs the
+// tangent of the previous marker when this one has none.  The moment
+// matrices and the probe's sums are added in support order from the row's
+// lanes, so every value is the serial loop's.
+//
+// A few hundred markers are far too few for the chip, so the time is the
+// serial chain of one marker; spread over lanes it is a weight, three solves
+// in two steps (the rows' odd lanes take the second derivative) and one
+// gather instead of 27 weights, nine solves and 81 gathers in one thread.
+// Normals and accelerations come straight from pinned host memory.  91
+// markers: 66 us with one thread per marker, 12 us here.
+__global__ __launch_bounds__(64) void k_loads(const FluidDev F, const LoadsIO io, double hpr)
 {
     DevScalars* S = F.S;
     if (S->err) return;
-    const int n = blockIdx.x * 64 + threadIdx.x + 1;
-    if (n > F.nlm) return;
+    const int lane = threadIdx.x, m = lane & 15, n = blockIdx.x + 1;
+    const int idir = min(lane >> 4, 2) + 1;
+    const double nor[2] = {io.nor[n - 1], io.nor[(size_t)(n - 1) + F.nlm]};
+    const double acc[2] = {io.acc[n - 1], io.acc[(size_t)(n - 1) + F.nlm]};
     const double pos[2] = {LMCC(n, 1), LMCC(n, 2)};
-    const double nor[2] = {LMNOR(n, 1), LMNOR(n, 2)};
+    const int mi1 = (idir == 3) ? LMIND(n, 2, 1) : LMIND(n, idir, 1);
+    const int mi2 = (idir == 3) ? LMIND(n, 1, 2) : LMIND(n, idir, 2);
+    if (!(F.zz[1] < pos[1] && pos[1] < F.zz[F.n3])) {   // whole wave
+        if (lane == 0) {
+            LW(n, 0) = 0.0;   // inside
+            LW(n, 1) = 0.0;   // has a tangent
+            LW(n, 19) = 0.0;  // pressure
+        }
+        return;
+    }
     const double probe[2] = {pos[0] + nor[0] * hpr, pos[1] + nor[1] * hpr};
-    F.press[n - 1] = 0.0;
-    LW(n, 0) = 0.0;   // inside
-    LW(n, 1) = 0.0;   // has a tangent
-    if (!(F.zz[1] < pos[1] && pos[1] < F.zz[F.n3])) return;
-    double u[3][7];
-    for (int idir = 1; idir <= 3; ++idir) {
-        const int mi1 = (idir == 3) ? LMIND(n, 2, 1) : LMIND(n, idir, 1);
-        const int mi2 = (idir == 3) ? LMIND(n, 1, 2) : LMIND(n, idir, 2);
-        const double* ya = (idir == 1) ? F.rc : F.rm;
-        const double* za = (idir == 2) ? F.zz : F.zm;
-        const int i1 = window_minloc(ya, F.n2, mi1, probe[0]);
-        const int i2 = window_minloc(za, F.n3, mi2, probe[1]);
-        // MLS_SD_ind
-        double sdc[2][FRIBO_DIMSD], sdd[2][FRIBO_DIMSD];
-        int eul[2][FRIBO_DIMSD];
-        int m = 0;
-        for (int j = 1; j <= 3; ++j)
-            for (int k = 1; k <= 3; ++k) {
-                const int jj = (i1 == 1) ? j + 1 : ((i1 == F.n2m) ? j - 1 : j);
-                const int kk = (i2 == 1) ? k + 1 : ((i2 == F.n3m) ? k - 1 : k);
-                const int ej = i1 + jj - 2, ek = i2 + kk - 2;
-                sdc[0][m] = ya[ej];
-                sdd[0][m] = ya[ej + 1] - ya[ej];
-                sdc[1][m] = za[ek];
-                sdd[1][m] = za[ek + 1] - za[ek];
-                eul[0][m] = ej;
-                eul[1][m] = ek;
-                ++m;
-            }
-        // MLS_SF_d with compute_AB_d
-        double w[FRIBO_DIMSD][3], pk[3][FRIBO_DIMSD], A[3][3][3];
-        for (int i = 0; i < FRIBO_DIMSD; ++i) {
-            pk[0][i] = 1.0;
-            pk[1][i] = sdc[0][i];
-            pk[2][i] = sdc[1][i];
-            double w1, d1, w2, d2;
-            weight1d_d(probe[0] - sdc[0][i], sdd[0][i], F.wfun, F.radiusSD, w1, d1);
-            weight1d_d(probe[1] - sdc[1][i], sdd[1][i], F.wfun, F.radiusSD, w2, d2);
-            w[i][0] = w1 * w2;
-            w[i][1] = w2 * d1;
-            w[i][2] = w1 * d2;
-        }
+    const double* ya = (idir == 1) ? F.rc : F.rm;
+    const double* za = (idir == 2) ? F.zz : F.zm;
+    const int i1 = window_minloc(ya, F.n2, mi1, probe[0]);
+    const int i2 = window_minloc(za, F.n3, mi2, probe[1]);
+    // MLS_SD_ind: support mm of the 3x3 block (lanes past the ninth repeat it)
+    const int mm = min(m, FRIBO_DIMSD - 1), j = mm / 3 + 1, k = mm % 3 + 1;
+    const int jj = (i1 == 1) ? j + 1 : ((i1 == F.n2m) ? j - 1 : j);
+    const int kk = (i2 == 1) ? k + 1 : ((i2 == F.n3m) ? k - 1 : k);
+    const int ej = i1 + jj - 2, ek = i2 + kk - 2;
+    const double sdc0 = ya[ej], sdd0 = ya[ej + 1] - ya[ej];
+    const double sdc1 = za[ek], sdd1 = za[ek + 1] - za[ek];
+    // the values getpbup gathers, in flight during the fit
+    const double* f = (idir == 1) ? F.q2 : ((idir == 2) ? F.q3 : F.pr);
+    const double fc = fat(F, f, idir == 3, ej, ek);
+    const double fjm = fat(F, f, idir == 3, ej - 1, ek);
+    const double fkm = fat(F, f, idir == 3, ej, ek - 1);
+    const double gj = F.g2rc[ej], gk = F.g3rc[ek];
+    // MLS_SF_d with compute_AB_d
+    const double pk[3] = {1.0, sdc0, sdc1};
+    double w1, d1, w2, d2;
+    weight1d_d(probe[0] - sdc0, sdd0, F.wfun, F.radiusSD, w1, d1);
+    weight1d_d(probe[1] - sdc1, sdd1, F.wfun, F.radiusSD, w2, d2);
+    const double w[3] = {w1 * w2, w2 * d1, w1 * d2};
+    double A[3][3][3];   // [l][a][b]; symmetric entry by entry: w*(pa*pb) == w*(pb*pa)
+#pragma unroll
+    for (int l = 0; l < 3; ++l)
+#pragma unroll
         for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b)
-                for (int l = 0; l < 3; ++l) A[a][b][l] = 0.0;
-        for (int i = 0; i < FRIBO_DIMSD; ++i)
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) {
-                    const double pp = pk[a][i] * pk[b][i];
-                    for (int l = 0; l < 3; ++l) A[a][b][l] = A[a][b][l] + w[i][l] * pp;
-                }
-        double Aa[3][3];
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b) Aa[a][b] = A[a][b][0];
-        double gam[3][3];
-        const double g0[3] = {1.0, probe[0], probe[1]};
-        double x[3] = {0.0, 0.0, 0.0};
-        gesolve3(Aa, g0, x);
-        for (int a = 0; a < 3; ++a) gam[a][0] = x[a];
-        for (int l = 1; l <= 2; ++l) {
-            double C[3];
-            for (int a = 0; a < 3; ++a) {
-                double mv = 0.0;
-                for (int b = 0; b < 3; ++b) mv = mv + A[a][b][l] * gam[b][0];
-                C[a] = ((a == l) ? 1.0 : 0.0) - mv;
-            }
-            x[0] = x[1] = x[2] = 0.0;
-            gesolve3(Aa, C, x);
-            for (int a = 0; a < 3; ++a) gam[a][l] = x[a];
+#pragma unroll
+            for (int b = a; b < 3; ++b) A[l][a][b] = A[l][b][a] = row_sum9(w[l] * (pk[a] * pk[b]));
+    const double g0[3] = {1.0, probe[0], probe[1]};
+    double gam[3][3];    // [l][a]
+#pragma unroll
+    for (int a = 0; a < 3; ++a) gam[0][a] = 0.0;
+    gesolve3(A[0], g0, gam[0]);
+    {
+        const bool two = m & 1;
+        double C[3], x[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            double mv = 0.0;
+#pragma unroll
+            for (int b = 0; b < 3; ++b) mv = mv + (two ? A[2][a][b] : A[1][a][b]) * gam[0][b];
+            C[a] = ((a == (two ? 2 : 1)) ? 1.0 : 0.0) - mv;
         }
-        double ph[3][FRIBO_DIMSD], sumphi = 0.0;
-        for (int i = 0; i < FRIBO_DIMSD; ++i) {
-            ph[0][i] = 0.0;
-            ph[1][i] = 0.0;
-            ph[2][i] = 0.0;
-            for (int a = 0; a < 3; ++a) {
-                const double b0 = pk[a][i] * w[i][0], b1 = pk[a][i] * w[i][1], b2 = pk[a][i] * w[i][2];
-                ph[0][i] = ph[0][i] + gam[a][0] * b0;
-                ph[1][i] = ph[1][i] + gam[a][1] * b0 + gam[a][0] * b1;
-                ph[2][i] = ph[2][i] + gam[a][2] * b0 + gam[a][0] * b2;
-            }
-        }
-        for (int i = 0; i < FRIBO_DIMSD; ++i) sumphi = sumphi + ph[0][i];
-        if (fabs(1.0 - fabs(sumphi)) > 1.0e-10) atomicCAS(&S->err, 0, FRIBO_E_PARTITION_UNITY);
-        // getpbup
-        double* uu = u[idir - 1];
-        for (int i = 0; i < 7; ++i) uu[i] = 0.0;
-        const double* f = (idir == 1) ? F.q2 : F.q3;
-        for (int i = 0; i < FRIBO_DIMSD; ++i) {
-            const int cy = eul[0][i], cz = eul[1][i];
-            double fc, fjm, fkm;
-            if (idir == 3) {
-                fc = prat(F, S, cy, cz);
-                fjm = prat(F, S, cy - 1, cz);
-                fkm = prat(F, S, cy, cz - 1);
-            } else {
-                fc = fat(F, f, cy, cz);
-                fjm = fat(F, f, cy - 1, cz);
-                fkm = fat(F, f, cy, cz - 1);
-            }
-            const double uk0 = fc;
-            const double uk1 = (fc - fjm) * F.dx2 / F.g2rc[cy];
-            const double uk2 = (fc - fkm) * F.dx3 / F.g3rc[cz];
-            for (int q = 0; q < 3; ++q) uu[q] = uu[q] + ph[q][i] * uk0;
-            uu[3] = uu[3] + ph[1][i] * uk1;
-            uu[4] = uu[4] + ph[1][i] * uk2;
-            uu[5] = uu[5] + ph[2][i] * uk1;
-            uu[6] = uu[6] + ph[2][i] * uk2;
+        gesolve3(A[0], C, x);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            gam[1][a] = row_bcast<0>(x[a]);
+            gam[2][a] = row_bcast<1>(x[a]);
         }
     }
-    const double* ucy = u[0];
-    const double* ucz = u[1];
-    const double* pc = u[2];
+    double ph[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const double b0 = pk[a] * w[0], b1 = pk[a] * w[1], b2 = pk[a] * w[2];
+        ph[0] = ph[0] + gam[0][a] * b0;
+        ph[1] = ph[1] + gam[1][a] * b0 + gam[0][a] * b1;
+        ph[2] = ph[2] + gam[2][a] * b0 + gam[0][a] * b2;
+    }
+    const double sumphi = row_sum9(ph[0]);
+    if (m == 0 && fabs(1.0 - fabs(sumphi)) > 1.0e-10) atomicCAS(&S->err, 0, FRIBO_E_PARTITION_UNITY);
+    // getpbup
+    const double uk0 = fc;
+    const double uk1 = (fc - fjm) * F.dx2 / gj;
+    const double uk2 = (fc - fkm) * F.dx3 / gk;
+    const double uu[7] = {row_sum9(ph[0] * uk0), row_sum9(ph[1] * uk0), row_sum9(ph[2] * uk0), row_sum9(ph[1] * uk1),
+                          row_sum9(ph[1] * uk2), row_sum9(ph[2] * uk1), row_sum9(ph[2] * uk2)};
+    double ucy[7], ucz[7], pc[7];
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+        ucy[q] = __shfl(uu[q], 0, 64);
+        ucz[q] = __shfl(uu[q], 16, 64);
+        pc[q] = __shfl(uu[q], 32, 64);
+    }
+    if (lane != 0) return;
     const double veln_md = ucy[0] * nor[0] + ucz[0] * nor[1];
     const double vt0 = ucy[0] - veln_md * nor[0], vt1 = ucz[0] - veln_md * nor[1];
     const double velt_md = sqrt(vt0 * vt0 + vt1 * vt1);
     LW(n, 0) = 1.0;
+    LW(n, 1) = 0.0;
     if (velt_md != 0.0) {
         const double nrm = sqrt(vt0 * vt0 + vt1 * vt1);
         LW(n, 1) = 1.0;
         LW(n, 2) = vt0 / nrm;
         LW(n, 3) = vt1 / nrm;
     }
-    double dpdnw = LMACC(n, 1) * nor[0] + LMACC(n, 2) * nor[1];
+    double dpdnw = acc[0] * nor[0] + acc[1] * nor[1];
     dpdnw = -1.0 * dpdnw;
     const double dpdne = pc[1] * nor[0] + pc[2] * nor[1];
-    F.press[n - 1] = pc[0] - 0.5 * (dpdnw + dpdne) * hpr;
     for (int q = 1; q < 7; ++q) {
         LW(n, 3 + q) = ucy[q];
         LW(n, 9 + q) = ucz[q];
     }
     const double nory = nor[0], norz = nor[1];
     LW(n, 16) = (pc[3] * nory * nory + pc[4] * nory * norz + pc[5] * norz * nory + pc[6] * norz * norz) * 1.0 / F.visc;
+    LW(n, 17) = nory;
+    LW(n, 18) = norz;
+    LW(n, 19) = pc[0] - 0.5 * (dpdnw + dpdne) * hpr;
 }
 
 // Tangent of every marker: its own, else the last one set before it
 // (loads_transfer.F90:94-96), by one wave with a "last set" scan over lane
-// chunks; then the friction stress (loads_transfer.F90:111-128).
-__global__ __launch_bounds__(64) void k_loads_tau(const FluidDev F, double hpr)
+// chunks; then the friction stress (loads_transfer.F90:111-128).  The results
+// and the error flag go straight to pinned host memory.
+__global__ __launch_bounds__(64) void k_loads_tau(const FluidDev F, const LoadsIO io, double hpr)
 {
-    DevScalars* S = F.S;
-    if (S->err) return;
-    const int lane = threadIdx.x, nlm = F.nlm;
+    const int lane = threadIdx.x, nlm = F.nlm, err = F.S->err;
+    if (lane == 0) *io.err = err;
+    if (err) return;
     const int per = (nlm + 63) / 64;
     const int n0 = lane * per + 1, n1 = min(nlm, n0 + per - 1);
     bool has = false;
@@ -1067,16 +1083,17 @@ __global__ __launch_bounds__(64) void k_loads_tau(const FluidDev F, double hpr)
     }
     const double visc = F.visc;
     for (int n = n0; n <= n1; ++n) {
-        F.tau[(size_t)(n - 1) + nlm] = 0.0;
+        io.press[n - 1] = LW(n, 19);
         if (LW(n, 0) == 0.0) {
-            F.tau[n - 1] = 0.0;
+            io.tau[n - 1] = 0.0;
+            io.tau[(size_t)(n - 1) + nlm] = 0.0;
             continue;
         }
         if (LW(n, 1) != 0.0) {
             cy = LW(n, 2);
             cz = LW(n, 3);
         }
-        const double nory = LMNOR(n, 1), norz = LMNOR(n, 2), tany = cy, tanz = cz;
+        const double nory = LW(n, 17), norz = LW(n, 18), tany = cy, tanz = cz;
         const double u1 = LW(n, 4), u2 = LW(n, 5), u3 = LW(n, 6), u4 = LW(n, 7), u5 = LW(n, 8), u6 = LW(n, 9);
         const double v1 = LW(n, 10), v2 = LW(n, 11), v3 = LW(n, 12), v4 = LW(n, 13), v5 = LW(n, 14), v6 = LW(n, 15);
         const double d3ucdn3 = LW(n, 16);
@@ -1085,23 +1102,26 @@ __global__ __launch_bounds__(64) void k_loads_tau(const FluidDev F, double hpr)
                                 u6 * tany * norz * norz + v3 * tanz * nory * nory + v4 * tanz * nory * norz +
                                 v5 * tanz * norz * nory + v6 * tanz * norz * norz);
         const double ducdnm = ducdn - d2ucdn2 * hpr - 0.5 * d3ucdn3 * (hpr * hpr);
-        F.tau[n - 1] = visc * ducdnm * tany;
-        F.tau[(size_t)(n - 1) + nlm] = visc * ducdnm * tanz;
+        io.tau[n - 1] = visc * ducdnm * tany;
+        io.tau[(size_t)(n - 1) + nlm] = visc * ducdnm * tanz;
     }
 }
 
-void launch_loads(const FluidDev& F, double hpr, hipStream_t st)
+void launch_loads(const FluidDev& F, const LoadsIO& io, double hpr, hipStream_t st)
 {
     if (F.nlm <= 0) return;
-    hipLaunchKernelGGL(k_loads, dim3((F.nlm + 63) / 64), dim3(64), 0, st, F, hpr);
-    hipLaunchKernelGGL(k_loads_tau, dim3(1), dim3(64), 0, st, F, hpr);
+    hipLaunchKernelGGL(k_loads, dim3(F.nlm), dim3(64), 0, st, F, io, hpr);
+    hipLaunchKernelGGL(k_loads_tau, dim3(1), dim3(64), 0, st, F, io, hpr);
 }
 
 // ckbcs.F90:5-86: velocity error at the markers after the step and the norms
-// sqrt(sum err^2)/nlm (fixed-order tree sum); nb[0..1] receive the norms.
-__global__ __launch_bounds__(1024) void k_checkbcs(const FluidDev F, double* nb)
+// sqrt(sum err^2)/nlm.  out (pinned host memory): the errors (nlm, 2), then
+// the two norms.  The sums are the binary tree over the 1024 threads (halves
+// added, 512 apart first): waves 0 and 1 add the sixteen values 64 apart and
+// finish in shuffles, with one barrier in place of ten.
+__global__ __launch_bounds__(1024) void k_checkbcs(const FluidDev F, double* out)
 {
-    __shared__ double sv[1024], sw[1024];
+    __shared__ double sh[2][1024];
     const int t = threadIdx.x;
     double av = 0.0, aw = 0.0;
     for (int np = 1 + t; np <= F.nlm; np += 1024) {
@@ -1109,35 +1129,36 @@ __global__ __launch_bounds__(1024) void k_checkbcs(const FluidDev F, double* nb)
         const double z = LMCC(np, 2);
         if (F.zz[1] < z && z < F.zz[F.n3]) {
             double ucy = 0.0, ucz = 0.0;
-            for (int m = 1; m <= FRIBO_DIMSD; ++m)
+#pragma unroll
+            for (int m = 1; m <= FRIBO_DIMSD; ++m) {
                 ucy = ucy + PHIPRED(np, 1, m) * F.q2[fidx(F, EULINS(np, 1, 1, m), EULINS(np, 1, 2, m))];
-            ev = LMVEL(np, 1) - ucy;
-            for (int m = 1; m <= FRIBO_DIMSD; ++m)
                 ucz = ucz + PHIPRED(np, 2, m) * F.q3[fidx(F, EULINS(np, 2, 1, m), EULINS(np, 2, 2, m))];
+            }
+            ev = LMVEL(np, 1) - ucy;
             ew = LMVEL(np, 2) - ucz;
         }
-        F.bcerr[np - 1] = ev;
-        F.bcerr[(size_t)(np - 1) + F.nlm] = ew;
+        out[np - 1] = ev;
+        out[(size_t)(np - 1) + F.nlm] = ew;
         av = av + ev * ev;
         aw = aw + ew * ew;
     }
-    sv[t] = av;
-    sw[t] = aw;
+    sh[0][t] = av;
+    sh[1][t] = aw;
     __syncthreads();
-    for (int h = 512; h > 0; h >>= 1) {
-        if (t < h) {
-            sv[t] = sv[t] + sv[t + h];
-            sw[t] = sw[t] + sw[t + h];
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        nb[0] = sqrt(sv[0]) / (double)F.nlm;
-        nb[1] = sqrt(sw[0]) / (double)F.nlm;
-    }
+    const int w = t >> 6, lane = t & 63;
+    if (w >= 2) return;
+    double v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = sh[w][lane + 64 * i];
+#pragma unroll
+    for (int h = 8; h > 0; h >>= 1)
+#pragma unroll
+        for (int i = 0; i < h; ++i) v[i] = v[i] + v[i + h];
+    for (int h = 32; h > 0; h >>= 1) v[0] = v[0] + __shfl_down(v[0], h, 64);
+    if (lane == 0) out[2 * (size_t)F.nlm + w] = sqrt(v[0]) / (double)F.nlm;
 }
 
-void launch_checkbcs(const FluidDev& F, double* nb, hipStream_t st)
+void launch_checkbcs(const FluidDev& F, double* out, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_checkbcs, dim3(1), dim3(1024), 0, st, F, nb);
+    hipLaunchKernelGGL(k_checkbcs, dim3(1), dim3(1024), 0, st, F, out);
 }

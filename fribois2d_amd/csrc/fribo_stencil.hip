@@ -1282,12 +1282,39 @@ void launch_mean_b(BatchSet& B, hipStream_t st)
 // (divergence.F90:49-78), kinen (utils_proc.F90:474-515) and cfl
 // (cfl.F90:19-38) as per-block partials; k_diag_final reduces them in a
 // fixed order and adds getintvort (utils_proc.F90:582-629) on the plane kv
-// nearest to z = 18.5 (0: outside the grid).  out[9] = {vmax2, vmax3, vmin2,
-// vmin3, max|div|, ektot, vorticity integral, cflm, q3avg}.
+// nearest to z = 18.5 (0: outside the grid).  out[9] (pinned host memory) =
+// {vmax2, vmax3, vmin2, vmin3, max|div|, ektot, vorticity integral, cflm,
+// q3avg}.
 #define DIAG_NB 256
+
+// The eight reductions of 256 threads, halves combined, 128 apart first:
+// values 2 and 3 minima, 5 and 7 sums, the others maxima.  All eight share one
+// barrier; wave w finishes values w and w + 4 in shuffles (r[0], r[1] of its
+// lane 0).  On 288 x 384 cells k_diag and k_diag_final take 5.3 and 3.9 us;
+// with eight barriers for each of the eight values they took 10 us each.
+__device__ inline double diag_op(int q, double a, double b)
+{
+    return (q == 2 || q == 3) ? fmin(a, b) : ((q == 5 || q == 7) ? a + b : fmax(a, b));
+}
+__device__ inline void diag_reduce(const double (&vals)[8], double (&r)[2])
+{
+    __shared__ double sv[8][256];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) sv[q][t] = vals[q];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int q = w + 4 * i;
+        double v = diag_op(q, diag_op(q, sv[q][lane], sv[q][lane + 128]),
+                           diag_op(q, sv[q][lane + 64], sv[q][lane + 192]));
+        for (int h = 32; h > 0; h >>= 1) v = diag_op(q, v, __shfl_down(v, h, 64));
+        r[i] = v;
+    }
+}
+
 __global__ __launch_bounds__(256) void k_diag(const FluidDev F, double* part)
 {
-    __shared__ double sh[256];
     const int t = threadIdx.x;
     const int per = (F.n3m + DIAG_NB - 1) / DIAG_NB;
     const int k0 = blockIdx.x * per + 1, k1 = min(k0 + per - 1, F.n3m);
@@ -1311,19 +1338,12 @@ __global__ __launch_bounds__(256) void k_diag(const FluidDev F, double* part)
             qs = qs + a3 * dz * dy;
         }
     }
-    double vals[8] = {v2, v3, m2, m3, qm, ek, cf, qs};
-    for (int q = 0; q < 8; ++q) {
-        sh[t] = vals[q];
-        __syncthreads();
-        for (int h = 128; h > 0; h >>= 1) {
-            if (t < h) {
-                const double a = sh[t], b = sh[t + h];
-                sh[t] = (q == 2 || q == 3) ? fmin(a, b) : ((q == 5 || q == 7) ? a + b : fmax(a, b));
-            }
-            __syncthreads();
-        }
-        if (t == 0) part[q * DIAG_NB + blockIdx.x] = sh[0];
-        __syncthreads();
+    const double vals[8] = {v2, v3, m2, m3, qm, ek, cf, qs};
+    double r[2];
+    diag_reduce(vals, r);
+    if ((t & 63) == 0) {
+        part[(t >> 6) * DIAG_NB + blockIdx.x] = r[0];
+        part[((t >> 6) + 4) * DIAG_NB + blockIdx.x] = r[1];
     }
 }
 
@@ -1331,20 +1351,9 @@ __global__ __launch_bounds__(256) void k_diag_final(const FluidDev F, const doub
 {
     __shared__ double sh[256];
     const int t = threadIdx.x;
-    double r[8];
-    for (int q = 0; q < 8; ++q) {
-        sh[t] = part[q * DIAG_NB + t];
-        __syncthreads();
-        for (int h = 128; h > 0; h >>= 1) {
-            if (t < h) {
-                const double a = sh[t], b = sh[t + h];
-                sh[t] = (q == 2 || q == 3) ? fmin(a, b) : ((q == 5 || q == 7) ? a + b : fmax(a, b));
-            }
-            __syncthreads();
-        }
-        r[q] = sh[0];
-        __syncthreads();
-    }
+    double vals[8], r[2];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) vals[q] = part[q * DIAG_NB + t];
     double vi = 0.0;
     if (kv > 0) {
         const double dz = F.zz[kv + 1] - F.zz[kv];
@@ -1356,28 +1365,68 @@ __global__ __launch_bounds__(256) void k_diag_final(const FluidDev F, const doub
         }
     }
     sh[t] = vi;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if (t < h) sh[t] = sh[t] + sh[t + h];
-        __syncthreads();
+    diag_reduce(vals, r);   // its barrier covers sh too
+    const int w = t >> 6;
+    if (w == 0) {
+        double v = (sh[t] + sh[t + 128]) + (sh[t + 64] + sh[t + 192]);
+        for (int h = 32; h > 0; h >>= 1) v = v + __shfl_down(v, h, 64);
+        if (t == 0) out[6] = v;
     }
-    if (t == 0) {
-        out[0] = r[0];
-        out[1] = r[1];
-        out[2] = r[2];
-        out[3] = r[3];
-        out[4] = r[4];
-        out[5] = 0.5 * r[5] / (F.rext2 * F.alx3);
-        out[6] = sh[0];
-        out[7] = r[6];
-        out[8] = r[7] / (F.rext2 * F.alx3);
-    }
+    if ((t & 63) != 0) return;
+    out[w] = r[0];           // vmax2, vmax3, vmin2, vmin3
+    const double vol = F.rext2 * F.alx3;
+    if (w == 0) out[4] = r[1];
+    else if (w == 1) out[5] = 0.5 * r[1] / vol;
+    else if (w == 2) out[7] = r[1];
+    else out[8] = r[1] / vol;
 }
 
 void launch_diag(const FluidDev& F, double* part, int kv, double* out, hipStream_t st)
 {
     hipLaunchKernelGGL(k_diag, dim3(DIAG_NB), dim3(256), 0, st, F, part);
     hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(256), 0, st, F, (const double*)part, kv, out);
+}
+
+// ---------------------------------------------------------------------------
+// Rollback copy of the prognostic state, one launch: blockIdx.y < 5 the
+// fields, two doubles per lane (the pitch is a multiple of 16 doubles, and
+// every field is an allocation of its own); blockIdx.y == 5 the boundary arrays and the step scalars.
+// Sixteen copies by the runtime took 65 us on 512 x 384 cells, almost all
+// of it between the copies; this takes 7 us.
+template <bool SAVE>
+__global__ __launch_bounds__(256) void k_snap(const SnapTab T, DevScalars* S, double* snap)
+{
+    const size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x, st = (size_t)gridDim.x * 256;
+    if (blockIdx.y < 5) {
+        double2* a = (double2*)T.field[blockIdx.y];
+        double2* b = (double2*)(snap + blockIdx.y * T.flen);
+        for (size_t i = i0; i < T.flen / 2; i += st) {
+            if (SAVE) b[i] = a[i];
+            else a[i] = b[i];
+        }
+        return;
+    }
+    double* b = snap + 5 * T.flen;
+    for (int q = 0; q < 10; ++q, b += T.blen) {
+        double* a = T.bnd[q];
+        for (size_t i = i0; i < T.blen; i += st) {
+            if (SAVE) b[i] = a[i];
+            else a[i] = b[i];
+        }
+    }
+    static_assert(sizeof(DevScalars) % sizeof(double) == 0, "copied as doubles");
+    if (i0 < sizeof(DevScalars) / sizeof(double)) {
+        if (SAVE) b[i0] = ((double*)S)[i0];
+        else ((double*)S)[i0] = b[i0];
+    }
+}
+
+void launch_snap(const SnapTab& T, DevScalars* S, double* snap, bool save, hipStream_t st)
+{
+    const size_t nb = (T.flen / 2 + 255) / 256;
+    const dim3 g((unsigned)std::min<size_t>(std::max<size_t>(nb, 1), 1024), 6);
+    if (save) hipLaunchKernelGGL(k_snap<true>, g, dim3(256), 0, st, T, S, snap);
+    else hipLaunchKernelGGL(k_snap<false>, g, dim3(256), 0, st, T, S, snap);
 }
 
 // ---------------------------------------------------------------------------

@@ -985,16 +985,6 @@ __global__ __launch_bounds__(64) void kb_ksolve3(const BGrid<FluidDev> G)
 // results.
 constexpr int KF_COLS = 16;
 
-// Lane n of each 16-lane row of the wave, broadcast to the row (DPP
-// row_newbcast), for a double.
-template <int N>
-__device__ inline double row_bcast(double v)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + N, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + N, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-
 // Row T of the chunk held by the lanes of this 16-lane row (T < 16 * NG).
 template <int T, int NG>
 __device__ inline double krow(const double (&v)[NG])

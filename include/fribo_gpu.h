@@ -145,7 +145,7 @@ int fribo_loads_transfer(fribo_handle h, double kprobe, const double* lmnor, con
  * cannot allocate device memory (code under HIP graph capture, tight
  * coupling loops, harnesses that forbid hipMalloc).  Same arguments, kernels
  * and results; every device buffer of the call lives in a static device
- * array of the library (1.8 MB per device, held until the process ends), so
+ * array of the library (1.3 MB per device, held until the process ends), so
  * it serves at most 8192 markers and returns FRIBO_ERR_LIMIT above that.
  * Calls on one device share that array: calls that overlap on one GPU (two
  * host threads, two handles on one device) race and must be serialised by
