@@ -340,7 +340,7 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
     static_assert(NI * (NST - 2) < 64, "loads in flight per wave");
     static_assert(TM % 16 == 0 && TN % 16 == 0 && BM % WM == 0 && BN % WN == 0, "wave tile");
     static_assert(BK == 16 || BK == 24 || BK == 32, "k-slices");
-    if (S && S->err) return;
+    const bool err = S && S->err;
     __shared__ __attribute__((aligned(1024))) double SM[NST * (SA + SBP)];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave % WM, wn = wave / WM;
@@ -420,6 +420,11 @@ __device__ __forceinline__ void gemm_dma_body(int M, int N, int K, const double*
             if (q > 0 && kleft < BK) set_off(kleft);
             issue(q * ST);
         }
+    if (err) {
+        // the loads on their way land before the wave gives up its LDS
+        wait_vm<0>();
+        return;
+    }
     // slice s is in the stage at cur; slice s + NST - 1 goes into the stage of
     // slice s - 1, at nxt
     int cur = 0, nxt = (NST - 1) * ST;

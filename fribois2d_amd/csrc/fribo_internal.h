@@ -168,6 +168,16 @@ struct SnapTab {
     size_t flen, blen;
 };
 
+// First row of chunk p of a line of n rows in nch chunks, floor(p*n/nch), as
+// the host filled cs[]: computed where a load of cs[] would be one more
+// memory round trip before the rows' own loads (p*n < 2^32 for every line
+// this build accepts; lines of 128 rows and more have 64 chunks).
+__device__ inline int chunk_start(int p, int n, int nch)
+{
+    const unsigned r = (unsigned)p * (unsigned)n;
+    return (int)(nch == 64 ? r >> 6 : r / (unsigned)nch);
+}
+
 // Lane n of each 16-lane row of the wave, broadcast to the row (DPP
 // row_newbcast), for a double.
 template <int N>

@@ -659,25 +659,27 @@ void launch_mls_setup(const FluidDev& F, hipStream_t st)
 __device__ __forceinline__ void mls_interp_body(const FluidDev& F, const VBlock& vb)
 {
     const DevScalars* S = F.S;
-    if (S->err) return;
     const int lane = threadIdx.x;
     const int g = vb.x * 4 + (lane >> 4), m = lane & 15;   // group (n,d), support m
     const bool ing = g < 2 * F.nlm;
     const int n = (ing ? g % F.nlm : 0) + 1, d = (ing ? g / F.nlm : 0) + 1;
-    const bool act = ing && F.active[n - 1];
-    const bool sup = act && m < FRIBO_DIMSD;
+    const int mm = min(m, FRIBO_DIMSD - 1) + 1;
+    // everything that needs no other load first: one memory round trip
+    const bool err = S->err;
+    const double dt = S->dt;
+    const int act = F.active[n - 1], j = EULINS(n, d, 1, mm), k = EULINS(n, d, 2, mm);
+    const double ph = PHI(n, d, mm), vel = LMVEL(n, d), cl = CL(n, d);
+    const bool sup = ing && act && m < FRIBO_DIMSD && !err;
     const double* q = (d == 1) ? F.q2 : F.q3;
     const double* r = (d == 1) ? F.rhs2 : F.rhs3;
-    double prod = 0.0, ph = 0.0;
+    double prod = 0.0;
     if (sup) {
-        const int j = EULINS(n, d, 1, m + 1), k = EULINS(n, d, 2, m + 1);
         // q2f is written for 2<=j<=n2m (INVTR.F90:145-149), q3f for
         // 2<=k<=n3m (INVTR.F90:273-277); elsewhere it keeps its zero start
         const bool def = (d == 1) ? (j >= 2 && j <= F.n2m && k >= 1 && k <= F.n3m)
                                   : (j >= 1 && j <= F.n2m && k >= 2 && k <= F.n3m);
         const size_t c = def ? fidx(F, j, k) : 0;
         const double qf = def ? q[c] + r[c] : 0.0;
-        ph = PHI(n, d, m + 1);
         prod = ph * qf;
     }
     const int base = lane & ~15;
@@ -685,9 +687,9 @@ __device__ __forceinline__ void mls_interp_body(const FluidDev& F, const VBlock&
 #pragma unroll
     for (int t = 0; t < FRIBO_DIMSD; ++t) u = u + __shfl(prod, base + t, 64);
     if (!sup) return;
-    const double f = (LMVEL(n, d) - u) / S->dt;
+    const double f = (vel - u) / dt;
     double* con = F.contrib + (size_t)(d - 1) * F.nlm * FRIBO_DIMSD;
-    con[(size_t)(n - 1) * FRIBO_DIMSD + m] = CL(n, d) * ph * f;
+    con[(size_t)(n - 1) * FRIBO_DIMSD + m] = cl * ph * f;
 }
 __global__ __launch_bounds__(64) void k_mls_interp(const FluidDev F)
 {
@@ -705,53 +707,51 @@ __global__ __launch_bounds__(64) void kb_mls_interp(const BGrid<FluidDev> G)
 __device__ __forceinline__ void mls_spread_body(const FluidDev& F, const VBlock& vb)
 {
     const DevScalars* S = F.S;
-    if (S->err) return;
     const int d = vb.y;
     const int i = vb.x * 64 + threadIdx.x;
-    if (i >= F.nlm * FRIBO_DIMSD) return;
-    const unsigned long long* gk = F.keys + (size_t)d * F.maxkeys;
-    const unsigned long long key = gk[i];
-    if (key == KEY_NONE) return;
-    const unsigned long long cell = key >> ENT_BITS;
-    if (i > 0 && (gk[i - 1] >> ENT_BITS) == cell) return;
-    const double* con = F.contrib + (size_t)d * F.nlm * FRIBO_DIMSD;
     const int nreal = F.nlm * FRIBO_DIMSD;
-    // the segment is read eight keys at a time (independent loads), summed in order
+    if (i >= nreal) return;
+    const unsigned long long* gk = F.keys + (size_t)d * F.maxkeys;
+    const double* con = F.contrib + (size_t)d * nreal;
+    // the segment is read eight keys at a time (independent loads), summed in
+    // order; the first eight travel with the key before it and the scalars
+    auto load = [&](unsigned long long (&kb)[8], int e0) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) kb[u] = gk[min(e0 + u, nreal - 1)];
+    };
+    const bool err = S->err;
+    const double dt = S->dt;
+    unsigned long long kb[8];
+    load(kb, i);
+    const unsigned long long before = gk[max(i - 1, 0)];
+    const unsigned long long key = kb[0];
+    const unsigned long long cell = key >> ENT_BITS;
+    if (err || key == KEY_NONE || (i > 0 && (before >> ENT_BITS) == cell)) return;
+    const unsigned cl32 = (unsigned)cell, n2u = (unsigned)F.n2;
+    const int j = (int)(cl32 % n2u) + 1, k = (int)(cl32 / n2u) + 1;
+    const bool put = k != F.n3m && (d == 0 ? (j >= 2 && j <= F.n2m && k >= 1) : (j >= 1 && j <= F.n2m && k >= 2));
+    double* dst = (d == 0 ? F.rhs2 : F.rhs3) + (put ? fidx(F, j, k) : 0);
+    const double old = *dst;
     double acc = 0.0;
     bool open = true;
     for (int e0 = i; open && e0 < nreal; e0 += 8) {
-        unsigned long long kb[8];
+        if (e0 != i) load(kb, e0);
         double cv[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) kb[u] = (e0 + u < nreal) ? gk[e0 + u] : KEY_NONE;
-#pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const bool in = kb[u] != KEY_NONE && (kb[u] >> ENT_BITS) == cell;
+            const bool in = e0 + u < nreal && kb[u] != KEY_NONE && (kb[u] >> ENT_BITS) == cell;
             cv[u] = in ? con[kb[u] & ENT_MASK] : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const bool in = open && kb[u] != KEY_NONE && (kb[u] >> ENT_BITS) == cell;
+            const bool in = open && e0 + u < nreal && kb[u] != KEY_NONE && (kb[u] >> ENT_BITS) == cell;
             if (in) acc = acc + cv[u];
             open = in;
         }
     }
-    const unsigned cl32 = (unsigned)cell, n2u = (unsigned)F.n2;
-    const int j = (int)(cl32 % n2u) + 1, k = (int)(cl32 / n2u) + 1;
     const double fval = (k == F.n3m) ? 0.0 : acc;
     F.segval[(size_t)d * F.maxkeys + i] = fval;
-    if (k == F.n3m) return;
-    if (d == 0) {
-        if (j >= 2 && j <= F.n2m && k >= 1) {
-            const size_t c = fidx(F, j, k);
-            F.rhs2[c] = F.rhs2[c] + fval * S->dt;
-        }
-    } else {
-        if (j >= 1 && j <= F.n2m && k >= 2) {
-            const size_t c = fidx(F, j, k);
-            F.rhs3[c] = F.rhs3[c] + fval * S->dt;
-        }
-    }
+    if (put) *dst = old + fval * dt;
 }
 __global__ __launch_bounds__(64) void k_mls_spread(const FluidDev F)
 {

@@ -143,7 +143,7 @@ struct StepScalars {
     int err;
 };
 
-__device__ StepScalars step_scalars(const FluidDev& F, int n, int ns, double dt_in, double dt_o, double s_dt,
+__device__ __forceinline__ StepScalars step_scalars(const FluidDev& F, int n, int ns, double dt_in, double dt_o, double s_dt,
                                     double s_cflm, double s_beta, int s_err, double* sh, double* sh2)
 {
     __shared__ StepScalars out;
@@ -229,13 +229,30 @@ __device__ inline void sys_coefs(const FluidDev& F, const KSys& K, const double*
     else { am = F.am3j; ac = F.ac3j; ap = F.ap3j; }
 }
 
+// Coefficients of rows t and t + 1024 of system K (clamped to the last row),
+// loaded at kernel entry while the step scalars are still on their way.
+struct SysRows {
+    double am[2], ac[2], ap[2];
+};
+__device__ __forceinline__ void sys_load(const double* am, const double* ac, const double* ap, int n, int kofs,
+                                         int r0, SysRows& v)
+{
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int idx = min(r0 + 1024 * u, n - 1) + kofs;
+        v.am[u] = am[idx];
+        v.ac[u] = ac[idx];
+        v.ap[u] = ap[idx];
+    }
+}
+
 // Line-invariant factors of one partitioned Helmholtz system for this
 // substep (solve_fluid.F90:77-87,126-143,185-200,260-278: rows normalised by
 // 1/(1 - betadx*ac)).  Row coefficients go to LDS; lane p of the first wave
 // then eliminates chunk p (forward multipliers, left-coupling vector and the
 // weights that turn forward values into first-row values), and the wave
 // builds the separator system and its PCR multipliers.
-__device__ void sys_prepare(const FluidDev& F, const KSys& K, double betadx, double* lds)
+__device__ __forceinline__ void sys_prepare(const FluidDev& F, const KSys& K, double betadx, double* lds, const SysRows& pre)
 {
     const int t = threadIdx.x;
     const int n = K.n;
@@ -243,28 +260,25 @@ __device__ void sys_prepare(const FluidDev& F, const KSys& K, double betadx, dou
     double* la = lds;
     double* lc = lds + ns;
     double* lS = lds + 2 * ns;
-    const double *am, *ac, *ap;
-    sys_coefs(F, K, am, ac, ap);
-    // rows t and t + 1024 per pass (workgroups of 1024 threads), both rows'
-    // loads issued before the first row's stores, which the compiler would
-    // otherwise keep ahead of the second row's loads (the coefficient arrays
-    // and K's factor arrays may alias as far as it knows)
+    // rows t and t + 1024 per pass (workgroups of 1024 threads), the first
+    // pass from pre; both rows' loads are issued before the first row's
+    // stores, which the compiler would otherwise keep ahead of the second
+    // row's loads (the coefficient arrays and K's factor arrays may alias as
+    // far as it knows)
     for (int r0 = t; r0 < n; r0 += 2048) {
-        double amr[2], acr[2], apr[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int idx = min(r0 + 1024 * u, n - 1) + K.kofs;
-            amr[u] = am[idx];
-            acr[u] = ac[idx];
-            apr[u] = ap[idx];
+        SysRows v = pre;
+        if (r0 != t) {
+            const double *am, *ac, *ap;
+            sys_coefs(F, K, am, ac, ap);
+            sys_load(am, ac, ap, n, K.kofs, r0, v);
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const int r = r0 + 1024 * u;
             if (r < n) {
-                const double b = 1.0 / (1.0 - acr[u] * betadx);
-                const double amv = -amr[u] * betadx * b;
-                const double apv = -apr[u] * betadx * b;
+                const double b = 1.0 / (1.0 - v.ac[u] * betadx);
+                const double amv = -v.am[u] * betadx * b;
+                const double apv = -v.ap[u] * betadx * b;
                 const double av = (r == 0) ? 0.0 : amv, cv = (r == n - 1) ? 0.0 : apv;
                 const int q = sp_slot(r);
                 la[q] = av;
@@ -285,7 +299,7 @@ __device__ void sys_prepare(const FluidDev& F, const KSys& K, double betadx, dou
     const int p = t;
     double alpha = 0.0, beta = 1.0, gamma = 0.0, vs = 0.0, ws = 0.0, ce = 0.0;
     if (p < K.nch) {
-        const int s = K.cs[p], e = K.cs[p + 1] - 1;
+        const int s = chunk_start(p, n, K.nch), e = chunk_start(p + 1, n, K.nch) - 1;
         double cpp = 0.0, vpp = 1.0, gg = 1.0, wl = 0.0, glast = 1.0, vsum = 0.0;
 #pragma unroll 4
         for (int i = s; i <= e - 1; ++i) {
@@ -360,8 +374,8 @@ size_t sysprep_lds_bytes(const FluidDev& F)
     return (size_t)3 * (n + (n >> 5) + 1) * sizeof(double);
 }
 
-// The first PR_PRE pressure partials of thread t (entries t, t+1024, ...,
-// clamped to the last), loaded ahead so that they travel with the kernel's
+// The first PR_PRE pressure partials of thread t (entries t, t+1024, ...),
+// loaded ahead so that they travel with the kernel's
 // other loads (8192 partials: the 2048x1536 grid has 6400, 3328 in the
 // mirror form).
 #define PR_PRE 8
@@ -369,7 +383,8 @@ __device__ inline void pr_load(const FluidDev& F, double* v)
 {
     const int t = threadIdx.x, n = F.npr_part;
 #pragma unroll
-    for (int u = 0; u < PR_PRE; ++u) v[u] = F.pr_part[min(t + 1024 * u, n - 1)];
+    for (int u = 0; u < PR_PRE; ++u)
+        if (t + 1024 * u < n) v[u] = F.pr_part[t + 1024 * u];
 }
 
 // Pressure mean of the previous substep (pr_submean, updvp.F90:125-141) from
@@ -477,11 +492,15 @@ struct BcRows {
     double qs2[2], qs3[2], dqs2[2], dqs3[2], dqn2[2], dqn3[2];
 };
 
+// Only rows that exist are loaded: of a small grid's 1024 threads most own
+// none, and a load that only repeats the last row still costs the CU's one
+// address unit its cycles.
 __device__ inline void bc_load(const FluidDev& F, int mean, int j0, BcRows& b)
 {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        const int j = min(j0 + 1024 * u, F.n2m);
+        const int j = j0 + 1024 * u;
+        if (j > F.n2m) continue;
         b.qn2[u] = F.qb2n[j];
         b.qn3[u] = F.qb3n[j];
         b.q2e[u] = F.q2[fidx(F, j, F.n3m)];
@@ -509,7 +528,7 @@ __device__ inline void bc_load(const FluidDev& F, int mean, int j0, BcRows& b)
 // step scalars are known, so that a single memory round trip serves the
 // common case n2m <= 2048; the outflow increments of those rows stay in
 // registers for the mass correction.
-__device__ void bc_rows(const FluidDev& F, const StepScalars& r, int mean, double* sh, const BcRows& pre,
+__device__ __forceinline__ void bc_rows(const FluidDev& F, const StepScalars& r, int mean, double* sh, const BcRows& pre,
                         const double* prv)
 {
     DevScalars* S = F.S;
@@ -586,6 +605,9 @@ __device__ void bc_rows(const FluidDev& F, const StepScalars& r, int mean, doubl
 // Workgroup 0: the previous substep's pressure mean and boucqt (mean != 0),
 // finalize CFL/dt (substep 1), RK coefficients, boucdq.
 // Workgroups 1..4: factors of the four Helmholtz systems of this substep.
+// Bound by workgroup 0's chain: one CU's address unit takes about eight cycles
+// for every wave's load, useful or not, so only what exists is loaded (9.1 ->
+// 7.2 us at 384x288, 13 -> 11.6 at 2048x1536).
 __device__ __forceinline__ void bc_body(const FluidDev& F, const VBlock& vb, int n, int mean)
 {
     extern __shared__ double dyn[];
@@ -597,26 +619,38 @@ __device__ __forceinline__ void bc_body(const FluidDev& F, const VBlock& vb, int
     const double dt_in = S->in_dt, dt_o_in = S->in_dto;
     const double s_dt = S->dt, s_cflm = S->cflm, s_beta = S->beta;
     const int s_err = S->err;
+    if (vb.x > 0) {
+        const int sys = vb.x - 1;
+        SysRows pre;
+        {
+            // member by member: a reference to one of the four systems, live
+            // across step_scalars, would put the kernel's arguments in scratch
+            const auto of = [&](auto get) {
+                return sys == 0 ? get(F.ks[0]) : sys == 1 ? get(F.ks[1]) : sys == 2 ? get(F.js[0]) : get(F.js[1]);
+            };
+            const int src = of([](const KSys& q) { return q.src; });
+            const double* am = src == 0 ? F.am3sk : src == 1 ? F.am2j : F.am3j;
+            const double* ac = src == 0 ? F.ac3sk : src == 1 ? F.ac2j : F.ac3j;
+            const double* ap = src == 0 ? F.ap3sk : src == 1 ? F.ap2j : F.ap3j;
+            sys_load(am, ac, ap, of([](const KSys& q) { return q.n; }), of([](const KSys& q) { return q.kofs; }), t, pre);
+        }
+        const KSys& K = (sys < 2) ? F.ks[sys] : F.js[sys - 2];
+        const StepScalars r = step_scalars(F, n, ns, dt_in, dt_o_in, s_dt, s_cflm, s_beta, s_err, sh, sh2);
+        if (!r.err) sys_prepare(F, K, r.betadx, dyn, pre);
+        return;
+    }
     // workgroup 0: its row values and pressure partials, in flight with the above
     BcRows pre;
     double prv[PR_PRE] = {};
-    if (vb.x == 0) {
-        bc_load(F, mean, 1 + t, pre);
-        if (mean) pr_load(F, prv);
-    }
+    bc_load(F, mean, 1 + t, pre);
+    if (mean) pr_load(F, prv);
     const StepScalars r = step_scalars(F, n, ns, dt_in, dt_o_in, s_dt, s_cflm, s_beta, s_err, sh, sh2);
     if (r.err) {
-        if (vb.x == 0 && t == 0 && n == 1) {
+        if (t == 0 && n == 1) {
             S->cflm = r.cflm;
             S->dt = r.dt;
             S->err = r.err;
         }
-        return;
-    }
-    if (vb.x > 0) {
-        const int sys = vb.x - 1;
-        const KSys& K = (sys < 2) ? F.ks[sys] : F.js[sys - 2];
-        sys_prepare(F, K, r.betadx, dyn);
         return;
     }
     if (t == 0) {
@@ -773,7 +807,7 @@ __device__ inline double dn1(double v) { return __shfl_down(v, 1, 64); }
 __device__ __forceinline__ void rhs_body(const FluidDev& F, const VBlock& vb)
 {
     const DevScalars* S = F.S;
-    if (S->err) return;
+    const bool err = S->err;
     const int lane = threadIdx.x & 63;
     const int ntj = (F.n2m + WJ - 1) / WJ, bx = (int)vb.x * SW_RHS + (int)(threadIdx.x >> 6);
     if (bx >= ntj) return;
@@ -865,7 +899,7 @@ __device__ __forceinline__ void rhs_body(const FluidDev& F, const VBlock& vb)
         const double q3W = up1(q3c), q3Wp = up1(q3p), q3E = dn1(q3c);
         const double prW = up1(prc);
         (void)q2Ep;
-        if (out) {
+        if (out && !err) {
             // ---- q2: hdnl2 + invtr2 (j >= 2)
             if (j >= 2) {
                 double a = q2E + q2c, b = q2W + q2c;
@@ -971,7 +1005,7 @@ template <bool MIRROR>
 __device__ __forceinline__ void div_body(const FluidDev& F, const VBlock& vb)
 {
     const DevScalars* S = F.S;
-    if (S->err) return;
+    const bool err = S->err;
     const int lane = threadIdx.x & 63;
     const int jtop = MIRROR ? F.n2m / 2 : F.n2m;   // last output row of the tiles
     const int ntj = (jtop + WJ - 1) / WJ, bx = (int)vb.x * SW_DIV + (int)(threadIdx.x >> 6);
@@ -1013,7 +1047,7 @@ __device__ __forceinline__ void div_body(const FluidDev& F, const VBlock& vb)
         const double q2E = dn1(q2c);
         const double q2Em = MIRROR ? up1(q2cm) : 0.0;
         const double udx3m_k = lane_bcast(l_udx3m, k - k0);
-        if (out) {
+        if (out && !err) {
             double dq = (q2E - q2c) * udx2m + (q3p - q3c) * udx3m_k;
             if (MIRROR) {
                 const double dqm = (q2Em - q2cm) * udx2mm + (q3pm - q3cm) * udx3m_k;
@@ -1077,7 +1111,7 @@ template <bool MIRROR>
 __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
 {
     const DevScalars* S = F.S;
-    if (S->err) return;
+    const bool err = S->err;
     const int lane = threadIdx.x & 63;
     const int h = F.n2m / 2;
     const int jtop = MIRROR ? h : F.n2m;   // last output row of the tiles
@@ -1115,30 +1149,27 @@ __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
         double* __restrict__ q3 = F.q3;
         double* __restrict__ pr = F.pr;
         const int n3m = F.n3m;
-        // gauge constant of the transform along y (0 along z): the backward
-        // transform's partials, summed in tile order
+        // dph of row j (t) and of the mirrored row (m) at plane offset o: the
+        // loads, and the values with the gauge constant doff off
+        auto raw = [&](size_t o, bool ok, double& a, double& b) {
+            a = (inj && ok) ? dph[c + o] : 0.0;
+            b = (injm && ok) ? dph[cm + o] : 0.0;
+        };
         double doff = 0.0;
-        if (F.taxis == 1) {
-            double g = 0.0;
-            for (int q = 0; q < F.ngpart; ++q) g = g + F.gpart[q];
-            doff = g * F.zginv;
-        }
-        if (vb.x == 0 && vb.y == 0 && lane == 0) F.S->dphoff = doff;
-        // dph of row j (t) and of the mirrored row (m) at plane offset o
-        auto ld = [&](size_t o, bool ok, double& t, double& m) {
+        auto val = [&](bool ok, double a, double b, double& t, double& m) {
             if (!MIRROR) {
-                t = (inj && ok) ? dph[c + o] - doff : 0.0;
+                t = (inj && ok) ? a - doff : 0.0;
                 return;
             }
-            const double a = (inj && ok) ? dph[c + o] : 0.0, b = (injm && ok) ? dph[cm + o] : 0.0;
             t = (lower ? a + b : b - a) - doff;
             m = (lower ? a - b : a + b) - doff;
         };
         double dm, dc, dn, dm_m = 0.0, dc_m = 0.0, dn_m = 0.0;
-        ld(-P, k0 > 1, dm, dm_m);
-        ld(0, true, dc, dc_m);
         // plane k+1 of dph and plane k of q2/q3/pr are loaded one iteration ahead
-        ld(P, k0 < n3m, dn, dn_m);
+        double r0, r1, r2, s0, s1, s2;
+        raw(-P, k0 > 1, r0, s0);
+        raw(0, true, r1, s1);
+        raw(P, k0 < n3m, r2, s2);
         double q2n = out ? q2[c] : 0.0, q3n = out ? q3[c] : 0.0, prn = out ? pr[c] : 0.0;
         double q2n_m = 0.0, q3n_m = 0.0, prn_m = 0.0;
         if (MIRROR && out) {
@@ -1150,6 +1181,18 @@ __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
         const int kl = min(k0 + lane, n3m);
         const double l_udx3c = F.udx3c[kl], l_apphk = F.apphk[kl], l_acphk = F.acphk[kl];
         const double l_amphk = F.amphk[kl], l_dz = F.zz[kl + 1] - F.zz[kl];
+        // gauge constant of the transform along y (0 along z): the backward
+        // transform's partials, summed in tile order, while the loads above
+        // are in flight
+        if (F.taxis == 1) {
+            double g = 0.0;
+            for (int q = 0; q < F.ngpart; ++q) g = g + F.gpart[q];
+            doff = g * F.zginv;
+        }
+        if (vb.x == 0 && vb.y == 0 && lane == 0 && !err) F.S->dphoff = doff;
+        val(k0 > 1, r0, s0, dm, dm_m);
+        val(true, r1, s1, dc, dc_m);
+        val(k0 < n3m, r2, s2, dn, dn_m);
         for (int k = k0; k <= k1; ++k, c += P, cm += P) {
             const int kk = k - k0;
             const double udx3c_k = lane_bcast(l_udx3c, kk), apphk_k = lane_bcast(l_apphk, kk);
@@ -1158,7 +1201,8 @@ __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
             const double dp = dn, q2v = q2n, q3v = q3n, prv0 = prn;
             const double dp_m = dn_m, q2v_m = q2n_m, q3v_m = q3n_m, prv0_m = prn_m;
             if (k < k1) {
-                ld(2 * P, k + 1 < n3m, dn, dn_m);
+                raw(2 * P, k + 1 < n3m, r2, s2);
+                val(k + 1 < n3m, r2, s2, dn, dn_m);
                 q2n = out ? q2[c + P] : 0.0;
                 q3n = out ? q3[c + P] : 0.0;
                 prn = out ? pr[c + P] : 0.0;
@@ -1170,7 +1214,7 @@ __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
             }
             const double dW = up1(dc), dE = dn1(dc);
             const double dW_m = MIRROR ? dn1(dc_m) : 0.0, dE_m = MIRROR ? up1(dc_m) : 0.0;
-            if (out) {
+            if (out && !err) {
                 const double usukm = al * dt * udx3c_k;
                 {
                     const double dJm = jlo ? dc : dW;     // dph(jmv(j))
@@ -1206,7 +1250,7 @@ __device__ __forceinline__ void upd_body(const FluidDev& F, const VBlock& vb)
             // end of a partial's planes: wave reduction (fixed order)
             if (k % mkp == 0 || k == n3m) {
                 for (int off = 32; off > 0; off >>= 1) part = part + __shfl_xor(part, off, 64);
-                if (lane == 0) F.pr_part[(k - 1) / mkp * ntj + bx] = part;
+                if (lane == 0 && !err) F.pr_part[(k - 1) / mkp * ntj + bx] = part;
                 part = 0.0;
             }
         }

@@ -30,11 +30,6 @@
 #include <algorithm>
 #include <utility>
 
-// j-lines per wave of the batched Helmholtz j-line launch
-#ifndef FRIBO_JB_LPW
-#define FRIBO_JB_LPW 16
-#endif
-
 // Row r of a j-line belongs to chunk owner(r) when chunk starts are
 // floor(p*n/nch); (r+1)*nch < 2^32 for every line this build accepts.
 __device__ inline int chunk_owner(int r, int n, int nch)
@@ -63,16 +58,13 @@ __device__ inline void line_map(int* slot, const int* cs, int n, int nch, int st
 // (off_p = MAXR - (m_p - 1)) and the separator at offset MAXR, so a solve step
 // tt reads offset tt of every lane with no per-lane clamping.
 template <int NR>
-__device__ inline void line_map_pad(int* slot, const int* cs, int n, int nch, int stride, int lane, int maxr)
+__device__ inline void line_map_pad(int* slot, int n, int nch, int stride, int lane, int maxr)
 {
-    const int csl = lane < nch ? cs[lane] : 0;
-    const int csn = lane < nch ? cs[lane + 1] : 0;
-    const int offl = maxr - (csn - csl - 1);
 #pragma unroll
     for (int u = 0; u < NR; ++u) {
         const int r = lane + 64 * u;
         const int p = chunk_owner(r < n ? r : n - 1, n, nch);
-        const int c0 = __shfl(csl, p, 64), o = __shfl(offl, p, 64);
+        const int c0 = chunk_start(p, n, nch), o = maxr - (chunk_start(p + 1, n, nch) - c0 - 1);
         slot[u] = r < n ? p * stride + (r - c0) + o : -1;
     }
 }
@@ -148,8 +140,7 @@ __device__ __forceinline__ void jsolve_hp_body(const FluidDev& F, const VBlock& 
 {
     constexpr int NR = MAXR + 1;
     extern __shared__ double lds[];
-    const DevScalars* S = F.S;
-    if (S->err) return;
+    const bool err = F.S->err;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int half = (int)vb.gx >> 1;
     const int f = (int)vb.x < half ? 0 : 1;
@@ -163,8 +154,15 @@ __device__ __forceinline__ void jsolve_hp_body(const FluidDev& F, const VBlock& 
     const int n = K.n, nch = K.nch, stride = F.jstride;
     const int p = lane;
     const bool own = p < nch;
-    const int m = own ? K.cs[p + 1] - K.cs[p] : 1;
+    const int m = own ? chunk_start(p + 1, n, nch) - chunk_start(p, n, nch) : 1;
     const int ie = (m - 1) * 64 + p;
+    const int step = nwgf * JW;
+    const int iters = (nlines + step - 1) / step;
+    int line = wg * JW + wave;
+    // the first line's rows, in flight with the factors
+    double pre[NR];
+    line_fetch<NR>(pre, srcb + fidx(F, K.kofs, kfirst + (line < nlines ? line : 0)), n, lane);
+    const double ce = own ? K.c[ie] : 0.0;
 
     double* fSI = lds;
     double* fAI = fSI + NR * 64;
@@ -186,7 +184,7 @@ __device__ __forceinline__ void jsolve_hp_body(const FluidDev& F, const VBlock& 
         for (int u = 0; u < NCP; ++u) {
             const int i = tid + u * 64 * JW;
             const int q = i & 63, tt = i >> 6;
-            const int mq = q < nch ? K.cs[q + 1] - K.cs[q] : 0;
+            const int mq = q < nch ? chunk_start(q + 1, n, nch) - chunk_start(q, n, nch) : 0;
             const int t = tt - MAXR + mq - 1;
             ok[u] = i < NR * 64 && mq > 0 && t >= 0;
             const int ic = ok[u] ? t * 64 + q : 0;
@@ -229,18 +227,14 @@ __device__ __forceinline__ void jsolve_hp_body(const FluidDev& F, const VBlock& 
         // the padding rows of the staging area start at zero
         for (int i = lane; i < 64 * stride; i += 64) stage[i] = 0.0;
     }
-    const double ce = own ? K.c[ie] : 0.0;
     int slot[NR];
-    line_map_pad<NR>(slot, K.cs, n, nch, stride, lane, MAXR);
-    const int step = nwgf * JW;
-    const int iters = (nlines + step - 1) / step;
-    int line = wg * JW + wave;
+    line_map_pad<NR>(slot, n, nch, stride, lane, MAXR);
     double* row = stage + p * stride;
     // one line: stage it, refill its buffer with the line `ahead` lines of
     // this wave later (one line of loads in flight: a second buffer takes
     // the kernel past 256 VGPRs), solve, write back
     auto solve = [&](double (&pre)[NR], int ahead) {
-        const bool act = line < nlines;
+        const bool act = line < nlines && !err;
         line_put<NR>(stage, pre, slot);
         const int nxt = line + ahead * step;
         line_fetch<NR>(pre, srcb + fidx(F, K.kofs, kfirst + (nxt < nlines ? nxt : 0)), n, lane);
@@ -284,8 +278,6 @@ __device__ __forceinline__ void jsolve_hp_body(const FluidDev& F, const VBlock& 
         wave_lds_sync();
         line += step;
     };
-    double pre[NR];
-    line_fetch<NR>(pre, srcb + fidx(F, K.kofs, kfirst + (line < nlines ? line : 0)), n, lane);
     __syncthreads();
     for (int it = 0; it < iters; ++it) solve(pre, 1);
 }
@@ -565,12 +557,18 @@ __global__ __launch_bounds__(64 * JW) void kb_jsolve_p(const BGrid<FluidDev> G)
     jsolve_p_body<MAXR, JW>(*Fp, vb);
 }
 
+static constexpr int kJh4Lines = 1536;
+
 template <int MAXR>
 static void launch_h(const FluidDev& F, hipStream_t st)
 {
     const int lines = 2 * F.n3m - 1;
     const int sd = F.jstride;
-    if (jsolve_h_lds_bytes(MAXR, 8, sd, true) <= (size_t)F.lds_max) {
+    // Few lines are spread over more workgroups of four waves; many share one
+    // staging of the factors among eight.  Eight / four waves, us: 64x48 8.0 /
+    // 6.8, 384x288 8.2 / 6.7, 480x600 11.4 / 9.6, 810x672 14.8 / 12.6, 1301x977
+    // 16.8 / 16.6, 2048x1536 24.5 / 29.8.
+    if (lines > kJh4Lines && jsolve_h_lds_bytes(MAXR, 8, sd, true) <= (size_t)F.lds_max) {
         const int g = std::max(2, std::min(256, (lines + 7) / 8) & ~1);
         hipLaunchKernelGGL((k_jsolve_hp<MAXR, 8>), dim3(g), dim3(512), jsolve_h_lds_bytes(MAXR, 8, sd, true), st, F);
     } else if (jsolve_h_lds_bytes(MAXR, 4, sd, true) <= (size_t)F.lds_max) {
@@ -658,11 +656,22 @@ static void launch_h_b(BatchSet& B, hipStream_t st)
     const size_t lim = (size_t)B.hF[0].lds_max;
     auto lines = [](const FluidDev& F) { return 2 * F.n3m - 1; };
     if (jsolve_h_lds_bytes(MAXR, 8, sd, true) <= lim) {
-        // FRIBO_JB_LPW lines per wave: each workgroup first stages the
-        // factors of its instance in LDS, which many short lines amortise
-        constexpr int LPW = FRIBO_JB_LPW;
-        blaunch(B, BK_JH, bdims(B, [&](const FluidDev& F) { return dim3(std::max(2, std::min(256, (lines(F) + 8 * LPW - 1) / (8 * LPW)) & ~1)); }),
-                kb_jsolve_hp<MAXR, 8>, dim3(512), jsolve_h_lds_bytes(MAXR, 8, sd, true), st);
+        // Lines per wave: each workgroup first stages the factors of its
+        // instance in LDS, so the fewest lines that still let every workgroup
+        // be resident at once.  24 instances of 96..448 x 70..380: 30.8 us
+        // with 2 lines, 25.5 with 3 (the rule's), 27.0 with 4, 30.1 with 8, 52.8
+        // with 16.
+        const size_t ldsb = jsolve_h_lds_bytes(MAXR, 8, sd, true);
+        const int resident = 256 * std::max(1, (int)(lim / ldsb));
+        auto groups = [&](const FluidDev& F, int lpw) { return std::max(2, std::min(256, (lines(F) + 8 * lpw - 1) / (8 * lpw)) & ~1); };
+        int lpw = 1;
+        for (; lpw < 16; ++lpw) {
+            int tot = 0;
+            for (const auto& F : B.hF) tot += groups(F, lpw);
+            if (tot <= resident) break;
+        }
+        blaunch(B, BK_JH, bdims(B, [&](const FluidDev& F) { return dim3(groups(F, lpw)); }),
+                kb_jsolve_hp<MAXR, 8>, dim3(512), ldsb, st);
     } else if (jsolve_h_lds_bytes(MAXR, 4, sd, true) <= lim) {
         blaunch(B, BK_JH, bdims(B, [&](const FluidDev& F) { return dim3(std::max(2, std::min(256, (lines(F) + 3) / 4) & ~1)); }),
                 kb_jsolve_hp<MAXR, 4>, dim3(256), jsolve_h_lds_bytes(MAXR, 4, sd, true), st);
@@ -971,25 +980,49 @@ __global__ __launch_bounds__(64) void kb_ksolve3(const BGrid<FluidDev> G)
 }
 
 // One-pass form of the three passes above for chunks of at most 32 rows
-// (lines of up to 2048 rows): a workgroup of 1024 threads owns KF_COLS = 16
-// columns of one field and every chunk of them; thread (column jl, chunk p)
-// with jl = lane % 16, p = 4 * wave + lane / 16, so a wave's loads cover 16
-// columns (128 bytes) of 4 chunks.  The chunk's forward-eliminated rows stay
-// in registers across the separator solve, so the right-hand side is read
-// once: read src, read q, write q.  The 16 lanes of a chunk hold its
-// coefficient rows (lane u rows u and u + 16) and each elimination step takes
-// its row by a DPP broadcast within the 16-lane row (no LDS traffic); the
-// chunk summaries go to LDS, wave w solves the separator system of column w
-// with the multipliers and operation order of k_ksolve2, and the
-// back-substitution is that of k_ksolve3, so both forms give identical
-// results.
-constexpr int KF_COLS = 16;
+// (lines of up to 2048 rows): a workgroup of 64 NC threads owns NC columns of
+// one field and every chunk of them, thread (column t % NC, chunk t / NC).
+// The chunk's forward-eliminated rows stay in registers across the separator
+// solve, so the right-hand side is read once: read src, read q, write q.  The
+// NC lanes of a chunk hold its coefficient rows (lane u rows u, u + NC, ...)
+// and each elimination step takes its row by a DPP broadcast within the
+// group (no LDS traffic); the chunk summaries go to LDS, wave w solves the
+// separator system of column w with the multipliers and operation order of
+// k_ksolve2, and the back-substitution is that of k_ksolve3, so both forms
+// give identical results.
+//
+// On small and middle grids it is bound by the chain of loads and by the CU's
+// address unit, through which every wave's loads pass: so the factors, and
+// with short chunks the rows of q, are on their way before the elimination
+// starts, nothing waits for the error flag before the first store, the chunk
+// bounds are computed instead of loaded, and the columns per workgroup follow
+// the grid (launch_kf).  384x288 9.3 -> 6.4 us, 810x672 15.0 -> 12.6,
+// 1301x977 22.8 -> 20.3; 2048x1536 36 -> 34, there bound by HBM (151 MB).
+// Lane N of each group of NC lanes, broadcast to the group, for a double.
+template <int NC, int N>
+__device__ inline double group_bcast(double v)
+{
+    static_assert(NC == 16 || NC == 8 || NC == 4, "groups of a DPP row");
+    if (NC == 16) return row_bcast<N & 15>(v);
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    if (NC == 4) {   // quad_perm
+        lo = __builtin_amdgcn_update_dpp(0, lo, 0x55 * (N & 3), 0xF, 0xF, false);
+        hi = __builtin_amdgcn_update_dpp(0, hi, 0x55 * (N & 3), 0xF, 0xF, false);
+        return __hiloint2double(hi, lo);
+    }
+    // lane N of the row to lanes 0-7, lane N + 8 to lanes 8-15
+    int l = __builtin_amdgcn_update_dpp(0, lo, 0x150 + (N & 7), 0xF, 0x3, false);
+    int h = __builtin_amdgcn_update_dpp(0, hi, 0x150 + (N & 7), 0xF, 0x3, false);
+    l = __builtin_amdgcn_update_dpp(l, lo, 0x158 + (N & 7), 0xF, 0xC, false);
+    h = __builtin_amdgcn_update_dpp(h, hi, 0x158 + (N & 7), 0xF, 0xC, false);
+    return __hiloint2double(h, l);
+}
 
-// Row T of the chunk held by the lanes of this 16-lane row (T < 16 * NG).
-template <int T, int NG>
+// Row T of the chunk held by the NC lanes of this group (T < NC * NG).
+template <int NC, int T, int NG>
 __device__ inline double krow(const double (&v)[NG])
 {
-    return row_bcast<T & 15>(v[T >> 4]);
+    return group_bcast<NC, T % NC>(v[T / NC]);
 }
 
 template <int... I, class Fn>
@@ -998,22 +1031,27 @@ __device__ inline void kf_unroll(std::integer_sequence<int, I...>, Fn fn)
     (fn(std::integral_constant<int, I>{}), ...);
 }
 
-template <int MAXM>
+constexpr int KFB_COLS = 16;   // columns per workgroup in batches
+
+template <int MAXM, int NC>
 __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBlock& vb)
 {
     static_assert(MAXM <= 32, "fused k-solve: chunks of at most 32 rows");
     constexpr int MI = MAXM - 1;                  // interior rows of the longest chunk
-    constexpr int NG = (MI + 15) / 16;            // coefficient rows per lane
-    __shared__ double sY[3][64][KF_COLS + 1];
-    __shared__ double sX[64][KF_COLS + 1];
+    constexpr int NG = (MI + NC - 1) / NC;        // coefficient rows per lane
+    __shared__ double sY[3][64][NC + 1];
+    __shared__ double sX[64][NC + 1];
+    // short chunks leave registers for loading more up front: the separator
+    // system's factors, and the rows of q
+    constexpr bool EARLY = MAXM <= 16, EARLYQ = MAXM <= 8;
     const DevScalars* S = F.S;
-    if (S->err) return;
+    const bool err = S->err;
     const int f = vb.z;
     const KSys& K = F.ks[f];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int jl = lane & (KF_COLS - 1), p = 4 * wave + (lane >> 4);
+    const int jl = t % NC, p = t / NC;
     const int nch = K.nch;
-    const int j = vb.x * KF_COLS + jl + 1;
+    const int j = vb.x * NC + jl + 1;
     const bool act = j <= F.n2m;
     const int jc = act ? j : F.n2m;
     // byte offsets of a field fit in 31 bits (the launcher checks), so every
@@ -1022,7 +1060,7 @@ __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBloc
     const int col = ((jc - 1) + (K.kofs + 2) * F.P) * 8;  // row 0 of this column's line
     const bool own = p < nch;
     const int pc = own ? p : nch - 1;             // idle rows of lanes work on the last chunk, store nothing
-    const int s = K.cs[pc], e = K.cs[pc + 1] - 1, m = e - s;
+    const int s = chunk_start(pc, K.n, nch), e = chunk_start(pc + 1, K.n, nch) - 1, m = e - s;
     const __amdgpu_buffer_rsrc_t src = kf_rsrc(f == 0 ? F.sA : F.sB);
     // row tt of the chunk: lane offset of row s plus the uniform tt * P8
     const int v0 = col + s * P8;
@@ -1030,11 +1068,11 @@ __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBloc
 #pragma unroll
     for (int tt = 0; tt < MI; ++tt) y[tt] = tt < m ? kf_load(src, v0, tt * P8) : 0.0;
     const double dsep = kf_load(src, col + e * P8);
-    // coefficient rows of the chunk: lane u of the row holds rows u + 16 g
+    // coefficient rows of the chunk: lane u of the group holds rows u + NC g
     double cS[NG], ca[NG], ci[NG], cg[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-        const int r = s + min(jl + 16 * g, m > 0 ? m - 1 : 0);
+        const int r = s + min(jl + NC * g, m > 0 ? m - 1 : 0);
         cS[g] = K.S[r];
         ca[g] = K.a[r];
         ci[g] = K.inv[r];
@@ -1043,13 +1081,47 @@ __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBloc
     const double Se = K.S[e];
     double b0, bn;
     kbound(F, K, f, jc, S, b0, bn);
+    const __amdgpu_buffer_rsrc_t q = kf_rsrc(f == 0 ? F.q2 : F.q3);
+    // rows past the chunks of q3's line: its first and last node
+    double qlo = 0.0, qhi = 0.0, blo = 0.0, bhi = 0.0;
+    double sa, sc, sk1[6], sk2[6], sib, swl, qv0[MI];
+    // line-invariant factors of this wave's separator system, lane = chunk
+    auto load_sep = [&]() __attribute__((always_inline)) {
+        const int eq = chunk_start(min(lane, nch - 1) + 1, K.n, nch) - 1;
+        sa = K.a[eq];
+        sc = K.c[eq];
+#pragma unroll
+        for (int li = 0; li < 6; ++li) {
+            sk1[li] = K.k1[li * 64 + lane];
+            sk2[li] = K.k2[li * 64 + lane];
+        }
+        sib = K.ib[lane];
+        swl = K.wl[pc];
+    };
+    auto load_ends = [&]() __attribute__((always_inline)) {
+        if (f == 1 && p == 0) {
+            qlo = F.q3[fidx(F, jc, 1)];
+            blo = F.dqb3s[jc];
+        }
+        if (f == 1 && p == nch - 1) {
+            qhi = F.q3[fidx(F, jc, F.n3)];
+            bhi = F.dqb3n[jc];
+        }
+    };
+    if (EARLY) {
+        load_ends();
+        load_sep();
+    }
+#pragma unroll
+    for (int tt = 0; tt < MI; ++tt)
+        if (EARLYQ) qv0[tt] = tt < m ? kf_load(q, v0, tt * P8) : 0.0;
     double yp = 0.0, acc = 0.0;
     kf_unroll(std::make_integer_sequence<int, MI>{}, [&](auto ic) {
         constexpr int tt = decltype(ic)::value;
         // one step at a time: hoisted, the broadcasts of all steps would be
         // live at once and spill
         __builtin_amdgcn_sched_barrier(0);
-        const double rS = krow<tt>(cS), ra = krow<tt>(ca), ri = krow<tt>(ci), rg = krow<tt>(cg);
+        const double rS = krow<NC, tt>(cS), ra = krow<NC, tt>(ca), ri = krow<NC, tt>(ci), rg = krow<NC, tt>(cg);
         if (tt < m) {
             const int i = s + tt;
             double d = y[tt] * rS;
@@ -1069,52 +1141,53 @@ __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBloc
     }
     // back-substitution rows and the separator row of q, loaded while the
     // separator systems are solved
-    const __amdgpu_buffer_rsrc_t q = kf_rsrc(f == 0 ? F.q2 : F.q3);
     const double qe = kf_load(q, col + e * P8);
     double cv[NG], cc[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-        const int r = s + min(jl + 16 * g, m > 0 ? m - 1 : 0);
+        const int r = s + min(jl + NC * g, m > 0 ? m - 1 : 0);
         cv[g] = K.vp[r];
         cc[g] = K.cp[r];
     }
-    __syncthreads();
+    if (!EARLY) load_sep();
+    lds_barrier();
     {
         // separator system of column wave (k_ksolve2's operations); lane = chunk
         const int c = wave, q = lane;
         double delta = 0.0;
         if (q < nch) {
-            const int eq = K.cs[q + 1] - 1;
             const double ysn = (q + 1 < nch) ? sY[0][q + 1][c] : 0.0;
-            delta = sY[2][q][c] - K.a[eq] * sY[1][q][c] - K.c[eq] * ysn;
+            delta = sY[2][q][c] - sa * sY[1][q][c] - sc * ysn;
         }
-        int li = 0;
-        for (int h = 1; h < 64; h <<= 1, ++li) {
+#pragma unroll
+        for (int li = 0; li < 6; ++li) {
+            const int h = 1 << li;
             double dm = __shfl_up(delta, h, 64), dp = __shfl_down(delta, h, 64);
             if (q - h < 0) dm = 0.0;
             if (q + h >= 64) dp = 0.0;
-            delta = delta - K.k1[li * 64 + q] * dm - K.k2[li * 64 + q] * dp;
+            delta = delta - sk1[li] * dm - sk2[li] * dp;
         }
-        if (q < nch) sX[q][c] = delta * K.ib[q];
+        if (q < nch) sX[q][c] = delta * sib;
     }
-    __syncthreads();
+    lds_barrier();
     const double X = sX[pc][jl];
     const double Xm = (pc > 0) ? sX[pc - 1][jl] : 0.0;
-    const double wlp = K.wl[pc];
-    const bool st = own && act;
+    const double wlp = swl;
+    const bool st = own && act && !err;
     const bool zero_row = (f == 0 && j == 1);
     // back-substitution into y (x of every interior row, no memory traffic)
     double x = 0.0;
     kf_unroll(std::make_integer_sequence<int, MI>{}, [&](auto ic) {
         constexpr int tt = MI - 1 - decltype(ic)::value;
         __builtin_amdgcn_sched_barrier(0);
-        const double rv = krow<tt>(cv), rc = krow<tt>(cc);
+        const double rv = krow<NC, tt>(cv), rc = krow<NC, tt>(cc);
         if (tt < m) {
             if (tt == m - 1) x = y[tt] + rv * Xm + wlp * X;
             else x = (y[tt] + rv * Xm) - rc * x;
             y[tt] = x;
         }
     });
+    if (!EARLY) load_ends();
     // q += x, rows in batches whose loads are issued together (the stores of
     // a batch precede the next batch's loads, which the compiler keeps in
     // order since both address the same field)
@@ -1126,7 +1199,7 @@ __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBloc
 #pragma unroll
         for (int u = 0; u < QB; ++u) {
             const int tt = b + u;
-            if (tt < MI) qv[u] = tt < m ? kf_load(q, v0, tt * P8) : 0.0;
+            if (tt < MI) qv[u] = EARLYQ ? qv0[tt] : tt < m ? kf_load(q, v0, tt * P8) : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < QB; ++u) {
@@ -1140,28 +1213,24 @@ __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBloc
     kf_store(q, col + e * P8, zero_row ? 0.0 : qe + X);
     if (zero_row) kf_store(q, coln + e * P8, 0.0);
     if (f == 1) {
-        double* qf = F.q3;
-        if (p == 0) {
-            const size_t c0 = fidx(F, j, 1);
-            qf[c0] = qf[c0] + F.dqb3s[j];
-        }
-        if (p == nch - 1) {
-            const size_t c1 = fidx(F, j, F.n3);
-            qf[c1] = qf[c1] + F.dqb3n[j];
-        }
+        if (p == 0) F.q3[fidx(F, j, 1)] = qlo + blo;
+        if (p == nch - 1) F.q3[fidx(F, j, F.n3)] = qhi + bhi;
     }
 }
-template <int MAXM>
-__global__ __launch_bounds__(1024) void k_ksolve_fused(const FluidDev F)
+template <int MAXM, int NC>
+__global__ __launch_bounds__(64 * NC) void k_ksolve_fused(const FluidDev F)
 {
-    ksolve_fused_body<MAXM>(F, vb_hw());
+    VBlock vb = vb_hw();
+    // neighbouring groups of columns share their cache lines: one XCD gets them
+    vb.x = (vb.x & 7) * (vb.gx >> 3) + (vb.x >> 3);
+    if (vb.x * NC < F.n2m) ksolve_fused_body<MAXM, NC>(F, vb);
 }
 template <int MAXM>
-__global__ __launch_bounds__(1024) void kb_ksolve_fused(const BGrid<FluidDev> G)
+__global__ __launch_bounds__(64 * KFB_COLS) void kb_ksolve_fused(const BGrid<FluidDev> G)
 {
     VBlock vb;
     const FluidDev* Fp = bg_block(G, vb);
-    ksolve_fused_body<MAXM>(*Fp, vb);
+    ksolve_fused_body<MAXM, KFB_COLS>(*Fp, vb);
 }
 
 // Largest chunk (rows incl. the separator) of either k-system.
@@ -1172,15 +1241,32 @@ bool ksolve_fused_fits(const FluidDev& F)
     return kmaxm(F) <= 32 && (long)F.P * F.nk * 8 < (1L << 31);
 }
 
+// Columns per workgroup of the single instance.  One CU's loads go through
+// one address unit, so a grid of few columns is fastest spread over more
+// workgroups of fewer columns, until every CU has one; more columns read
+// longer runs of every row.  Four / eight / sixteen columns, us: 64x48 5.6 /
+// 6.6 / 8.0, 384x288 6.4 / 7.5 / 9.4, 1000x400 9.6 / 8.7 / 11.9, 480x600 10.0
+// / 8.8 / 12.0, 810x672 13.5 / 12.6 / 15.3, 1301x977 22.8 / 20.3 / 22.8;
+// chunks of up to 32 rows (eight columns take 142 registers, so a CU holds
+// one workgroup of them where it holds one of sixteen): 256x1500 23.0 / 19.2
+// / 23.0, 700x1500 23.8 / 20.6 / 23.9, 1200x1500 25.6 / 37.6 / 25.4.
+static constexpr int kKf4 = 512, kKf8Long = 1024;
+
+template <int MAXM, int NC>
+static void launch_kf(const FluidDev& F, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_ksolve_fused<MAXM, NC>), dim3(((F.n2m + NC - 1) / NC + 7) / 8 * 8, 1, 2), dim3(64 * NC), 0,
+                       st, F);
+}
+
 void launch_ksolve(const FluidDev& F, hipStream_t st)
 {
     int nchmax = F.ks[0].nch > F.ks[1].nch ? F.ks[0].nch : F.ks[1].nch;
     int maxm = kmaxm(F);
     if (F.kform && ksolve_fused_fits(F)) {
-        const dim3 gf((F.n2m + KF_COLS - 1) / KF_COLS, 1, 2);
-        if (maxm <= 8) hipLaunchKernelGGL(k_ksolve_fused<8>, gf, dim3(1024), 0, st, F);
-        else if (maxm <= 16) hipLaunchKernelGGL(k_ksolve_fused<16>, gf, dim3(1024), 0, st, F);
-        else hipLaunchKernelGGL(k_ksolve_fused<32>, gf, dim3(1024), 0, st, F);
+        if (maxm <= 8) F.n2m <= kKf4 ? launch_kf<8, 4>(F, st) : launch_kf<8, 8>(F, st);
+        else if (maxm <= 16) launch_kf<16, 8>(F, st);
+        else F.n2m <= kKf8Long ? launch_kf<32, 8>(F, st) : launch_kf<32, 16>(F, st);
         return;
     }
     dim3 g((F.n2m + 63) / 64, nchmax, 2);
@@ -1207,10 +1293,10 @@ void launch_ksolve_b(BatchSet& B, hipStream_t st)
         fused = fused && F.kform && ksolve_fused_fits(F);
     }
     if (fused) {
-        const auto gf = bdims(B, [](const FluidDev& F) { return dim3((F.n2m + KF_COLS - 1) / KF_COLS, 1, 2); });
-        if (maxm <= 8) blaunch(B, BK_KF, gf, kb_ksolve_fused<8>, dim3(1024), 0, st);
-        else if (maxm <= 16) blaunch(B, BK_KF, gf, kb_ksolve_fused<16>, dim3(1024), 0, st);
-        else blaunch(B, BK_KF, gf, kb_ksolve_fused<32>, dim3(1024), 0, st);
+        const auto gf = bdims(B, [](const FluidDev& F) { return dim3((F.n2m + KFB_COLS - 1) / KFB_COLS, 1, 2); });
+        if (maxm <= 8) blaunch(B, BK_KF, gf, kb_ksolve_fused<8>, dim3(64 * KFB_COLS), 0, st);
+        else if (maxm <= 16) blaunch(B, BK_KF, gf, kb_ksolve_fused<16>, dim3(64 * KFB_COLS), 0, st);
+        else blaunch(B, BK_KF, gf, kb_ksolve_fused<32>, dim3(64 * KFB_COLS), 0, st);
         return;
     }
     const auto g = bdims(B, [](const FluidDev& F) {

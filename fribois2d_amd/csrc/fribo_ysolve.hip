@@ -236,13 +236,13 @@ __device__ __forceinline__ void ysolve_fused_body(const FluidDev& F, const VBloc
     extern __shared__ double dyn[];
     __shared__ double sY[6][64][NM + 1];
     __shared__ double sX[64][NM + 1];
-    if (F.S->err) return;
+    const bool err = F.S->err;
     const KSys& K = F.ks[0];
     const int t = threadIdx.x, jl = t % NM, p = t / NM, nch = K.nch, n = F.n3m;
     const int j = vb.x * NM + jl + 1;
-    const bool own = p < nch, st = own && j <= F.n2m;
+    const bool own = p < nch, st = own && j <= F.n2m && !err;
     const int jc = min(j, F.n2m), pc = own ? p : nch - 1;
-    const int s = K.cs[pc], e = K.cs[pc + 1] - 1, m = e - s;
+    const int s = chunk_start(pc, n, nch), e = chunk_start(pc + 1, n, nch) - 1, m = e - s;
     const int P8 = F.P * 8, v0 = (jc - 1) * 8 + s * P8;
     const __amdgpu_buffer_rsrc_t hm = kf_rsrc(F.hmn);
     double y[MI];
@@ -298,7 +298,7 @@ __device__ __forceinline__ void ysolve_fused_body(const FluidDev& F, const VBloc
             beta = sY[1][q][c];
             delta = sY[2][q][c];
             if (q + 1 < nch) {
-                const int eq = K.cs[q + 1] - 1;
+                const int eq = chunk_start(q + 1, n, nch) - 1;
                 const double ce = lc[eq + (eq >> 5)];
                 beta = beta + ce * sY[4][q + 1][c];
                 gamma = ce * sY[5][q + 1][c];
