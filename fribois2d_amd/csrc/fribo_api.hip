@@ -77,8 +77,10 @@ struct fribo_ctx {
     // one (it reads only q2/q3, so it runs while the host prepares the next
     // step); cleared by anything that changes the velocities in between
     bool cfl_ready = false;
-    // captured step (hipGraph): rebuilt when the marker buffers change
-    bool use_graph = false;
+    // captured step (hipGraph): rebuilt when the marker buffers change.  1 / 0 as
+    // the caller set it, -1 by auto_graph
+    int use_graph = -1;
+    int plain_steps = 0;         // steps by launches since the marker buffers were made
     bool yavail = false;     // transform along y set up
     double dmin = 0.0;       // smallest node spacing of the grid (cordin.F90:217-231)
     double* dpart = nullptr; // device: diagnostics partials [8][256]
@@ -729,6 +731,7 @@ extern "C" int fribo_set_markers(fribo_handle h, int32_t nlm, const double* lmcc
             h->gexec = nullptr;
         }
         h->graph_nlm = -1;
+        h->plain_steps = 0;
         ++h->mk_gen;
         for (void* q : h->mk_allocs) hipFree(q);
         h->mk_allocs.clear();
@@ -1006,6 +1009,19 @@ static void enqueue_step(fribo_ctx* c, bool cfl)
     for (int n = 1; n <= c->F.nsst; ++n) enqueue_substep(c, n, n > 1, n == c->F.nsst);
 }
 
+// Whether the step is replayed as a graph where the caller has not said:
+// grids whose kernels are as short as their launches, from the third step
+// with the same marker buffers on, so that a few steps, or marker counts that
+// keep changing, do not pay for captures.  ms per run with launches / graph:
+// 64x48 4.06 / 3.82, coupled 384x288 9.1 / 8.2, strongly coupled 512x384 10.5 /
+// 9.5, 480x600 20.9 / 20.7, 810x672 45.5 / 46.2.
+static constexpr long kGraphCells = 300000;
+
+static bool auto_graph(const fribo_ctx* c)
+{
+    return (long)c->F.n2m * c->F.n3m <= kGraphCells && c->F.refine < 0 && c->plain_steps >= 2;
+}
+
 // Capture the whole step once; every kernel reads its per-step inputs from
 // device memory, so the same graph replays for every step.
 static int ensure_graph(fribo_ctx* c)
@@ -1015,13 +1031,23 @@ static int ensure_graph(fribo_ctx* c)
         hipGraphExecDestroy(c->gexec);
         c->gexec = nullptr;
     }
+    // captured on a stream of its own that the null stream does not wait for: a
+    // launch on the null stream by another thread would break off the capture
+    // of an ordinary stream
     hipGraph_t g = nullptr;
+    hipStream_t cap = nullptr, st = c->st;
+    HIPCHK(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
     const bool prof = c->profiling;
-    c->profiling = false;
-    HIPCHK(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-    enqueue_step(c, false);
-    hipError_t e = hipStreamEndCapture(c->st, &g);
-    c->profiling = prof;
+    hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
+    if (e == hipSuccess) {
+        c->profiling = false;
+        c->st = cap;
+        enqueue_step(c, false);
+        c->st = st;
+        c->profiling = prof;
+        e = hipStreamEndCapture(cap, &g);
+    }
+    hipStreamDestroy(cap);
     if (e != hipSuccess) return set_err(FRIBO_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
     e = hipGraphInstantiate(&c->gexec, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
@@ -1055,12 +1081,19 @@ extern "C" int fribo_fluid_tsch(fribo_handle h, int32_t ns, double* dt, double d
     if ((e = write_inputs(h, ns, *dt, dt_o))) return e;
     const bool cfl = !h->cfl_ready;
     h->cfl_ready = false;
-    if (h->use_graph && !h->profiling) {
-        if ((e = ensure_graph(h))) return e;
+    bool graph = !h->profiling && (h->use_graph > 0 || (h->use_graph < 0 && auto_graph(h)));
+    if (graph && (e = ensure_graph(h))) {
+        if (h->use_graph > 0) return e;
+        hipGetLastError();   // by launches instead, from here on
+        h->use_graph = 0;
+        graph = false;
+    }
+    if (graph) {
         if (cfl) enqueue_cfl(h);
         HIPCHK(hipGraphLaunch(h->gexec, h->st));
     } else {
         enqueue_step(h, cfl);
+        h->plain_steps = std::min(h->plain_steps + 1, 2);
     }
     // with per-class profiling the next step's k_cfl stays in that step
     return finish(h, dt, cflm, !h->profiling);
@@ -1069,7 +1102,7 @@ extern "C" int fribo_fluid_tsch(fribo_handle h, int32_t ns, double* dt, double d
 extern "C" int fribo_set_graph(fribo_handle h, int32_t on)
 {
     if (!h) return set_err(FRIBO_ERR_ARG, "null handle");
-    h->use_graph = on != 0;
+    h->use_graph = on != 0 ? 1 : 0;
     return FRIBO_OK;
 }
 

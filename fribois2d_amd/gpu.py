@@ -334,7 +334,8 @@ class FluidStep:
         return load().fribo_get_precision(self.h)
 
     def set_graph(self, on=True):
-        """Replay the step as one captured HIP graph (same results)."""
+        """Replay the step as one captured HIP graph (same results); off:
+        launch its kernels.  Without a call the library chooses by the grid."""
         _check(load().fribo_set_graph(self.h, 1 if on else 0))
 
     # -- profiling ----------------------------------------------------------

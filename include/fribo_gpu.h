@@ -180,7 +180,9 @@ int fribo_checkbcs(fribo_handle h, double* bcerrv, double* bcerrw, double* nbcv,
 /* Execution option (no reference counterpart): with on != 0 the step's
  * kernels are captured once into a HIP graph and replayed by every
  * fribo_fluid_tsch call (re-captured when the marker count changes);
- * results are identical to the default stream launches. */
+ * results are identical to stream launches, which on == 0 selects.  Without
+ * a call the library replays a graph on small grids, from the third step
+ * with the same marker count on. */
 int fribo_set_graph(fribo_handle h, int32_t on);
 const char* fribo_last_error(void);
 
