@@ -308,16 +308,19 @@ __device__ inline void wait_vm()
 // in every lane).  Issued as inline assembly, the compiler does not track the
 // LDS write, so it adds no wait for it before later LDS reads of other
 // stages; the kernel's own vmcnt wait and barrier order every read after the
-// loads of its slice.
+// loads of its slice.  The compiler adds no wait states inside it either: a
+// load into LDS reads M0 one wait state after a scalar write at the earliest
+// (s_nop), else it may use the address before.
 __device__ inline void dma16(const double* base, unsigned off, unsigned lds)
 {
     const unsigned long long b = (unsigned long long)base;
     const unsigned long long sb =
         ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(b >> 32)) << 32) |
         (unsigned)__builtin_amdgcn_readfirstlane((unsigned)b);
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
+                     __builtin_amdgcn_readfirstlane(lds)),
                  "v"(off), "s"(sb)
-                 : "memory");
+                 : "memory", "m0");
 }
 
 template <int BK, bool NN, int WM = 2, int WN = 8, int BN = 128, int BM = 96>
