@@ -557,28 +557,41 @@ __global__ __launch_bounds__(64 * JW) void kb_jsolve_p(const BGrid<FluidDev> G)
     jsolve_p_body<MAXR, JW>(*Fp, vb);
 }
 
-static constexpr int kJh4Lines = 1536;
+// Workgroups of the Helmholtz j-lines of a grid of n3m planes: as many for
+// each of the two fields, `per` lines each at a time (at most `most` in all).
+// Rounded up: one workgroup too few sends all of them round again for the
+// last lines (two fields of 810 lines in eight waves, 672 rows: 14.6 us with
+// 101 workgroups each, 11.5 with 102).
+static int jh_groups(int n3m, int per, int most) { return 2 * std::max(1, std::min(most / 2, (n3m + per - 1) / per)); }
+
+// Four waves per workgroup up to 512 planes, where 128 such workgroups for
+// each field, one per CU, take every line at once: fewer lines per CU share
+// its LDS and address unit.  With more planes they would go round again, and
+// eight waves, one round up to 1024 planes, share one staging of the factors.
+// Four / eight waves, us, by planes:
+//   rows         300          512          513          810          1024
+//    288   6.5 /  7.6   6.8 /  7.7   8.2 /  7.7   8.5 /  8.0   8.5 /  8.2
+//    672   9.1 / 11.4   9.4 / 11.3  13.0 / 12.4  13.0 / 12.8  13.9 / 13.1
+//    977   9.6 / 12.2  10.5 / 12.8  13.8 / 12.1  13.4 / 12.1  13.6 / 12.7
+//   1300  13.5 / 14.6  14.1 / 15.2  16.8 / 15.4  17.5 / 15.9  18.0 / 16.9
+// and within 3% of each other at 1025 to 1536, eight 10-15% ahead from there.
+static constexpr int kJh4Planes = 512;
 
 template <int MAXR>
 static void launch_h(const FluidDev& F, hipStream_t st)
 {
-    const int lines = 2 * F.n3m - 1;
     const int sd = F.jstride;
-    // Few lines are spread over more workgroups of four waves; many share one
-    // staging of the factors among eight.  Eight / four waves, us: 64x48 8.0 /
-    // 6.8, 384x288 8.2 / 6.7, 480x600 11.4 / 9.6, 810x672 14.8 / 12.6, 1301x977
-    // 16.8 / 16.6, 2048x1536 24.5 / 29.8.
-    if (lines > kJh4Lines && jsolve_h_lds_bytes(MAXR, 8, sd, true) <= (size_t)F.lds_max) {
-        const int g = std::max(2, std::min(256, (lines + 7) / 8) & ~1);
+    if (F.n3m > kJh4Planes && jsolve_h_lds_bytes(MAXR, 8, sd, true) <= (size_t)F.lds_max) {
+        const int g = jh_groups(F.n3m, 8, 256);
         hipLaunchKernelGGL((k_jsolve_hp<MAXR, 8>), dim3(g), dim3(512), jsolve_h_lds_bytes(MAXR, 8, sd, true), st, F);
     } else if (jsolve_h_lds_bytes(MAXR, 4, sd, true) <= (size_t)F.lds_max) {
-        const int g = std::max(2, std::min(256, (lines + 3) / 4) & ~1);
+        const int g = jh_groups(F.n3m, 4, 256);
         hipLaunchKernelGGL((k_jsolve_hp<MAXR, 4>), dim3(g), dim3(256), jsolve_h_lds_bytes(MAXR, 4, sd, true), st, F);
     } else if (jsolve_h_lds_bytes(MAXR, 2, sd, true) <= (size_t)F.lds_max) {
-        const int g = std::max(2, std::min(512, (lines + 1) / 2) & ~1);
+        const int g = jh_groups(F.n3m, 2, 512);
         hipLaunchKernelGGL((k_jsolve_hp<MAXR, 2>), dim3(g), dim3(128), jsolve_h_lds_bytes(MAXR, 2, sd, true), st, F);
     } else {
-        const int g = std::max(2, std::min(2048, lines) & ~1);
+        const int g = jh_groups(F.n3m, 1, 2048);
         hipLaunchKernelGGL((k_jsolve_h<MAXR>), dim3(g), dim3(64), jsolve_h_lds_bytes(MAXR, 1, sd, false), st, F);
     }
 }

@@ -1,0 +1,43 @@
+"""Line solves where their launch rules change, and one line or column to the
+other side.
+
+The Helmholtz j-lines take four waves per workgroup up to 512 planes and eight
+above, in as many workgroups as take every line at once (up to 1024 planes); a
+batch takes eight and as many lines per wave as keep its workgroups resident.
+Every line is solved by one wave with the same operations whatever the shape,
+so an instance alone and the same instance in a batch (on the transform tiles
+of the instance alone) give the same bits."""
+import numpy as np
+import pytest
+
+from fribois2d_amd import cases
+from helpers import gpu_for
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(n2m, n3m):
+    h = 0.02
+    rc, zz = np.linspace(0.0, n2m * h, n2m + 1), np.linspace(0.0, n3m * h, n3m + 1)
+    p = cases.FluidParams(n2=n2m + 1, n3=n3m + 1, alx3=n3m * h, rext2=n2m * h, visc=0.01, dt0=1.0e-4, ibact=False)
+    return cases.Case(f"rules{n2m}x{n3m}", p, rc, zz, None, (0.5 * n2m * h, 0.5 * n3m * h), None, 20261205)
+
+
+# 512 | 513 planes: four | eight waves; 1024 | 1025: one | two rounds of them;
+# 17, 49: one line more than whole workgroups hold
+@pytest.mark.parametrize("n2m,n3m", [(20, 17), (20, 49), (30, 512), (30, 513), (30, 1024), (30, 1025)])
+def test_j_lines_where_the_rule_changes(n2m, n3m):
+    from fribois2d_amd.gpu import FluidBatch
+    c = _case(n2m, n3m)
+    alone, member, other = gpu_for(c), gpu_for(c), gpu_for(_case(24, 40))
+    b = FluidBatch([member, other])
+    b.set_gemm_shape(0)
+    dt = np.full(2, c.params.dt0)
+    for ns in range(2):
+        dta, _ = alone.fluid_tsch(ns, dt[0], dt[0])
+        dt = b.step(ns, dt)[0]
+        assert dt[0] == dta
+    sa, sm = alone.get_state(), member.get_state()
+    for f in sa:
+        assert np.isfinite(sa[f]).all() and np.array_equal(sa[f], sm[f]), f
+    b.close()
