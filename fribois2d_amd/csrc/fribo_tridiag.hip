@@ -1259,10 +1259,14 @@ bool ksolve_fused_fits(const FluidDev& F)
 // workgroups of fewer columns, until every CU has one; more columns read
 // longer runs of every row.  Four / eight / sixteen columns, us: 64x48 5.6 /
 // 6.6 / 8.0, 384x288 6.4 / 7.5 / 9.4, 1000x400 9.6 / 8.7 / 11.9, 480x600 10.0
-// / 8.8 / 12.0, 810x672 13.5 / 12.6 / 15.3, 1301x977 22.8 / 20.3 / 22.8;
-// chunks of up to 32 rows (eight columns take 142 registers, so a CU holds
-// one workgroup of them where it holds one of sixteen): 256x1500 23.0 / 19.2
-// / 23.0, 700x1500 23.8 / 20.6 / 23.9, 1200x1500 25.6 / 37.6 / 25.4.
+// / 8.8 / 12.0, 810x672 13.5 / 12.6 / 15.3, 1301x977 22.8 / 20.3 / 22.8.
+// With chunks of more than 8 rows a CU holds one workgroup of eight columns at
+// a time (their loads up front and the rows in registers), so past 1024
+// columns, where there are more of them than CUs, sixteen are faster.  Eight /
+// sixteen: 600x1024 12.3 / 13.8, 600x1025 15.5 / 14.3, 900x1100 17.9 / 16.9,
+// 1000x1300 19.5 / 18.7; chunks of up to 32 rows 256x1500 19.2 / 23.0,
+// 700x1500 20.6 / 23.9, 1200x1500 37.6 / 25.4.  With chunks of up to 8 rows
+// both take the same there (400x1300 11.2 / 12.0, 400x2040 12.2 / 12.1).
 static constexpr int kKf4 = 512, kKf8Long = 1024;
 
 template <int MAXM, int NC>
@@ -1278,7 +1282,7 @@ void launch_ksolve(const FluidDev& F, hipStream_t st)
     int maxm = kmaxm(F);
     if (F.kform && ksolve_fused_fits(F)) {
         if (maxm <= 8) F.n2m <= kKf4 ? launch_kf<8, 4>(F, st) : launch_kf<8, 8>(F, st);
-        else if (maxm <= 16) launch_kf<16, 8>(F, st);
+        else if (maxm <= 16) F.n2m <= kKf8Long ? launch_kf<16, 8>(F, st) : launch_kf<16, 16>(F, st);
         else F.n2m <= kKf8Long ? launch_kf<32, 8>(F, st) : launch_kf<32, 16>(F, st);
         return;
     }

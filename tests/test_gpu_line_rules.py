@@ -6,7 +6,11 @@ above, in as many workgroups as take every line at once (up to 1024 planes); a
 batch takes eight and as many lines per wave as keep its workgroups resident.
 Every line is solved by one wave with the same operations whatever the shape,
 so an instance alone and the same instance in a batch (on the transform tiles
-of the instance alone) give the same bits."""
+of the instance alone) give the same bits.
+
+The one-pass k-lines with chunks of 9 to 16 rows own eight columns per
+workgroup up to 1024 columns and sixteen above; every form does the operations
+of the three passes in the same order."""
 import numpy as np
 import pytest
 
@@ -41,3 +45,18 @@ def test_j_lines_where_the_rule_changes(n2m, n3m):
     for f in sa:
         assert np.isfinite(sa[f]).all() and np.array_equal(sa[f], sm[f]), f
     b.close()
+
+
+@pytest.mark.parametrize("n2m,n3m", [(1024, 513), (1025, 513), (1040, 1024), (1041, 600)])
+def test_k_lines_where_the_rule_changes(n2m, n3m):
+    st = []
+    for form in ("fused", "3pass"):
+        g = gpu_for(_case(n2m, n3m))
+        g.set_ksolve(form)
+        dt = g.params.dt0
+        for ns in range(2):
+            dt, _ = g.fluid_tsch(ns, dt, dt)
+        st.append(g.get_state())
+        g.close()
+    for f in st[0]:
+        assert np.isfinite(st[0][f]).all() and np.array_equal(st[0][f], st[1][f]), f
