@@ -561,13 +561,14 @@ static void launch_timed(Kern kern, dim3 g, dim3 b, hipStream_t st, hipEvent_t e
 // is one 16x16 block per SIMD over all of K: a workgroup of 4 waves with one
 // block each (32x32) costs 1, one of 32x64 costs 2, one of 96x128 costs 12,
 // and a CU works through ceil(workgroups / 256) of them.  Per unit the larger
-// tiles are the faster ones (fewer loads and barriers per block): measured
-// with 12 units each, 1536x2048x1536 in the mirror form takes 84.4 us in
-// 96x128 tiles, 89.8 in 32x64 and 97.6 in 32x32, hence the weights 1, 0.94
-// and 0.87; but smaller tiles round up less (977x1301x977: 56.0 us with 5
-// units of 32x32, 62.1 with 6 of 32x64, 105 with 12 of 96x128).  With fewer
-// than 4 units the time is latency and the shorter tiles win ties (600x480
-// NT: 13.3 against 14.0 us).
+// tiles are the faster ones (fewer loads and barriers per block): against
+// 96x128, 32x64 tiles take 1.08 to 1.16 times as long a unit (3500x4000x3500
+// NN 2053 us for 56 units, 1945 for 60; 2500^3 NT 648 for 26, 794 for 36;
+// 1700^3 NT 212 and 192 for 12) and 32x32 tiles 1.20 to 1.28 times (1700x1500
+// x1500 NT 177 for 10, 167 for 12), hence 1.11 and 1.22; but smaller tiles
+// round up less (977x1301x977: 63 us with 5 units of 32x32, 71 with 6 of
+// 32x64, 106 with 12 of 96x128).  With fewer than 4 units the time is latency
+// and the shorter tiles win ties (600x480 NT: 13.3 against 14.0 us).
 enum { TILE_32x32, TILE_32x64, TILE_96x128 };
 static int gemm_tile(int M, int N, int ks)
 {
@@ -575,7 +576,7 @@ static int gemm_tile(int M, int N, int ks)
     const long u32 = rounds((long)tiles_m(M, ks, 32) * cdiv(N, 32));
     const long u64 = 2 * rounds((long)tiles_m(M, ks, 32) * cdiv(N, 64));
     const long u96 = 12 * rounds((long)tiles_m(M, ks, 96) * cdiv(N, 128));
-    if (100 * u96 <= 106 * u64 && 100 * u96 <= 115 * u32) return TILE_96x128;
+    if (100 * u96 <= 111 * u64 && 100 * u96 <= 122 * u32) return TILE_96x128;
     return u32 >= 4 && 100 * u64 <= 108 * u32 ? TILE_32x64 : TILE_32x32;
 }
 
