@@ -1054,9 +1054,11 @@ __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBloc
     constexpr int NG = (MI + NC - 1) / NC;        // coefficient rows per lane
     __shared__ double sY[3][64][NC + 1];
     __shared__ double sX[64][NC + 1];
-    // short chunks leave registers for loading more up front: the separator
-    // system's factors, and the rows of q
-    constexpr bool EARLY = MAXM <= 16, EARLYQ = MAXM <= 8;
+    // short chunks leave registers for loading more up front: the rows of q,
+    // and in narrow workgroups the separator system's factors (sixteen columns:
+    // 900x1080 17.1 us with, 16.2 without, 1000x1300 19.4 / 19.0; 24 instances
+    // 29.4 / 29.2)
+    constexpr bool EARLY = MAXM <= 16 && NC <= 8, EARLYQ = MAXM <= 8;
     const DevScalars* S = F.S;
     const bool err = S->err;
     const int f = vb.z;
@@ -1263,7 +1265,7 @@ bool ksolve_fused_fits(const FluidDev& F)
 // With chunks of more than 8 rows a CU holds one workgroup of eight columns at
 // a time (their loads up front and the rows in registers), so past 1024
 // columns, where there are more of them than CUs, sixteen are faster.  Eight /
-// sixteen: 600x1024 12.3 / 13.8, 600x1025 15.5 / 14.3, 900x1100 17.9 / 16.9,
+// sixteen: 600x1024 12.3 / 13.8, 600x1025 15.5 / 14.3, 900x1100 17.9 / 16.2,
 // 1000x1300 19.5 / 18.7; chunks of up to 32 rows 256x1500 19.2 / 23.0,
 // 700x1500 20.6 / 23.9, 1200x1500 37.6 / 25.4.  With chunks of up to 8 rows
 // both take the same there (400x1300 11.2 / 12.0, 400x2040 12.2 / 12.1).
