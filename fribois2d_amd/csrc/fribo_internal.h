@@ -204,6 +204,16 @@ __device__ inline void lds_barrier()
     raw_barrier();
 }
 
+// Orders a wave's own LDS accesses across its lanes (LDS executes a wave's
+// accesses in order): for LDS that is private to the wave, where a workgroup
+// barrier would also wait for the loads of the wave's next line or plane.
+__device__ inline void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Value of v in lane l of the wave (l wave-uniform): a matrix row that one
 // lane loaded and every lane of the wave uses, moved through scalar registers
 // instead of a scalar memory load per use.

@@ -98,17 +98,6 @@ __device__ inline void line_get(double* __restrict__ dst, const double* stage, c
         if (slot[u] >= 0) dst[lane + 64 * u] = stage[slot[u]];
 }
 
-// The staging rows of a j-line are private to its wave, so the line loop
-// only has to order the wave's own LDS accesses across its lanes (LDS
-// executes a wave's accesses in order).  A workgroup barrier here would also
-// wait for the next line's global loads, serialising load and solve.
-__device__ inline void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 size_t jsolve_h_lds_bytes(int maxr, int jw, int stride, bool fl)
 {
     const size_t nr = (size_t)maxr + 1;

@@ -60,3 +60,42 @@ def test_k_lines_where_the_rule_changes(n2m, n3m):
         g.close()
     for f in st[0]:
         assert np.isfinite(st[0][f]).all() and np.array_equal(st[0][f], st[1][f]), f
+
+
+def _alone_and_together(sizes, axis):
+    """Fields of the instances after two steps alone and after two steps as a
+    batch on 32x32 transform tiles."""
+    from fribois2d_amd.gpu import FluidBatch
+    cs = [_case(*s) for s in sizes]
+    gs, out = [gpu_for(c, axis=axis) for c in cs], []
+    b = FluidBatch(gs)
+    b.set_gemm_shape(0)
+    dt = np.array([c.params.dt0 for c in cs])
+    for ns in range(2):
+        dt, _, err = b.step(ns, dt)
+        assert not err.any()
+    together = [g.get_state() for g in gs]
+    b.close()
+    for i, c in enumerate(cs):
+        gs[i].close()
+        a, d = gpu_for(c, axis=axis), c.params.dt0
+        for ns in range(2):
+            d, _ = a.fluid_tsch(ns, d, d)
+        assert d == dt[i]
+        out.append((a.get_state(), together[i]))
+        a.close()
+    return out
+
+
+# Pressure partials of a batch's taller tiles (kb_upd): the large members make
+# the tiles eight planes tall, the others' partials cover 1, 2 and 4 of them,
+# the last tiles are cut short (z order: the first member has no y order);
+# then four planes with partials of one in the mirror form, 160 and 61 planes
+@pytest.mark.parametrize("sizes,axis", [
+    ([(70, 63), (620, 1100), (620, 1101), (311, 517), (311, 700), (64, 97)], "z"),
+    ([(126, 160)] * 26 + [(50, 61), (63, 97), (64, 130)], "y"),
+])
+def test_batch_pressure_partials_are_those_of_the_instances_alone(sizes, axis):
+    for i, (alone, together) in enumerate(_alone_and_together(sizes, axis)):
+        for f in alone:
+            assert np.isfinite(alone[f]).all() and np.array_equal(alone[f], together[f]), (sizes[i], f)
