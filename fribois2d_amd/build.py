@@ -23,7 +23,11 @@ SOURCES = ["fribo_api.hip", "fribo_stencil.hip", "fribo_tridiag.hip", "fribo_mls
            "fribo_eig.hip", "fribo_ysolve.hip", "fribo_mlp.hip", "fribo_xfer.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+# Host functions start on cache lines: the speed of the eigen-decomposition's
+# loops depends on where they lie in theirs (384 nodes: 18 or 29 ms with the same
+# code), and without this on the size of whatever is linked before them.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-shared", "-std=c++17", "-ffp-contract=off",
+         "-Xarch_host", "-falign-functions=64",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-result", "-I", os.path.join(ROOT, "include"), "-I", CSRC]
 
