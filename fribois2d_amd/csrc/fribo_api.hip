@@ -72,7 +72,7 @@ struct fribo_ctx {
     // the nine results of the diagnostics
     DevScalars* hsp = nullptr;
     hipEvent_t ev_rb = nullptr;  // the read-back copy of those scalars
-    XferRing xfer;               // staging ring of the state transfers
+    XferEvents xfer;             // of the state transfers
     // k_cfl of the next step already enqueued behind the read-back of this
     // one (it reads only q2/q3, so it runs while the host prepares the next
     // step); cleared by anything that changes the velocities in between
@@ -603,6 +603,7 @@ extern "C" int fribo_init(const fribo_params* p, const double* rc, const double*
             return set_err(FRIBO_ERR_HIP, hipGetErrorString(he));
         }
     }
+    xfer_attach();
     *out = c;
     return FRIBO_OK;
 }
@@ -624,6 +625,7 @@ extern "C" int fribo_finalize(fribo_handle h)
     for (void* q : h->allocs) hipFree(q);
     hipStreamDestroy(h->st);
     delete h;
+    xfer_detach();
     return FRIBO_OK;
 }
 
@@ -636,7 +638,7 @@ static XferSeg field_seg(const FluidDev& F, double* dev, const double* host, int
 
 static int xfer(fribo_ctx* c, XferSeg* segs, int nseg, bool put)
 {
-    const hipError_t he = xfer_run(c->xfer, c->F, segs, nseg, put, c->st);
+    const hipError_t he = xfer_run(c->xfer, c->dev, c->F, segs, nseg, put, c->st);
     return he == hipSuccess ? FRIBO_OK : set_err(FRIBO_ERR_HIP, std::string("state transfer: ") + hipGetErrorString(he));
 }
 
@@ -1807,7 +1809,7 @@ static int batch_refresh(fribo_batch_ctx* b)
 
 // The staging events of an instance whose stream is about to be destroyed:
 // their last records would be on that stream, so a fresh (unrecorded) marker
-// event takes the old one's place, and the transfer ring makes its own again.
+// event takes the old one's place, and the next transfer makes its own again.
 static void rearm_events(fribo_ctx* h)
 {
     xfer_free(h->xfer);

@@ -15,16 +15,19 @@ struct XferSeg {
     int n, pitch, rows, k0, pressure;
 };
 
-// Staging ring of one handle: pinned chunks and the events of their kernels.
-struct XferRing {
+// Events of one handle's transfers, one per chunk in flight.
+struct XferEvents {
     static constexpr int SLOTS = 3;
-    double* stage = nullptr;     // SLOTS chunks of `chunk` doubles
-    size_t chunk = 0;
     hipEvent_t ev[SLOTS] = {nullptr, nullptr, nullptr};
 };
 
 // Moves every segment (put: host to device, else device to host) on stream
-// st and returns when the host side is complete; a put may leave its last
-// kernels running (they read the ring, which the next transfer waits for).
-hipError_t xfer_run(XferRing& R, const FluidDev& F, XferSeg* segs, int nseg, bool put, hipStream_t st);
-void xfer_free(XferRing& R);
+// st of device dev and returns when it is complete on both sides.
+hipError_t xfer_run(XferEvents& R, int dev, const FluidDev& F, XferSeg* segs, int nseg, bool put, hipStream_t st);
+void xfer_free(XferEvents& R);
+
+// The pinned staging memory belongs to the library: a transfer takes a block
+// for as long as it runs.  Handles attach while they live; the last one to
+// detach gives the memory back.
+void xfer_attach();
+void xfer_detach();

@@ -6,10 +6,11 @@
 // length (2.6 ms for the state of a 64x48 grid, 84 ms at 2048x1536), so the
 // rows are packed by a kernel that writes pinned host memory directly, all
 // arrays of the call as one flat range cut into chunks of at most 4 MB.
-// Three chunks are in flight: while the kernels of the next two run, the host
-// copies the finished one out, with up to seven helper threads where there is
-// enough to copy (first writes to fresh pages cost a single thread several
-// times the PCIe time).  The pressure's pending means are subtracted by the
+// Where there are several, three chunks are in flight: while the kernels of
+// the next two run, the host copies the finished one out.  Up to seven helper
+// threads copy where there is enough to copy (first writes to fresh pages cost
+// a single thread several times the PCIe time).  A transfer of one chunk runs
+// its kernel, then its copy: 0.25 ms for a state of 2 MB.  The pressure's pending means are subtracted by the
 // kernel.  Uploads take the same way back.  The whole state's read-back:
 // 83.7 -> 5.8 ms at 2048x1536 (22 GB/s into fresh host pages), 13.6 -> 0.36
 // ms at 384x288, 2.6 -> 0.04 ms at 64x48.
@@ -154,21 +155,123 @@ private:
 };
 
 constexpr size_t kChunk = 512 * 1024;   // doubles: 4 MB
+constexpr int SLOTS = XferEvents::SLOTS;
+
+// Pinned staging blocks.  A transfer leases one and is complete when it gives
+// it back, so a block serves every handle, stream and thread in turn, and
+// there are as many as transfers run at once (each handle with a block of its
+// own kept up to 12 MB of locked memory, 3 GB with 256 of them, and allocated
+// it in its first transfer).  Sizes are powers of two of 1 MB up to the
+// largest a transfer can use, 12 MB; a block that is too small is replaced.
+// At most kIdle blocks wait for the next transfer.
+struct Block {
+    double* p = nullptr;
+    size_t n = 0;      // doubles
+    int dev = -1;
+};
+constexpr int kIdle = 8;
+std::mutex g_mu;
+Block g_idle[kIdle];
+size_t g_held = 0;     // doubles in idle and leased blocks
+int g_users = 0;
+
+hipError_t lease(int dev, size_t want, Block& b)
+{
+    size_t n = 128 * 1024;
+    while (n < want) n *= 2;
+    n = std::min<size_t>(n, SLOTS * kChunk);
+    Block old;
+    {
+        std::lock_guard<std::mutex> l(g_mu);
+        Block *fit = nullptr, *small = nullptr;
+        for (auto& q : g_idle) {
+            if (!q.p || q.dev != dev) continue;
+            if (q.n >= want) {
+                if (!fit || q.n < fit->n) fit = &q;
+            } else if (!small || q.n > small->n) {
+                small = &q;
+            }
+        }
+        if (fit) {
+            b = *fit;
+            *fit = Block();
+            return hipSuccess;
+        }
+        if (small) {
+            old = *small;
+            *small = Block();
+        }
+        g_held += n;
+        g_held -= old.n;
+    }
+    if (old.p) hipHostFree(old.p);
+    b.dev = dev;
+    b.n = n;
+    const hipError_t e = hipHostMalloc((void**)&b.p, n * sizeof(double), hipHostMallocDefault);
+    if (e != hipSuccess) {
+        b = Block();
+        std::lock_guard<std::mutex> l(g_mu);
+        g_held -= n;
+    }
+    return e;
+}
+
+void give(Block& b)
+{
+    if (!b.p) return;
+    {
+        std::lock_guard<std::mutex> l(g_mu);
+        if (g_users > 0)
+            for (auto& q : g_idle)
+                if (!q.p) {
+                    q = b;
+                    return;
+                }
+        g_held -= b.n;
+    }
+    hipHostFree(b.p);
+}
 
 }  // namespace
 
-void xfer_free(XferRing& R)
+void xfer_attach()
 {
-    if (R.stage) hipHostFree(R.stage);
-    R.stage = nullptr;
-    R.chunk = 0;
+    std::lock_guard<std::mutex> l(g_mu);
+    ++g_users;
+}
+
+void xfer_detach()
+{
+    Block out[kIdle];
+    {
+        std::lock_guard<std::mutex> l(g_mu);
+        if (--g_users > 0) return;
+        for (int i = 0; i < kIdle; ++i) {
+            out[i] = g_idle[i];
+            g_idle[i] = Block();
+            g_held -= out[i].n;
+        }
+    }
+    for (auto& q : out)
+        if (q.p) hipHostFree(q.p);
+}
+
+// Bytes of pinned staging memory the library holds.
+extern "C" long fribo_staging_bytes(void)
+{
+    std::lock_guard<std::mutex> l(g_mu);
+    return (long)(g_held * sizeof(double));
+}
+
+void xfer_free(XferEvents& R)
+{
     for (auto& e : R.ev) {
         if (e) hipEventDestroy(e);
         e = nullptr;
     }
 }
 
-hipError_t xfer_run(XferRing& R, const FluidDev& F, XferSeg* segs, int nseg, bool put, hipStream_t st)
+hipError_t xfer_run(XferEvents& R, int dev, const FluidDev& F, XferSeg* segs, int nseg, bool put, hipStream_t st)
 {
     XferTab T{};
     double* host[XFER_MAXSEG];
@@ -189,43 +292,39 @@ hipError_t xfer_run(XferRing& R, const FluidDev& F, XferSeg* segs, int nseg, boo
     hipError_t e = hipSuccess;
     for (auto& ev : R.ev)
         if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
-    const size_t want = std::min<size_t>(kChunk, total);
-    if (R.chunk < want) {
-        // a put of an earlier call may still read the ring
-        if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
-        if (R.stage) hipHostFree(R.stage);
-        R.stage = nullptr;
-        R.chunk = 0;
-        e = hipHostMalloc((void**)&R.stage, want * XferRing::SLOTS * sizeof(double), hipHostMallocDefault);
-        if (e != hipSuccess) return e;
-        R.chunk = want;
-    }
-    constexpr int NS = XferRing::SLOTS;
-    const unsigned chunk = (unsigned)R.chunk, nc = (total + chunk - 1) / chunk;
-    auto slot = [&](unsigned c) { return R.stage + (size_t)(c % NS) * chunk; };
+    const unsigned chunk = (unsigned)std::min<size_t>(kChunk, total), nc = (total + chunk - 1) / chunk;
+    Block b;
+    if ((e = lease(dev, (size_t)std::min<unsigned>(SLOTS, nc) * chunk, b)) != hipSuccess) return e;
+    auto slot = [&](unsigned c) { return b.p + (size_t)(c % SLOTS) * chunk; };
     auto len = [&](unsigned c) { return std::min(chunk, total - c * chunk); };
+    auto wait = [&](unsigned c) { return hipEventSynchronize(R.ev[c % SLOTS]); };
     auto launch = [&](unsigned c) {
         const unsigned l = len(c);
         const dim3 g(std::min(1024u, (l + 255) / 256));
         if (put) hipLaunchKernelGGL(k_xfer<true>, g, dim3(256), 0, st, T, c * chunk, l, slot(c), F.S, F.n2, F.n3m);
         else hipLaunchKernelGGL(k_xfer<false>, g, dim3(256), 0, st, T, c * chunk, l, slot(c), F.S, F.n2, F.n3m);
         const hipError_t le = hipGetLastError();
-        return le != hipSuccess ? le : hipEventRecord(R.ev[c % NS], st);
+        return le != hipSuccess ? le : hipEventRecord(R.ev[c % SLOTS], st);
     };
     const size_t bytes = (size_t)total * sizeof(double);
     const int helpers = bytes >= (size_t)16 << 20 ? 7 : bytes >= (size_t)2 << 20 ? 3 : 0;
     // the kernels of the first chunks run while the helpers start
     if (!put)
-        for (unsigned c = 0; c < std::min<unsigned>(NS, nc); ++c)
-            if ((e = launch(c)) != hipSuccess) return e;
-    Crew crew(helpers, T, host, put);
-    for (unsigned c = 0; c < nc; ++c) {
-        // put: the slot's last kernel (of this call or an earlier one) has read it;
-        // get: the chunk's kernel has written it
-        if ((e = hipEventSynchronize(R.ev[c % NS])) != hipSuccess) return e;
-        crew.run(c * chunk, len(c), slot(c));
-        const unsigned nx = put ? c : c + NS;
-        if (nx < nc && (e = launch(nx)) != hipSuccess) return e;
+        for (unsigned c = 0; c < std::min<unsigned>(SLOTS, nc) && e == hipSuccess; ++c) e = launch(c);
+    if (e == hipSuccess) {
+        Crew crew(helpers, T, host, put);
+        for (unsigned c = 0; c < nc && e == hipSuccess; ++c) {
+            // put: the slot's last kernel has read it; get: the chunk's
+            // kernel has written it
+            if ((!put || c >= SLOTS) && (e = wait(c)) != hipSuccess) break;
+            crew.run(c * chunk, len(c), slot(c));
+            const unsigned nx = put ? c : c + SLOTS;
+            if (nx < nc) e = launch(nx);
+        }
+        // the block is free again when the last kernels have read it
+        if (put && e == hipSuccess) e = wait(nc - 1);
     }
-    return hipSuccess;
+    if (e != hipSuccess) hipStreamSynchronize(st);
+    give(b);
+    return e;
 }

@@ -35,7 +35,7 @@ EXPORTS = ["fribo_init", "fribo_finalize", "fribo_set_state", "fribo_get_state",
            "fribo_batch_set_graph", "fribo_batch_set_gemm_shape", "fribo_batch_get_gemm_shape",
            "fribo_batch_autotune", "fribo_set_precision", "fribo_get_precision", "fribo_test_gemm32",
            "fribo_mlp_create", "fribo_mlp_destroy", "fribo_mlp_size", "fribo_mlp_get_params", "fribo_mlp_grad",
-           "fribo_mlp_train", "fribo_mlp_predict", "fribo_fetch_fields"]
+           "fribo_mlp_train", "fribo_mlp_predict", "fribo_fetch_fields", "fribo_staging_bytes"]
 
 NPROF = 12
 
@@ -89,6 +89,8 @@ def load():
     L.fribo_array_size.restype = C.c_long
     L.fribo_get_array.argtypes = [vp, C.c_char_p, vp, C.c_long]
     L.fribo_sync.argtypes = [vp]
+    L.fribo_staging_bytes.argtypes = []
+    L.fribo_staging_bytes.restype = C.c_long
     L.fribo_last_error.restype = C.c_char_p
     L.fribo_test_gemm.argtypes = [C.c_int32, C.c_int32, C.c_int32, dp, C.c_int32, dp, C.c_int32, dp, C.c_int32]
     L.fribo_test_gemm_nn.argtypes = [C.c_int32, C.c_int32, C.c_int32, dp, C.c_int32, dp, C.c_int32, dp, C.c_int32]

@@ -119,6 +119,12 @@ int fribo_get_array(fribo_handle h, const char* name, void* out, long n);
 
 int fribo_sync(fribo_handle h);
 
+/* Diagnostic (no reference counterpart): bytes of pinned host memory the
+ * library holds for the state transfers of all handles.  One block of at most
+ * 12 MB per transfer that runs at the same time; given back when the last
+ * handle is finalised. */
+long fribo_staging_bytes(void);
+
 /* Windowed read-back for host consumers that need only some planes (output
  * slices, restart in pieces, probes): planes kfirst..klast (reference k
  * indices, -2..n3m+3) of the fields selected by mask (1 q2, 2 q3, 4 pr,
