@@ -288,7 +288,8 @@ hipError_t xfer_run(XferEvents& R, int dev, const FluidDev& F, XferSeg* segs, in
     }
     T.nseg = nseg;
     T.off[nseg] = total;
-    if (total == 0) return hipSuccess;
+    // nothing selected: still wait, and report what the stream's work ended with
+    if (total == 0) return hipStreamSynchronize(st);
     hipError_t e = hipSuccess;
     for (auto& ev : R.ev)
         if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;

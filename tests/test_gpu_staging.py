@@ -78,3 +78,28 @@ def test_concurrent_transfers_have_blocks_of_their_own():
     assert held() <= max(before, len(hs) * BLOCK)
     for g, _ in hs:
         g.close()
+
+
+def test_a_read_back_of_nothing_waits_for_the_handle():
+    """fribo_get_state without arrays and fribo_fetch_fields without fields
+    return when the handle's work is done: a fribo_sync after them has nothing
+    left to wait for (the 200 rollbacks take about 2.5 ms; the sync
+    itself some microseconds)."""
+    import time
+    from fribois2d_amd import gpu
+    L = gpu.load()
+    g, st = _step(1200, 1000, 3)
+    g.set_state(st)
+    g.save_state()
+    for call in (lambda: L.fribo_get_state(g.h, *[None] * 11),
+                 lambda: L.fribo_fetch_fields(g.h, 0, 1, 1, *[None] * 5)):
+        for _ in range(200):
+            g.restore_state()
+        t0 = time.perf_counter()
+        assert call() == 0
+        t1 = time.perf_counter()
+        g.sync()
+        t2 = time.perf_counter()
+        print(f"read-back {1e3 * (t1 - t0):.2f} ms, sync {1e3 * (t2 - t1):.3f} ms", flush=True)
+        assert t2 - t1 < 1e-3
+    g.close()
