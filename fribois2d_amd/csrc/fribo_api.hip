@@ -81,6 +81,7 @@ struct fribo_ctx {
     // the caller set it, -1 by auto_graph
     int use_graph = -1;
     int plain_steps = 0;         // steps by launches since the marker buffers were made
+    int last_launch = -1;        // the last fribo_fluid_tsch: 1 a graph, 0 launches (-1: none yet)
     bool yavail = false;     // transform along y set up
     double dmin = 0.0;       // smallest node spacing of the grid (cordin.F90:217-231)
     double* dpart = nullptr; // device: diagnostics partials [8][256]
@@ -1097,6 +1098,7 @@ extern "C" int fribo_fluid_tsch(fribo_handle h, int32_t ns, double* dt, double d
         enqueue_step(h, cfl);
         h->plain_steps = std::min(h->plain_steps + 1, 2);
     }
+    h->last_launch = graph ? 1 : 0;
     // with per-class profiling the next step's k_cfl stays in that step
     return finish(h, dt, cflm, !h->profiling);
 }
@@ -1106,6 +1108,13 @@ extern "C" int fribo_set_graph(fribo_handle h, int32_t on)
     if (!h) return set_err(FRIBO_ERR_ARG, "null handle");
     h->use_graph = on != 0 ? 1 : 0;
     return FRIBO_OK;
+}
+
+// How the last fribo_fluid_tsch ran: 1 as a replayed graph, 0 by launches, -1
+// no step yet.
+extern "C" int fribo_last_launch(fribo_handle h)
+{
+    return h ? h->last_launch : -1;
 }
 
 extern "C" int fribo_cfl_dt(fribo_handle h, int32_t ns, double* dt, double dt_o, double* cflm)

@@ -35,7 +35,8 @@ EXPORTS = ["fribo_init", "fribo_finalize", "fribo_set_state", "fribo_get_state",
            "fribo_batch_set_graph", "fribo_batch_set_gemm_shape", "fribo_batch_get_gemm_shape",
            "fribo_batch_autotune", "fribo_set_precision", "fribo_get_precision", "fribo_test_gemm32",
            "fribo_mlp_create", "fribo_mlp_destroy", "fribo_mlp_size", "fribo_mlp_get_params", "fribo_mlp_grad",
-           "fribo_mlp_train", "fribo_mlp_predict", "fribo_fetch_fields", "fribo_staging_bytes"]
+           "fribo_mlp_train", "fribo_mlp_predict", "fribo_fetch_fields", "fribo_staging_bytes",
+           "fribo_last_launch"]
 
 NPROF = 12
 
@@ -89,6 +90,7 @@ def load():
     L.fribo_array_size.restype = C.c_long
     L.fribo_get_array.argtypes = [vp, C.c_char_p, vp, C.c_long]
     L.fribo_sync.argtypes = [vp]
+    L.fribo_last_launch.argtypes = [vp]
     L.fribo_staging_bytes.argtypes = []
     L.fribo_staging_bytes.restype = C.c_long
     L.fribo_last_error.restype = C.c_char_p
@@ -339,6 +341,12 @@ class FluidStep:
         """Replay the step as one captured HIP graph (same results); off:
         launch its kernels.  Without a call the library chooses by the grid."""
         _check(load().fribo_set_graph(self.h, 1 if on else 0))
+
+    @property
+    def replayed(self):
+        """Whether the last fluid_tsch replayed a graph (None: no step yet)."""
+        r = load().fribo_last_launch(self.h)
+        return None if r < 0 else r == 1
 
     # -- profiling ----------------------------------------------------------
     def set_profiling(self, on=True, gemm_only=False):

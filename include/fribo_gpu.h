@@ -190,6 +190,9 @@ int fribo_checkbcs(fribo_handle h, double* bcerrv, double* bcerrw, double* nbcv,
  * a call the library replays a graph on small grids, from the third step
  * with the same marker count on. */
 int fribo_set_graph(fribo_handle h, int32_t on);
+/* Diagnostic: how the last fribo_fluid_tsch ran, 1 as a replayed graph, 0 by
+ * launches, -1 no step yet. */
+int fribo_last_launch(fribo_handle h);
 const char* fribo_last_error(void);
 
 /* Diagnostic entry point (no reference counterpart): C = A * B^T in FP64 on
