@@ -1037,6 +1037,7 @@ static int ensure_graph(fribo_ctx* c)
     // captured on a stream of its own that the null stream does not wait for: a
     // launch on the null stream by another thread would break off the capture
     // of an ordinary stream
+    const DeviceGuard guard(c->dev);
     hipGraph_t g = nullptr;
     hipStream_t cap = nullptr, st = c->st;
     HIPCHK(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));

@@ -152,6 +152,20 @@ struct FluidDev {
     DevScalars* S;
 };
 
+// Makes a handle's device current while it creates a stream, an event or
+// pinned memory in a call that may come from a thread on another device.
+struct DeviceGuard {
+    int old = -1;
+    bool moved = false;
+    explicit DeviceGuard(int dev) { moved = hipGetDevice(&old) == hipSuccess && old != dev && hipSetDevice(dev) == hipSuccess; }
+    ~DeviceGuard()
+    {
+        if (moved) hipSetDevice(old);
+    }
+    DeviceGuard(const DeviceGuard&) = delete;
+    DeviceGuard& operator=(const DeviceGuard&) = delete;
+};
+
 // Host side of a load computation, in pinned memory the kernels read and write
 // directly: normals and accelerations (nlm,2) in, pressure (nlm), friction
 // stress (nlm,2) and the error flag out.

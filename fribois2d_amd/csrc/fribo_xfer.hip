@@ -291,6 +291,7 @@ hipError_t xfer_run(XferEvents& R, int dev, const FluidDev& F, XferSeg* segs, in
     // nothing selected: still wait, and report what the stream's work ended with
     if (total == 0) return hipStreamSynchronize(st);
     hipError_t e = hipSuccess;
+    const DeviceGuard guard(dev);
     for (auto& ev : R.ev)
         if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
     const unsigned chunk = (unsigned)std::min<size_t>(kChunk, total), nc = (total + chunk - 1) / chunk;
