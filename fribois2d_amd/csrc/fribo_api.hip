@@ -1762,8 +1762,24 @@ static BGrid<GemmProb> batch_gemm(BatchSet* B, int key, const std::vector<GemmPr
     return BGrid<GemmProb>{T.dprob, g.off, g.dims, B->n};
 }
 
-// Default tile shape of the batch's transforms: the one the largest
-// instance would take on its own, among those every instance can run.
+// Default tile shape of a batch's transforms by the size of its largest
+// instance (M x N), among the shapes every instance can run (mask, bit c for
+// shape c); shape 2, which takes operands of any alignment, where the choice
+// is not among them.  The thresholds see neither the other instances nor the
+// present kernels: for 256 members of 256x192 to 1024x768 they give 64x64,
+// 1.70 ms a launch where shapes 0, 2, 3 and 4 take 1.62, 1.52, 1.44 and 1.41
+// (fribo_batch_autotune finds 4).
+static int gemm_pick(int M, int N, int mask)
+{
+    const auto cdiv = [](int a, int c) { return (a + c - 1) / c; };
+    int cfg = 0;
+    if ((long)cdiv(M, 96) * cdiv(N, 128) >= 192) cfg = 3;
+    else if ((long)cdiv(M, 64) * cdiv(N, 64) >= 96) cfg = 1;
+    return (mask >> cfg) & 1 ? cfg : 2;
+}
+
+extern "C" int fribo_test_gemm_pick(int32_t M, int32_t N, int32_t mask) { return gemm_pick(M, N, mask); }
+
 static int batch_default_gemm(const fribo_batch_ctx* b)
 {
     int mask = 31;
@@ -1777,13 +1793,7 @@ static int batch_default_gemm(const fribo_batch_ctx* b)
             big = &h->F;
         }
     }
-    const int M = big->n2m, N = big->n3m;
-    const auto cdiv = [](int a, int c) { return (a + c - 1) / c; };
-    int cfg = 0;
-    if ((long)cdiv(M, 96) * cdiv(N, 128) >= 192) cfg = (mask & 8) ? 3 : 2;
-    else if ((long)cdiv(M, 64) * cdiv(N, 64) >= 96) cfg = 1;
-    while (cfg > 0 && !((mask >> cfg) & 1)) --cfg;
-    return cfg;
+    return gemm_pick(big->n2m, big->n3m, mask);
 }
 
 // The instances' FluidDev as the batched kernels see them: the j-line

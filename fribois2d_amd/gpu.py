@@ -36,7 +36,7 @@ EXPORTS = ["fribo_init", "fribo_finalize", "fribo_set_state", "fribo_get_state",
            "fribo_batch_autotune", "fribo_set_precision", "fribo_get_precision", "fribo_test_gemm32",
            "fribo_mlp_create", "fribo_mlp_destroy", "fribo_mlp_size", "fribo_mlp_get_params", "fribo_mlp_grad",
            "fribo_mlp_train", "fribo_mlp_predict", "fribo_fetch_fields", "fribo_staging_bytes",
-           "fribo_last_launch"]
+           "fribo_last_launch", "fribo_test_gemm_pick"]
 
 NPROF = 12
 
@@ -91,6 +91,7 @@ def load():
     L.fribo_get_array.argtypes = [vp, C.c_char_p, vp, C.c_long]
     L.fribo_sync.argtypes = [vp]
     L.fribo_last_launch.argtypes = [vp]
+    L.fribo_test_gemm_pick.argtypes = [C.c_int32] * 3
     L.fribo_staging_bytes.argtypes = []
     L.fribo_staging_bytes.restype = C.c_long
     L.fribo_last_error.restype = C.c_char_p

@@ -345,6 +345,10 @@ int fribo_batch_step(fribo_batch b, int32_t ns, double* dt, const double* dt_o, 
 int fribo_batch_set_graph(fribo_batch b, int32_t on);
 int fribo_batch_set_gemm_shape(fribo_batch b, int32_t cfg);
 int fribo_batch_get_gemm_shape(fribo_batch b);
+/* Diagnostic: the default tile shape of a batch whose largest instance has
+ * transforms of M x N, when its instances can all run the shapes in mask (bit
+ * c for shape c; shape 2 is always among them). */
+int fribo_test_gemm_pick(int32_t M, int32_t N, int32_t mask);
 /* Autotuner (no reference counterpart): times the batch's forward transform
  * with every tile shape all its instances can run (reps launches each, no
  * change to any state) and keeps the fastest; ms[10] gets the time per
