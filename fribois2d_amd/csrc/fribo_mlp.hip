@@ -11,8 +11,9 @@
 // by input, the 64 units side by side), so that every access of 64 lanes, one
 // per unit, is one run; fribo_mlp_create and the read-backs convert.
 //
-// Training (FP32): the samples of a call go to the device once; one step over
-// a minibatch is two launches and no synchronisation:
+// Training (FP32): the samples of a call go to the device once (sets of more
+// than 64 MB in pieces); one step over a minibatch is two launches and no
+// synchronisation:
 //   k_mlp_step  workgroups of MLP_NS samples: both hidden layers, the outputs,
 //               the back-propagated errors of the mean squared loss, and the
 //               workgroup's part of the gradient, with the weights in LDS;
@@ -306,6 +307,11 @@ typedef fribo_mlp_ctx* fribo_mlp;
 // inputs and outputs the inference kernel reads and writes on the host.
 #define MLP_PIN 16384
 
+// Most floats of a training set (inputs and targets, 64 MB) that are copied to
+// the device at once and kept there with the network; a larger set goes in
+// pieces, again in every epoch.
+#define MLP_SET ((size_t)16 << 20)
+
 static int mlp_reserve(fribo_mlp m, size_t floats)
 {
     if (floats <= m->cap) return 0;
@@ -426,21 +432,34 @@ static int mlp_run(fribo_mlp m, int n, const float* X, const float* T, int epoch
     const MlpDims& d = m->d;
     batch = std::min(batch, n);
     const int most = std::min((batch + MLP_NS - 1) / MLP_NS, MLP_PARTS);
-    const size_t nx = (size_t)n * d.ni, nt = (size_t)n * d.no, ny = loss ? (size_t)batch * d.no : 0;
+    // the samples on the device at a time: all of them, or as many whole
+    // minibatches as MLP_SET floats hold (one at least)
+    const size_t per = (size_t)d.ni + d.no;
+    int win = n;
+    if (per * n > MLP_SET) win = std::max(1, (int)std::min<size_t>(MLP_SET / per, n) / batch) * batch;
+    win = std::min(win, n);
+    const size_t nx = (size_t)win * d.ni, nt = (size_t)win * d.no, ny = loss ? (size_t)batch * d.no : 0;
     if (mlp_reserve(m, nx + nt + ny + (size_t)most * d.np)) return FRIBO_E_HIP;
     float *dX = m->work, *dT = dX + nx, *dY = dT + nt, *dG = dY + ny;
-    if (hipMemcpyAsync(dX, X, nx * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess ||
-        hipMemcpyAsync(dT, T, nt * sizeof(float), hipMemcpyHostToDevice, m->st) != hipSuccess)
-        return FRIBO_E_HIP;
     const size_t lds = mlp_lds_floats(d) * sizeof(float);
-    int b = 0, s = 0;
+    int b = 0, s = 0, w0 = -1;   // w0: first sample on the device
     for (int e = 0; e < epochs; ++e)
         for (s = 0; s < n; s += batch) {
             b = std::min(batch, n - s);
+            if (w0 < 0 || s < w0 || s - w0 >= win) {
+                w0 = s;
+                const size_t c = std::min(win, n - s);
+                if (hipMemcpyAsync(dX, X + (size_t)s * d.ni, c * d.ni * sizeof(float), hipMemcpyHostToDevice, m->st) !=
+                        hipSuccess ||
+                    hipMemcpyAsync(dT, T + (size_t)s * d.no, c * d.no * sizeof(float), hipMemcpyHostToDevice, m->st) !=
+                        hipSuccess)
+                    return FRIBO_E_HIP;
+            }
+            const size_t o = s - w0;
             const bool last = e == epochs - 1 && s + batch >= n;
             const int parts = std::min((b + MLP_NS - 1) / MLP_NS, MLP_PARTS);
             hipLaunchKernelGGL(k_mlp_step, dim3(parts), dim3(MLP_NT), lds, m->st, d, (const float*)m->p, b,
-                               (const float*)dX + (size_t)s * d.ni, (const float*)dT + (size_t)s * d.no, dG,
+                               (const float*)dX + o * d.ni, (const float*)dT + o * d.no, dG,
                                last && loss ? dY : (float*)nullptr);
             float c1 = 1.0f, c2 = 1.0f;
             if (lr > 0.0f) {
