@@ -327,6 +327,8 @@ def createnorm(verts, orient=-1.0):
     """rigid.F90:468-495: unit normal of every segment from the cross product
     of the segment (x=0 plane) with the vector to its midpoint lifted to x=or."""
     v = np.asarray(verts, dtype=np.float64)
+    if v.shape[0] < 1:
+        raise ValueError("no vertices")
     t1, t2 = v[:-1], v[1:]
     mid = (t1 + t2) * 0.5
     # a = t2 - t1 and b = t3 - t1 with a leading x component (0 and orient);
