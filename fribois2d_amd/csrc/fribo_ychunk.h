@@ -90,14 +90,3 @@ __device__ inline void ysum_vals(double (&v)[6], const double* amphk, const doub
     v[4] = vs;
     v[5] = ws;
 }
-
-// The six separator summaries of chunk p of y-mode j, stored.
-__device__ inline void ysum_store(double* Y, int n2m, int j, int p, const double* amphk, const double* acphk, int e,
-                                  double w, double de, double yl, double vl, double wl, double ys, double vs,
-                                  double ws)
-{
-    double v[6];
-    ysum_vals(v, amphk, acphk, e, w, de, yl, vl, wl, ys, vs, ws);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) Y[ysum_idx(n2m, q, j, p)] = v[q];
-}
