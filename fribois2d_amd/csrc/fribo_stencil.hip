@@ -486,7 +486,7 @@ __device__ void mean_block(const FluidDev& F, double* sh)
     }
 }
 
-// Row values read by boucqt/boucdq for rows j0 and j0 + 1024 (clamped to n2m).
+// Row values read by boucqt/boucdq for rows j0 and j0 + 1024 (those up to n2m).
 struct BcRows {
     double qn2[2], qn3[2], q2e[2], q3e[2], o2[2], o3[2], g[2];
     double qs2[2], qs3[2], dqs2[2], dqs3[2], dqn2[2], dqn3[2];

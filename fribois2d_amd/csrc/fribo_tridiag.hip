@@ -1033,7 +1033,11 @@ __device__ inline void kf_unroll(std::integer_sequence<int, I...>, Fn fn)
     (fn(std::integral_constant<int, I>{}), ...);
 }
 
-constexpr int KFB_COLS = 16;   // columns per workgroup in batches
+// Columns per workgroup in batches, whose instances fill the chip together: a
+// row's run of sixteen columns is a whole cache line.  Four / eight / sixteen:
+// 24 instances of 96..448 x 70..380 40.1 / 28.6 / 29.2 us, 256 of 256..1024 x
+// 192..768 1989 / 1170 / 1028.
+constexpr int KFB_COLS = 16;
 
 template <int MAXM, int NC>
 __device__ __forceinline__ void ksolve_fused_body(const FluidDev& F, const VBlock& vb)

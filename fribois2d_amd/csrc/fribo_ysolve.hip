@@ -223,8 +223,11 @@ __global__ __launch_bounds__(64 * YW) void kb_ysolve3(const BGrid<FluidDev> G)
 // give the same bits.  The z operator's couplings are staged in LDS (one pad
 // slot per 32 rows: the chunks of a wave start on different banks); its
 // diagonal is minus their sum, as the host formed it.
-// Bound by latency: the two eliminations are serial chains of about 100
-// cycles a row, with one workgroup per CU or less.  Against the three passes
+// Bound by latency, one workgroup per CU or less with its phases after each
+// other: at 2048x1536 (192 workgroups) 6.1 us until the rows and couplings are
+// there, 5.3 and 3.0 the two eliminations (31 dependent rows each), 2.6 the
+// separator systems, 1.5 back-substitution and stores; at 384x288 1.5, 0.7,
+// 0.6, 1.7 and 0.4.  Against the three passes
 // (the first of which ran in the forward transform's epilogue where the
 // partition fitted its tiles: 5 us of it): 64x48 13.8 -> 5.7 us, 384x288 16.0
 // -> 7.2, 810x672 19.3 -> 10.2, 1301x977 23.4 -> 15.2, 2048x1536 19.1 and 10
@@ -422,6 +425,9 @@ void launch_ysolve_b(BatchSet& B, hipStream_t st)
         mm = std::max(mm, F.ks[0].maxm - 1);
     }
     if (fused) {
+        // eight modes per workgroup: the instances fill the chip together.
+        // Four / eight / sixteen: 24 instances of 96..448 x 70..380 16.3 / 17.5
+        // / 22.8 us, 256 of 256..1024 x 192..768 531 / 456 / 522
         if (mm < 8) launch_yf_b<8, 8>(B, st);
         else if (mm < 16) launch_yf_b<16, 8>(B, st);
         else launch_yf_b<32, 8>(B, st);
