@@ -924,7 +924,9 @@ __device__ inline double row_sum9(double v)
 // in two steps (the rows' odd lanes take the second derivative) and one
 // gather instead of 27 weights, nine solves and 81 gathers in one thread.
 // Normals and accelerations come straight from pinned host memory.  91
-// markers: 66 us with one thread per marker, 12 us here.
+// markers: 66 us with one thread per marker, 12 us here; from about 5000 on one
+// thread each would take less of the GPU (8192: 62 / 98 us, 110000: 0.19 / 1.29
+// ms), far beyond the bodies of the inputs.
 __global__ __launch_bounds__(64) void k_loads(const FluidDev F, const LoadsIO io, double hpr)
 {
     DevScalars* S = F.S;
@@ -1047,71 +1049,72 @@ __global__ __launch_bounds__(64) void k_loads(const FluidDev F, const LoadsIO io
 }
 
 // Tangent of every marker: its own, else the last one set before it
-// (loads_transfer.F90:94-96), by one wave with a "last set" scan over lane
-// chunks; then the friction stress (loads_transfer.F90:111-128).  The results
-// and the error flag go straight to pinned host memory.
-__global__ __launch_bounds__(64) void k_loads_tau(const FluidDev F, const LoadsIO io, double hpr)
+// (loads_transfer.F90:94-96), else zero; then the friction stress
+// (loads_transfer.F90:111-128).  One thread per marker; the last set marker is
+// found by ballots within a wave, through LDS within the workgroup, and by a
+// search back over the markers before it only where the workgroup's first
+// markers have no tangent of their own.  The results and the error flag go
+// straight to pinned host memory, in whole runs.  1000 markers 4.1 us, 110000
+// 52; one wave for all markers, each lane a run of them, took 25 us for 1000,
+// and with its stores scattered over the host's memory the call for 110000
+// took 4.1 ms where it takes 1.5 now.
+__device__ __forceinline__ bool has_tangent(const FluidDev& F, int n) { return LW(n, 0) != 0.0 && LW(n, 1) != 0.0; }
+
+#define TAU_T 256
+__global__ __launch_bounds__(TAU_T) void k_loads_tau(const FluidDev F, const LoadsIO io, double hpr)
 {
-    const int lane = threadIdx.x, nlm = F.nlm, err = F.S->err;
-    if (lane == 0) *io.err = err;
+    constexpr int NW = TAU_T / 64;
+    __shared__ int last[NW], found[NW];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, nlm = F.nlm, err = F.S->err;
+    const int before = blockIdx.x * TAU_T;   // markers before this workgroup's
+    if (blockIdx.x == 0 && t == 0) *io.err = err;
     if (err) return;
-    const int per = (nlm + 63) / 64;
-    const int n0 = lane * per + 1, n1 = min(nlm, n0 + per - 1);
-    bool has = false;
+    const int n = before + t + 1;
+    const bool in = n <= nlm, inside = in && LW(n, 0) != 0.0;
+    const unsigned long long set = __ballot(inside && LW(n, 1) != 0.0);
+    // the last marker with a tangent, up to this one (0: none)
+    const unsigned long long upto = set & (~0ull >> (63 - lane));
+    int src = upto ? before + 64 * w + 64 - __clzll((long long)upto) : 0;
+    if (lane == 0) last[w] = set ? before + 64 * w + 64 - __clzll((long long)set) : 0;
+    __syncthreads();
+    for (int q = w - 1; q >= 0 && !src; --q) src = last[q];
+    if (__syncthreads_or(inside && !src)) {
+        int carry = 0;
+        for (int e = before; e > 0 && !carry; e -= TAU_T) {   // marker e - t
+            const unsigned long long m = __ballot(e - t >= 1 && has_tangent(F, e - t));
+            if (lane == 0) found[w] = m ? e - 64 * w - (__ffsll((long long)m) - 1) : 0;
+            __syncthreads();
+            for (int q = 0; q < NW && !carry; ++q) carry = found[q];
+            __syncthreads();
+        }
+        if (!src) src = carry;
+    }
+    if (!in) return;
+    io.press[n - 1] = LW(n, 19);
     double ty = 0.0, tz = 0.0;
-    for (int n = n0; n <= n1; ++n)
-        if (LW(n, 0) != 0.0 && LW(n, 1) != 0.0) {
-            has = true;
-            ty = LW(n, 2);
-            tz = LW(n, 3);
-        }
-    // inclusive scan of (has, t) with "later set wins", then shift by one lane
-    for (int h = 1; h < 64; h <<= 1) {
-        const int oh = __shfl_up((int)has, h, 64);
-        const double oy = __shfl_up(ty, h, 64), oz = __shfl_up(tz, h, 64);
-        if (lane >= h && !has && oh) {
-            has = true;
-            ty = oy;
-            tz = oz;
-        }
-    }
-    int ih = __shfl_up((int)has, 1, 64);
-    double cy = __shfl_up(ty, 1, 64), cz = __shfl_up(tz, 1, 64);
-    if (lane == 0 || !ih) {
-        cy = 0.0;
-        cz = 0.0;
-    }
-    const double visc = F.visc;
-    for (int n = n0; n <= n1; ++n) {
-        io.press[n - 1] = LW(n, 19);
-        if (LW(n, 0) == 0.0) {
-            io.tau[n - 1] = 0.0;
-            io.tau[(size_t)(n - 1) + nlm] = 0.0;
-            continue;
-        }
-        if (LW(n, 1) != 0.0) {
-            cy = LW(n, 2);
-            cz = LW(n, 3);
-        }
-        const double nory = LW(n, 17), norz = LW(n, 18), tany = cy, tanz = cz;
+    if (inside) {
+        const double nory = LW(n, 17), norz = LW(n, 18);
+        const double tany = src ? LW(src, 2) : 0.0, tanz = src ? LW(src, 3) : 0.0;
         const double u1 = LW(n, 4), u2 = LW(n, 5), u3 = LW(n, 6), u4 = LW(n, 7), u5 = LW(n, 8), u6 = LW(n, 9);
         const double v1 = LW(n, 10), v2 = LW(n, 11), v3 = LW(n, 12), v4 = LW(n, 13), v5 = LW(n, 14), v6 = LW(n, 15);
-        const double d3ucdn3 = LW(n, 16);
+        const double d3ucdn3 = LW(n, 16), visc = F.visc;
         const double ducdn = (u1 * tany * nory + u2 * tany * norz + v1 * tanz * nory + v2 * tanz * norz);
         const double d2ucdn2 = (u3 * tany * nory * nory + u4 * tany * nory * norz + u5 * tany * norz * nory +
                                 u6 * tany * norz * norz + v3 * tanz * nory * nory + v4 * tanz * nory * norz +
                                 v5 * tanz * norz * nory + v6 * tanz * norz * norz);
         const double ducdnm = ducdn - d2ucdn2 * hpr - 0.5 * d3ucdn3 * (hpr * hpr);
-        io.tau[n - 1] = visc * ducdnm * tany;
-        io.tau[(size_t)(n - 1) + nlm] = visc * ducdnm * tanz;
+        ty = visc * ducdnm * tany;
+        tz = visc * ducdnm * tanz;
     }
+    io.tau[n - 1] = ty;
+    io.tau[(size_t)(n - 1) + nlm] = tz;
 }
 
 void launch_loads(const FluidDev& F, const LoadsIO& io, double hpr, hipStream_t st)
 {
     if (F.nlm <= 0) return;
     hipLaunchKernelGGL(k_loads, dim3(F.nlm), dim3(64), 0, st, F, io, hpr);
-    hipLaunchKernelGGL(k_loads_tau, dim3(1), dim3(64), 0, st, F, io, hpr);
+    hipLaunchKernelGGL(k_loads_tau, dim3((F.nlm + TAU_T - 1) / TAU_T), dim3(TAU_T), 0, st, F, io, hpr);
 }
 
 // ckbcs.F90:5-86: velocity error at the markers after the step and the norms
