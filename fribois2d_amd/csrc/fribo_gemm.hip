@@ -52,9 +52,8 @@
 // workgroup per CU; 96 x 64 tiles of 8 waves, two per CU, measured the same
 // within 2%) with K-slices of 24 (144 KB of LDS for the three stages;
 // 16-deep slices measured 4-8% slower).  The 1536 x 2048 transforms of the
-// 2048x1536-cell grid give 256 workgroups, one per CU (84.4 us alone in the
-// mirror form; 87 in the step, with the operands out of the caches);
-// workgroups are
+// 2048x1536-cell grid give 256 workgroups, one per CU (83-84 us in the
+// step in the mirror form); workgroups are
 // dispatched to the 8 XCDs round-robin, so when the grid is a multiple of 256
 // tiles in 8 x 4 patches the tile indices are permuted to give each XCD
 // compact patches (its L2 then serves 8 A- and 4 B-tiles to 32 workgroups).
